@@ -239,9 +239,12 @@ def prepare(case, seed):
     base, churn = _base_and_churn(case, g)
     alg = _started(case, seed, base)
     if kind == "serve":
-        # the arrival pattern belongs to the case; who asks about whom comes from the seed, and one
-        # query in four is about an id without edges
+        # the arrival pattern belongs to the case and ends with one group of point queries; who asks
+        # about whom comes from the seed, and one query in four is about an id without edges
         trace = gen.serving_trace(n, churn.shape[0], 5, case["per_request"], cc_frac=0.05)
+        last = np.zeros(32, dtype=trace.dtype)
+        last["kind"] = gz.REQ_POINT
+        trace = np.concatenate([trace, last])
         point = trace["kind"] == gz.REQ_POINT
         trace["u"][point] = np.where(rng.random(point.sum()) < 0.25, n - 1, rng.integers(0, n - n // 256, point.sum()))
         trace["v"][point] = rng.integers(0, n - n // 256, point.sum())
