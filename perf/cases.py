@@ -273,6 +273,7 @@ def run(state):
     alg = state["alg"]
     if kind == "plugin":
         for src, dsts in state["gutters"]:
+            alg.pre_insert(src, int(dsts[0]))  # without the eager DSU it only marks the answer as old
             alg.apply_update_batch(0, src, dsts)
         cc = alg.connected_components()
         return {"num_cc": cc.size(), "labels": cc.canonical_labels().astype(np.int64), "image": alg.dump_sketches()}
