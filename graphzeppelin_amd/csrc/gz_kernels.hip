@@ -202,16 +202,23 @@ constexpr uint32_t kNoLink = 0xFFFFFFFFu;
 // merges into a hub go through the smaller roots' own parent words instead of all contending for
 // the hub's.  Returns the root that was linked under the other one, or kNoLink when a and b were
 // already connected.
+// LATE: the hints are loaded once the roots are known to differ (a batch whose edges are mostly
+// connected already); otherwise with the first parents (Borůvka's samples, which mostly link).
+template <bool LATE = false>
 __device__ inline uint32_t dsu_link(uint32_t* parent, uint32_t a, uint32_t b, uint32_t pseed,
-                                    const unsigned char* hint = nullptr) {
+                                    const unsigned char* hint) {
   while (true) {
     // both first parents (and hints) in one round trip; a root (the common case) needs no more
     const uint32_t a_up = ld_acq(parent + a), b_up = ld_acq(parent + b);
-    uint32_t ha = hint ? hint[a] : 0, hb = hint ? hint[b] : 0;
+    uint32_t ha = 0, hb = 0;
+    if (!LATE) {
+      ha = hint[a];
+      hb = hint[b];
+    }
     const uint32_t ra = dsu_find_from(parent, a, a_up), rb = dsu_find_from(parent, b, b_up);
     if (ra == rb) return kNoLink;
-    if (hint && ra != a) ha = hint[ra];
-    if (hint && rb != b) hb = hint[rb];
+    if (LATE || ra != a) ha = hint[ra];
+    if (LATE || rb != b) hb = hint[rb];
     a = ra;
     b = rb;
     const uint32_t pa = dsu_prio(a, pseed), pb = dsu_prio(b, pseed);
@@ -842,13 +849,29 @@ inline uint32_t grid_for(size_t work, uint32_t block, uint32_t cap = 8192) {
 // reference's stream threads are concurrent as well): a deleted forest edge always invalidates,
 // and any edge that merged and occurs again in the batch invalidates.
 // ================================================================================================
+// Rank classes for a batch on an instance that no query has ranked yet (RoundBufs::hint): every
+// update draws a level that is l or more with probability 2^-l, and a vertex's class is the highest
+// level among its updates, about the logarithm of its degree in the batch.  Plain stores race, which
+// can only lose a level: any classes give the same components.
+__global__ void k_eager_rank(const uint2* __restrict__ pairs, size_t count, uint32_t n, unsigned char* hint) {
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
+    const unsigned char level = (unsigned char)__builtin_ctzll(mix64(i) | (1ull << 40));
+    if (level == 0) continue;
+    const uint2 p = pairs[i];
+    if (p.x >= n || p.y >= n) continue;
+    if (hint[p.x] < level) hint[p.x] = level;
+    if (hint[p.y] < level) hint[p.y] = level;
+  }
+}
+
 // src != pairs: the batch is also copied from src into pairs (the staging buffer) on the way, so
 // ingesting device pairs needs no separate copy launch; the copy happens whether or not the DSU
 // is still valid.
 // build_sf: the first batch after a query also fills the forest membership set from the query's
 // forest edges (sf_edge) -- lock-free inserts like this batch's own, so the two need no order.
 __global__ void k_eager_union(const uint2* __restrict__ src, uint2* __restrict__ pairs, size_t count,
-                              uint8_t* __restrict__ merged, DsuDev d, uint32_t build_sf) {
+                              uint8_t* __restrict__ merged, DsuDev d, uint32_t build_sf,
+                              const unsigned char* __restrict__ hint) {
   const bool live = !ld_acq(d.flags + kFlagEagerInvalid);
   if (!live && src == pairs) return;
   if (build_sf && live)
@@ -865,7 +888,7 @@ __global__ void k_eager_union(const uint2* __restrict__ src, uint2* __restrict__
       st_rlx(d.flags + kFlagBadInput, 1u);
       continue;
     }
-    const uint32_t child = dsu_link(d.parent, p.x, p.y, d.prio_seed);
+    const uint32_t child = dsu_link<true>(d.parent, p.x, p.y, d.prio_seed, hint);
     merged[i] = child != kNoLink ? 1 : 0;
     if (child != kNoLink) {
       const uint64_t key = concat_pairing(p.x, p.y);
@@ -1052,7 +1075,7 @@ __device__ inline uint32_t walk_vertex(const uint32_t* act_list, uint32_t round,
   return round >= 2 ? act_list[i] : i;
 }
 
-__device__ inline bool apply_sample(const DsuDev& d, uint64_t s, const unsigned char* hint = nullptr) {
+__device__ inline bool apply_sample(const DsuDev& d, uint64_t s, const unsigned char* hint) {
   if (s == kSampZero) return false;
   if (s == kSampFail) return true;
   const uint32_t a = (uint32_t)(s >> 32), b = (uint32_t)s;
@@ -2185,14 +2208,35 @@ void launch_group(const uint32_t* pairs, size_t count, uint32_t n, uint32_t tile
 
 size_t part_hist_len() { return (size_t)kPartBins * kPartMaxBlocks + 1; }
 
+// A large batch on an instance that no query has ranked gets classes first and is merged in launches
+// of doubling size.  The time of the first merges is failed CAS attempts on hubs' words: every update
+// in flight that joins two hubs' components tries the lower hub.  With hubs ranked first and few
+// updates in flight until the largest component holds the hubs, the rest mostly find themselves
+// connected.  First batch of 936k updates on 2^17 vertices, median of 5, one launch unranked -> this:
+// R-MAT 2249 -> 157 us, uniform 963 -> 267; 1M Chung-Lu updates on 2^18 vertices 1932 -> 210.  With
+// first launches of 32768 or steps of 8 it takes up to ten times as long.  Below kRankMin one launch
+// costs less than these.
+constexpr size_t kRankMin = 32768, kRankFirst = 8192;
 void launch_eager(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged, const DsuDev& d,
-                  hipStream_t s, bool build_sf) {
+                  hipStream_t s, bool build_sf, unsigned char* hint, bool ranked) {
   if (!count) return;
   uint2* p2 = reinterpret_cast<uint2*>(pairs);
+  const uint2* s2 = reinterpret_cast<const uint2*>(src);
   const uint32_t grid = grid_for(count, 256);
-  const uint32_t ugrid = build_sf ? std::max(grid, grid_for(d.n, 256, 4096)) : grid;
-  hipLaunchKernelGGL(k_eager_union, dim3(ugrid), dim3(256), 0, s, reinterpret_cast<const uint2*>(src), p2, count,
-                     merged, d, build_sf ? 1u : 0u);
+  size_t lo = 0, hi = count;
+  if (!ranked && count >= kRankMin) {
+    hipLaunchKernelGGL(k_eager_rank, dim3(grid), dim3(256), 0, s, s2, count, d.n, hint);
+    hi = std::min(count, kRankFirst);
+  }
+  while (lo < count) {
+    const size_t m = hi - lo;
+    const uint32_t ugrid = build_sf ? std::max(grid_for(m, 256), grid_for(d.n, 256, 4096)) : grid_for(m, 256);
+    hipLaunchKernelGGL(k_eager_union, dim3(ugrid), dim3(256), 0, s, s2 + lo, p2 + lo, m, merged + lo, d,
+                       build_sf ? 1u : 0u, hint);
+    build_sf = false;
+    lo = hi;
+    hi = std::min(count, 2 * hi);
+  }
   hipLaunchKernelGGL(k_eager_sf_check, dim3(grid), dim3(256), 0, s, p2, count, merged, d);
 }
 

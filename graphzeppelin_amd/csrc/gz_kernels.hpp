@@ -82,9 +82,10 @@ void launch_group(const uint32_t* pairs, size_t count, uint32_t n, uint32_t tile
 // ---- eager DSU (batch form of pre_insert, src/cc_sketch_alg.cpp:79-104) ----
 // src != pairs: the batch is copied from src into pairs by the same launch.
 // build_sf: the same launch first fills the forest membership set from d.sf_edge (the first
-// batch after a query).
+// batch after a query).  hint: n rank classes (RoundBufs::hint); ranked: false while no query
+// has written them and the instance is new.
 void launch_eager(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged, const DsuDev& d,
-                  hipStream_t s, bool build_sf = false);
+                  hipStream_t s, bool build_sf, unsigned char* hint, bool ranked);
 
 // ---- Borůvka ----
 struct RoundBufs;

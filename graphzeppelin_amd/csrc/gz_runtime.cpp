@@ -244,7 +244,8 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   r_totals.alloc(16);
   r_stats.alloc(128);
   r_det.alloc((size_t)n * (8 + gb));
-  r_hint.alloc(n);
+  r_hint.alloc(((size_t)n + 3) & ~size_t(3));
+  launch_fill_u32(reinterpret_cast<uint32_t*>(r_hint.p), 0, r_hint.n / 4, st);  // no classes before the first query
   launch_fill_u32(r_stats.p, 0, 128, st);
   // cross-workgroup accumulators of the reduce: one slot per workgroup and one for the giant
   const size_t xslots = (size_t)reduce_blocks(n) + 1;
@@ -878,6 +879,7 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
     }
     hround_pending = true;
     sf_pending = cfg.eager_dsu;
+    unranked_seen = 4ull * n;
     // every eager batch enqueued before the query has finished (the query ended with a stream
     // synchronisation), so none can set the mirror after this
     eager_inv.p[0] = 0;
@@ -894,7 +896,8 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
 
 void GzAlg::eager_batch(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged) {
   if (!count) return;
-  launch_eager(src, pairs, count, merged, dsu, st, sf_pending);  // builds the forest set when pending
+  launch_eager(src, pairs, count, merged, dsu, st, sf_pending, rb.hint, unranked_seen >= 4ull * n);
+  unranked_seen += count;  // builds the forest set when pending
   sf_pending = false;
 }
 

@@ -340,6 +340,10 @@ class GzAlg {
   // The spanning-forest membership set that the eager DSU's deletion check reads is built from the
   // forest edges after a query, but only before the first eager batch that needs it.
   bool sf_pending = false;
+  // Updates the eager DSU took before the first query wrote the rank classes (RoundBufs::hint): the
+  // large batches among the first 4n are ranked and merged stepwise (launch_eager); after those the
+  // largest component holds the hubs.
+  uint64_t unranked_seen = 0;
   // src != pairs: the batch is copied from src into pairs (device memory) by the same launch
   void eager_batch(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged);
   void enqueue_query_prefix(bool giant_ok, uint32_t last);
