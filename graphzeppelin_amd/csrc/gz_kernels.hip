@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <stdexcept>
+#include <utility>
 
 #include "gz_kernels.hpp"
 
@@ -1420,15 +1421,23 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
 
 // Segmented XOR-reduce + sample (range_merge of column `round` + the deterministic bucket over
 // every member of a supernode, then sample_supernode).  Entries are the member list, grouped by
-// root.  A wave takes 64 consecutive entries; lane l < D accumulates depth l of the column and lane
-// D the deterministic bucket.  A supernode whose entries all lie inside the range is sampled from
-// registers; its sample record goes to samp[root] for k_apply_samples.  A supernode that crosses
-// the range's first (head) or last (tail) boundary leaves its partial XOR in the range's head or
-// tail slot under its root; a slot left unused gets root kNoRoot and a zero value.
+// root.  A wave takes 64 consecutive entries (reduce_members).  A supernode whose entries all lie
+// inside the range is sampled from registers; its sample record goes to samp[root] for
+// k_apply_samples.  A supernode that crosses the range's first (head) or last (tail) boundary leaves
+// its partial XOR in the range's head or tail slot under its root; a slot left unused gets root
+// kNoRoot and a zero value.
 //
-// A workgroup of 16 waves covers 1024 entries: the waves leave their slots in LDS, then one wave
-// reduces those 32 slots the same way, so at most two supernodes of a workgroup are unfinished:
-// the one continuing from the previous workgroup and the one continuing into the next.
+// A workgroup of 16 waves covers 1024 entries: the waves leave their slots in LDS, then the wave in
+// which a crossing supernode starts adds up that supernode's slots, so at most two supernodes of a
+// workgroup are unfinished: the one continuing from the previous workgroup and the one continuing
+// into the next.
+//
+// A full round over 2^18 members reads three lines per member (122 MB) and is bound by them: a
+// workgroup's records arrive over 7..20 us of its 28 and the sampling runs behind.  Before the rows of
+// 16 lanes a member filled 16 of a load's 64 lanes and a wave took its members in 8 dependent
+// batches: the launched rounds of a 24M-update, 2^18-vertex serving trace went from 39.1 to 25.0 us on
+// average, those of 32k vertices from 34.3 to 15.0 us, of 2^20 R-MAT vertices from 147 to 79 us, and
+// the single-workgroup finish of about 1500 members from 95 to 47 us.
 //
 // Cross-workgroup supernodes.  A supernode whose entries span workgroups f..l (f < l) is combined
 // with device-scope XOR atomics into the accumulator slot of f, its first workgroup (only one
@@ -1463,143 +1472,269 @@ struct XAcc {
   const uint32_t* seg_end;  // segment end per root (the scatter cursor after k_bv_scatter)
 };
 
-// Reduce entries [p0, p0 + len) (len <= 64) with one wave.  prev_root / next_root: roots of the
-// entries just before and after the range (kNoRoot when none), which decide whether the first and
-// last segments are open.  FIRST: entries are members (rows of the slab); otherwise partial
-// entries (in_part / in_root in LDS).  FIRST with ROOTPOS: the entries' roots by position in
-// root_pos (members and root_pos may be in LDS) instead of by vertex in vroot.  *all_a / *all_g get the XOR
-// of every entry read.  FIRST
-// with s_bnd: the wave holding the workgroup's first entry [blk_b0] loads that entry's segment
-// bounds into s_bnd[0..1], the one holding its last entry the end of that entry's segment into
-// s_bnd[2], in flight with the values.
-template <class G, bool FIRST, bool ROOTPOS = false, bool SKIP = false>
-__device__ inline void reduce_range(uint32_t p0, uint32_t len, uint32_t prev_root, uint32_t next_root,
-                                    const uint32_t* __restrict__ members, const uint32_t* __restrict__ vroot,
-                                    const unsigned char* __restrict__ slab, const Geo& g, uint32_t round,
-                                    const uint64_t* in_part, const uint32_t* in_root, Slot head, Slot tail,
-                                    uint64_t* __restrict__ samp, uint32_t* __restrict__ flags, uint64_t* all_a_out,
-                                    uint64_t* all_g_out, const unsigned char* __restrict__ det_cpy,
-                                    const XAcc* xa, uint32_t blk_b0, uint32_t blk_b1, uint32_t* s_bnd,
-                                    const uint32_t* root_pos = nullptr, bool deep_on = true) {
-  const uint32_t lane = lane_id();
-  uint32_t m = 0, rt = kNoRoot;
-  if (lane < len) {
-    if (FIRST) {
-      m = members[p0 + lane];
-      rt = ROOTPOS ? root_pos[p0 + lane] : vroot[m];
-    } else {
-      rt = in_root[p0 + lane];
-    }
+// Value of lane K of every row of 16 lanes, given to all lanes of that row.  Every lane must be active.
+template <uint32_t K>
+__device__ inline uint32_t row_bcast(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + K, 0xf, 0xf, false);  // row_newbcast:K
+}
+template <class F, uint32_t... K>
+__device__ inline void for_each_index(F&& f, std::integer_sequence<uint32_t, K...>) {
+  (f(std::integral_constant<uint32_t, K>{}), ...);
+}
+// Bits 0 .. k - 1 (k <= 64).
+__device__ inline uint64_t low_bits(uint32_t k) { return k >= 64 ? ~0ull : (1ull << k) - 1; }
+
+// Reduce entries [p0, p0 + len) of a grouped member list with one wave (len <= 4q, q <= 16).  members /
+// mroot: the list and its roots by position, list_end entries (global or LDS).
+//
+// Four entries per load: row j of 16 lanes takes entries p0 + jq .. p0 + jq + q - 1 one after the
+// other; lane i < 15 of a row reads depth i of column `round`, lane 15 the deterministic bucket from
+// the compact copy.  All q records of a lane are loaded at once, so the entries of a wave cost one
+// dependent round trip instead of one per 8 entries, and a load fills all 64 lanes where 16 of 64
+// did the work.  A run of entries of one supernode that lies inside the wave is sampled from
+// registers; runs crossing rows are carried from row to row.  The entries' deeper records (depths
+// >= 15) are read by the whole wave, one entry per load, only where the sum needs them: for a run
+// without a good bucket below, and for the parts that leave the wave.  With deep flags and deep_on
+// only the entries whose flag is set are read (the others hold zeros); otherwise all of them.
+//
+// A run that started before the range is left in the head slot under its root, one that continues
+// past it in the tail slot; one that does both is left in the head slot, with a zero value under the
+// same root in the tail slot, so the supernode's entries stay contiguous in the next reduce.  A slot
+// left unused gets root kNoRoot and a zero value.  s_tot, if given, gets the XOR of every entry.  With
+// s_bnd, the wave holding the workgroup's first entry [blk_b0] loads that entry's segment bounds into
+// s_bnd[0..1], the one holding its last entry the end of that entry's segment into s_bnd[2].
+constexpr uint32_t kRow = 16, kRowDet = kRow - 1;  // lanes of a row; the lane of the deterministic bucket
+typedef uint32_t Words __attribute__((ext_vector_type(16)));  // one word of a row's 16 entries per lane
+template <class G>
+__device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uint32_t list_end,
+                                      const uint32_t* members, const uint32_t* mroot,
+                                      const unsigned char* __restrict__ slab, const Geo& g, uint32_t round, Slot head,
+                                      Slot tail, uint64_t* __restrict__ samp, uint32_t* __restrict__ flags,
+                                      const unsigned char* __restrict__ det_cpy, bool deep_on, uint64_t* s_tot,
+                                      const XAcc* xa, uint32_t blk_b0, uint32_t blk_b1, uint32_t* s_bnd) {
+  constexpr uint32_t RB = 8 + sizeof(G);
+  const uint32_t lane = lane_id(), i = lane % kRow, base = lane - i, row = lane / kRow;
+  // lane base + k holds entry k of its row
+  const bool mine = i < q && row * q + i < len;
+  const uint32_t pe = p0 + row * q + i;
+  uint32_t m = 0, rt = kNoRoot, before = kNoRoot;
+  if (mine) {
+    m = members[pe];
+    rt = mroot[pe];
+    if (pe > 0) before = mroot[pe - 1];
   }
-  // SKIP with deep_on (members only): each member's deep flag of column `round`; its deep records
-  // are read only when it is set.  The flag shares a line with the column's low records, which the
-  // batch loads below read anyway.
-  uint32_t deep = 1;
-  if (SKIP && FIRST && deep_on && lane < len)
-    deep = *reinterpret_cast<const uint32_t*>(slab + (size_t)m * g.row + deep_flag_off(round));
-  const uint32_t first_root = rd_lane_u32(rt, 0), last_root = rd_lane_u32(rt, len - 1);
-  const bool head_open = first_root != kNoRoot && prev_root == first_root;
-  const bool tail_open = last_root != kNoRoot && next_root == last_root;
   const uint32_t p1 = p0 + len;
-  const bool holds_first = FIRST && s_bnd && p0 == blk_b0;
-  const bool holds_last = FIRST && s_bnd && p1 == blk_b1;
+  const uint32_t next_root = p1 < list_end ? mroot[p1] : kNoRoot;
+  // bit l: lane l's entry begins a run.  Lanes without an entry continue the run before them with zeros.
+  const uint64_t starts = __ballot(mine && rt != before);
+  const uint32_t rowst = (uint32_t)(starts >> base) & 0xffffu;
+  const uint32_t first_root = rd_lane_u32(rt, 0);
+  const uint32_t last_root = rd_lane_u32(rt, (int)((len - 1) / q * kRow + (len - 1) % q));
+  const bool tail_open = next_root == last_root;
+  const bool holds_first = s_bnd && p0 == blk_b0;
+  const bool holds_last = s_bnd && p1 == blk_b1;
   uint32_t bnd = 0;
   if (holds_first && lane == 0) bnd = xa->seg_off[first_root];
   if (holds_first && lane == 1) bnd = xa->seg_end[first_root];
   if (holds_last && lane == 2) bnd = xa->seg_end[last_root];
 
-  const bool in_col = lane < g.D;
-  const uint32_t coff = in_col ? rec_col_off<G>(g, round, lane) : 0;  // depth `lane` of column `round`
-  const bool loads = lane <= g.D;
-  const bool deep_lane = SKIP && deep_on && in_col && rec_is_deep(g, lane);
-  bool wrote_head = false, wrote_tail = false;
+  const bool live = i == kRowDet || i < g.D;
+  const unsigned char* src = i == kRowDet ? det_cpy : slab + (live ? rec_col_off<G>(g, round, i) : 0u);
+  const uint32_t stride = i == kRowDet ? RB : g.row;
+  const uint32_t row_n = row * q < len ? (len - row * q < q ? len - row * q : q) : 0u;  // the row's entries
+  constexpr bool kWide = sizeof(G) == 8;
+  Words lo = 0, hi = 0, glo = 0, ghi = 0;
+  for_each_index(
+      [&](auto kc) {
+        constexpr uint32_t k = kc;
+        const uint32_t mv = row_bcast<k>(m);
+        uint64_t a = 0;
+        G gm = 0;
+        if (live && k < row_n) ld_rec<G>(src + (size_t)mv * stride, &a, &gm);
+        lo[k] = (uint32_t)a;
+        hi[k] = (uint32_t)(a >> 32);
+        glo[k] = (uint32_t)gm;
+        if constexpr (kWide) ghi[k] = (uint32_t)((uint64_t)gm >> 32);
+      },
+      std::make_integer_sequence<uint32_t, kRow>{});
+  uint32_t flag = 1;
+  if (kDeepFlags<G> && deep_on && mine)
+    flag = *reinterpret_cast<const uint32_t*>(slab + (size_t)m * g.row + deep_flag_off(round));
 
-  // Every lane stores the root (the same value), so every lane of this wave may read it back
-  // without a barrier.
-  auto put = [&](Slot sl, uint32_t R, uint64_t a, uint64_t gm) {
-    sl.vals[lane] = a;
-    sl.vals[kWave + lane] = gm;
-    *sl.root = R;
-  };
-  auto emit = [&](uint32_t R, uint64_t acc_a, uint64_t acc_g, uint32_t seg_start, uint32_t seg_end) {
-    const bool started_before = seg_start == p0 && head_open;
-    const bool continues = seg_end == p1 && tail_open;
-    if (!started_before && !continues) {
-      if (R != kNoRoot) {
-        uint64_t idx;
-        const int code = wave_sample<G>(acc_a, (G)acc_g, g.D, g.chk_bf, &idx);
-        if (lane == 0) samp[R] = sample_record(code, idx, g.n, flags);
+  uint64_t again = 0;  // first lanes of the runs inside the wave whose sample is left to the deep records
+  // Sample the runs of the rows with `done` set (the same in all lanes of a row); first: the run's first lane.
+  auto emit = [&](bool done, uint64_t a, G gm, uint32_t R, uint32_t first) {
+    const uint32_t good =
+        (uint32_t)(__ballot(done && live && (G)xxh3_mix(xxh3_prep(a), g.chk_bf) == gm) >> base) & 0xffffu;
+    const bool zero =
+        ((uint32_t)(__ballot(done && i == kRowDet && (a | (uint64_t)gm) == 0) >> base) >> kRowDet) & 1u;
+    const uint32_t col = good & ((1u << kRowDet) - 1);
+    const bool det = (good >> kRowDet) & 1u;
+    bool left = false;
+    if (done) {
+      if (i == kRowDet) {
+        if (zero) samp[R] = kSampZero;
+        else if (det) samp[R] = sample_record(kGood, a, g.n, flags);
+        else left = col == 0;
+      } else if (!zero && !det && col && i == (uint32_t)__builtin_ctz(col)) {
+        samp[R] = sample_record(kGood, a, g.n, flags);
       }
-      return;
     }
-    // Partial of a spanning supernode: the head slot if it started before this range, else the
-    // tail slot.  When it covers the whole range the tail slot carries the same root with a zero
-    // value, so the supernode's entries stay contiguous in the next reduce.
-    if (started_before) {
-      put(head, R, acc_a, acc_g);
-      wrote_head = true;
-      if (continues) {
-        put(tail, R, 0, 0);
-        wrote_tail = true;
-      }
-    } else {
-      put(tail, R, acc_a, acc_g);
-      wrote_tail = true;
-    }
+    for (uint64_t b = __ballot(left); b; b &= b - 1) again |= 1ull << rd_lane_u32(first, __builtin_ctzll(b));
   };
 
-  uint64_t acc_a = 0, acc_g = 0, all_a = 0, all_g = 0;
-  uint32_t cur = first_root, seg_start = p0;
-  constexpr uint32_t U = FIRST ? 8 : 16;  // loads in flight per lane
-  for (uint32_t j = 0; j < len; j += U) {
-    uint64_t va[U], vg[U];
-#pragma unroll
-    for (uint32_t k = 0; k < U; ++k) {
-      va[k] = 0;
-      vg[k] = 0;
-      if (j + k < len && loads && !(deep_lane && rd_lane_u32(deep, j + k) == 0)) {
-        if (FIRST) {
-          // lanes < D read the column's records, lane D the compact deterministic bucket: one
-          // load instruction with per-lane addresses
-          const uint32_t mv = rd_lane_u32(m, j + k);
-          const unsigned char* src = in_col ? slab + (size_t)mv * g.row + coff
-                                            : reinterpret_cast<const unsigned char*>(det_cpy) + (size_t)mv * (8 + sizeof(G));
-          G gw;
-          ld_rec<G>(src, &va[k], &gw);
-          vg[k] = (uint64_t)gw;
-        } else {  // empty slots hold zeros, so the values need not wait for the roots
-          const uint64_t* e = in_part + (size_t)(p0 + j + k) * 2 * kWave;
-          va[k] = e[lane];
-          vg[k] = e[kWave + lane];
-        }
-      }
+  // The XOR of every prefix of the row's entries; a run is the XOR of two of them.  The runs are then
+  // taken in a loop over the places where one ends in some row (a uniform register index), not in 16
+  // unrolled copies of the sampling code, whose instruction fetches cost more than the sampling.
+  for_each_index(
+      [&](auto kc) {
+        constexpr uint32_t k = kc + 1;
+        lo[k] ^= lo[k - 1];
+        hi[k] ^= hi[k - 1];
+        glo[k] ^= glo[k - 1];
+        if constexpr (kWide) ghi[k] ^= ghi[k - 1];
+      },
+      std::make_integer_sequence<uint32_t, kRow - 1>{});
+  auto prefix = [&](uint32_t k, uint64_t* a, G* gm) {
+    *a = ((uint64_t)hi[k] << 32) | lo[k];
+    *gm = kWide ? (G)(((uint64_t)ghi[k] << 32) | glo[k]) : (G)glo[k];
+  };
+  // h: the row's first run, when it began before the row and ends inside it; acc: its last run
+  uint64_t acc, h_a = 0, tot, done_a = 0;
+  G accg, h_g = 0, totg, done_g = 0;
+  for (uint32_t at = (uint32_t)(starts | starts >> kRow | starts >> 2 * kRow | starts >> 3 * kRow) & 0xfffeu; at;
+       at &= at - 1) {
+    const uint32_t k = (uint32_t)__builtin_ctz(at);
+    uint64_t pa;
+    G pg;
+    prefix(k - 1, &pa, &pg);
+    const bool ends = (rowst >> k) & 1u;
+    const uint32_t earlier = rowst & ((1u << k) - 1);
+    if (ends && !earlier) {
+      h_a = pa;
+      h_g = pg;
     }
-#pragma unroll
-    for (uint32_t k = 0; k < U; ++k) {
-      if (j + k < len) {
-        const uint32_t R = rd_lane_u32(rt, j + k);
-        if (R != cur) {
-          emit(cur, acc_a, acc_g, seg_start, p0 + j + k);
-          acc_a = 0;
-          acc_g = 0;
-          cur = R;
-          seg_start = p0 + j + k;
-        }
-        acc_a ^= va[k];
-        acc_g ^= vg[k];
-        all_a ^= va[k];
-        all_g ^= vg[k];
+    emit(ends && earlier, pa ^ done_a, (G)(pg ^ done_g), __shfl((unsigned)rt, (int)(base + k - 1)),
+         base + 31u - (uint32_t)__builtin_clz(earlier | 1u));
+    if (ends) {
+      done_a = pa;
+      done_g = pg;
+    }
+  }
+  prefix(kRow - 1, &tot, &totg);
+  acc = tot ^ done_a;
+  accg = totg ^ done_g;
+  // carry each row's last run into the next row while it continues there
+  const bool cont = !(rowst & 1u), single = (rowst >> 1) == 0;
+  for (uint32_t r = 1; r < 4; ++r) {
+    if ((starts >> (kRow * r)) & 1) continue;  // uniform
+    const uint64_t ca = shfl_u64(acc, (int)(lane - kRow));
+    const G cg = sizeof(G) == 4 ? (G)__shfl((unsigned)accg, (int)(lane - kRow)) : (G)shfl_u64((uint64_t)accg, (int)(lane - kRow));
+    if (row == r) {
+      if (single) {
+        acc ^= ca;
+        accg ^= cg;
+      } else {
+        h_a ^= ca;
+        h_g ^= cg;
       }
     }
   }
-  emit(cur, acc_a, acc_g, seg_start, p1);
-  // an unused slot: no root, zero value (the next reduce reads values without looking at roots)
-  if (!wrote_head) put(head, kNoRoot, 0, 0);
-  if (!wrote_tail) put(tail, kNoRoot, 0, 0);
+  const uint64_t st_h = starts & low_bits(base), st_x = starts & low_bits(base + kRow);
+  const bool has_h = cont && !single;
+  const bool ends_x = row == 3 ? !tail_open : ((starts >> (base + kRow)) & 1) != 0;
+  if (__ballot(has_h && st_h)) {
+    const uint32_t f = 63u - (uint32_t)__builtin_clzll(st_h | 1ull);
+    emit(has_h && st_h, h_a, h_g, __shfl((unsigned)rt, (int)f), f);
+  }
+  if (__ballot(ends_x && st_x)) {
+    const uint32_t f = 63u - (uint32_t)__builtin_clzll(st_x | 1ull);
+    emit(ends_x && st_x, acc, accg, __shfl((unsigned)rt, (int)f), f);
+  }
+
+  // deep records: lane d < D of depths >= kRowDet; the XOR over the entries in lanes `of`
+  const uint64_t deep = g.D > kRowDet ? __ballot(mine && flag != 0) : 0;
+  auto deep_sum = [&](uint64_t of, uint64_t* a_out, G* g_out) {
+    const bool in = lane >= kRowDet && lane < g.D;
+    const unsigned char* dsrc = slab + (in ? rec_col_off<G>(g, round, lane) : 0u);
+    uint64_t a = 0;
+    G gm = 0;
+    constexpr uint32_t U = 8;  // loads in flight per lane
+    for (of &= deep; of;) {
+      uint64_t da[U];
+      G dg[U];
+#pragma unroll
+      for (uint32_t k = 0; k < U; ++k) {
+        da[k] = 0;
+        dg[k] = 0;
+        if (of) {
+          const uint32_t mv = rd_lane_u32(m, __builtin_ctzll(of));
+          of &= of - 1;
+          if (in) ld_rec<G>(dsrc + (size_t)mv * g.row, &da[k], &dg[k]);
+        }
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < U; ++k) {
+        a ^= da[k];
+        gm ^= dg[k];
+      }
+    }
+    *a_out = a;
+    *g_out = gm;
+  };
+  for (; again; again &= again - 1) {
+    const uint32_t f = (uint32_t)__builtin_ctzll(again);
+    const uint64_t later = starts & ~low_bits(f + 1);
+    const uint32_t end = later ? (uint32_t)__builtin_ctzll(later) : 64u;
+    uint64_t a;
+    G gm;
+    deep_sum(low_bits(end) & ~low_bits(f), &a, &gm);
+    const uint64_t good =
+        __ballot(lane >= kRowDet && lane < g.D && (G)xxh3_mix(xxh3_prep(a), g.chk_bf) == gm);
+    const uint32_t R = rd_lane_u32(rt, (int)f);
+    if (good ? lane == (uint32_t)__builtin_ctzll(good) : lane == 0)
+      samp[R] = sample_record(good ? kGood : kFail, a, g.n, flags);
+  }
+
+  // Every lane stores the root (the same value), so every lane of this wave may read it back
+  // without a barrier.  Slots are ordered by depth, the deterministic bucket at D.
+  const uint32_t pos = i == kRowDet ? g.D : i;
+  auto put = [&](Slot sl, uint32_t R, bool holds, uint64_t a, G gm, uint64_t of) {
+    uint64_t da;
+    G dg;
+    deep_sum(of, &da, &dg);
+    sl.vals[lane] = da;
+    sl.vals[kWave + lane] = (uint64_t)dg;
+    if (holds && live) {
+      sl.vals[pos] = a;
+      sl.vals[kWave + pos] = (uint64_t)gm;
+    }
+    *sl.root = R;
+  };
+  if (!(starts & 1)) {  // the first run began before the wave
+    const bool from_h = has_h && !st_h;
+    const bool from_x = row == 3 && tail_open ? !starts : (ends_x && !st_x);
+    put(head, first_root, from_h || from_x, from_h ? h_a : acc, from_h ? h_g : accg,
+        starts ? low_bits((uint32_t)__builtin_ctzll(starts)) : ~0ull);
+  } else {
+    put(head, kNoRoot, false, 0, 0, 0);
+  }
+  if (!tail_open) put(tail, kNoRoot, false, 0, 0, 0);
+  else if (!starts) put(tail, last_root, false, 0, 0, 0);
+  else put(tail, last_root, row == 3, acc, accg, ~low_bits(63u - (uint32_t)__builtin_clzll(starts)));
+  if (s_tot) {
+    uint64_t da;
+    G dg;
+    deep_sum(~0ull, &da, &dg);
+    if (da) lds_xor(s_tot + lane, da);
+    if (dg) lds_xor(s_tot + kWave + lane, (uint64_t)dg);
+    if (live) {
+      lds_xor(s_tot + pos, tot);
+      lds_xor(s_tot + kWave + pos, (uint64_t)totg);
+    }
+  }
   if (holds_first && lane < 2) s_bnd[lane] = bnd;
   if (holds_last && lane == 2) s_bnd[2] = bnd;
-  *all_a_out = all_a;
-  *all_g_out = all_g;
 }
 
 // Per lane: XOR (a, gm) into an accumulator slot with device-scope atomics (zero words skipped).
@@ -1609,14 +1744,12 @@ __device__ inline void xacc_add(uint64_t* slot, uint64_t a, uint64_t gm) {
   if (gm) __hip_atomic_fetch_xor(slot + kWave + lane, gm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// LDS of one reduce workgroup: 32 slots of 128 u64 and their roots, the giant total, the
-// workgroup's two unfinished supernodes and the segment bounds of its first and last entries.
+// LDS of one reduce workgroup: 32 slots of 128 u64 and their roots, the giant total and the segment
+// bounds of its first and last entries.
 #define GZ_REDUCE_LDS                                             \
   __shared__ uint64_t s_vals[2 * kRedWaves * 2 * kWave];          \
   __shared__ uint32_t s_root[2 * kRedWaves];                      \
   __shared__ uint64_t s_tot[2 * kWave];                           \
-  __shared__ uint64_t s_out[2 * 2 * kWave];                       \
-  __shared__ uint32_t s_oroot[2];                                 \
   __shared__ uint32_t s_bnd[3];
 
 // The reduce of a whole round: one workgroup per 1024 entries of the member list (e1 entries,
@@ -1652,11 +1785,7 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
   const uint32_t nblk = (e1 + span - 1) / span;
   const uint32_t b0 = blk * span;
   const uint32_t b1 = b0 + span < e1 ? b0 + span : e1;
-  auto root_at = [&](uint32_t p) -> uint32_t { return mroot[p]; };
   const bool giant_tot = giant != kNoRoot;
-  // neighbours of the workgroup's range, for phase 2; loaded early so they are in flight with phase 1
-  const uint32_t blk_prev = (wid == 0 && b0 > 0) ? root_at(b0 - 1) : kNoRoot;
-  const uint32_t blk_next = (wid == 0 && b1 < e1) ? root_at(b1) : kNoRoot;
   if (giant_tot)
     for (uint32_t k = threadIdx.x; k < 2 * kWave; k += blockDim.x) s_tot[k] = 0;
   __syncthreads();
@@ -1666,16 +1795,8 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
   Slot ts{s_vals + (size_t)(2 * wid + 1) * 2 * kWave, s_root + 2 * wid + 1};
   if (p0 < b1) {
     const uint32_t len = b1 - p0 < W ? b1 - p0 : W;
-    const uint32_t prev = p0 == 0 ? kNoRoot : root_at(p0 - 1);
-    const uint32_t next = p0 + len >= e1 ? kNoRoot : root_at(p0 + len);
-    uint64_t wa, wg;
-    reduce_range<G, true, true, kDeepFlags<G>>(p0, len, prev, next, members, nullptr, slab, g, round, nullptr,
-                                               nullptr, hs, ts, samp, flags, &wa, &wg, det_cpy, &xa, b0, b1, s_bnd,
-                                               mroot, deep_skip != 0);
-    if (giant_tot) {
-      lds_xor(s_tot + lane, wa);
-      lds_xor(s_tot + kWave + lane, wg);
-    }
+    reduce_members<G>(p0, len, W / 4, e1, members, mroot, slab, g, round, hs, ts, samp, flags, det_cpy, deep_skip != 0,
+                      giant_tot ? s_tot : nullptr, &xa, b0, b1, s_bnd);
   } else {
     hs.vals[lane] = 0;
     hs.vals[kWave + lane] = 0;
@@ -1687,53 +1808,64 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
     }
   }
   __syncthreads();
-  if (wid != 0) return;  // no barrier follows
-  // phase 2: wave 0 reduces the workgroup's 32 slots; the supernodes continuing past either end of
-  // the range are left in s_out
-  Slot oh{s_out, s_oroot}, ot{s_out + 2 * kWave, s_oroot + 1};
-  uint64_t wa, wg;
-  reduce_range<G, false>(0, 2 * kRedWaves, blk_prev, blk_next, nullptr, nullptr, nullptr, g, round, s_vals, s_root, oh,
-                         ot, samp, flags, &wa, &wg, nullptr, nullptr, 0, 0, nullptr);
-  if (nblk == 1) {  // one workgroup: nothing continues, and its total is the giant's whole sum
-    if (giant_tot) {
-      uint64_t idx;
-      const int code = wave_sample<G>(s_tot[lane], (G)s_tot[kWave + lane], g.D, g.chk_bf, &idx);
-      if (lane == 0) samp[giant] = sample_record(code, idx, g.n, flags);
+  // phase 2, no barrier follows: the supernodes that cross waves, each summed by one wave.  Lane w
+  // holds the head and tail roots of wave w.
+  const uint32_t nw = (b1 - b0 + W - 1) / W;  // waves with entries
+  const uint32_t hr = lane < nw ? s_root[2 * lane] : kNoRoot, tr = lane < nw ? s_root[2 * lane + 1] : kNoRoot;
+  // XOR the head slots of waves x, x + 1, ... that R covers whole, and of the one it ends in; returns
+  // whether it goes on past the workgroup
+  auto follow = [&](uint32_t R, uint32_t x, uint64_t& a, uint64_t& gm) -> bool {
+    const uint32_t whole = (uint32_t)__ballot(hr == R && tr == R) >> x;
+    const uint32_t open = x + (uint32_t)__builtin_ctz(~whole);
+    const uint32_t end = open < nw ? open + 1 : nw;
+#pragma unroll 4
+    for (; x < end; ++x) {
+      a ^= s_vals[(size_t)(2 * x) * 2 * kWave + lane];
+      gm ^= s_vals[(size_t)(2 * x) * 2 * kWave + kWave + lane];
     }
-    return;
-  }
-  // Cross-workgroup parts: the head supernode started in workgroup fh (its segment start), the
-  // tail one starts here; each ends in the workgroup holding its segment's last entry.
-  const uint32_t hr = s_oroot[0], tr = s_oroot[1];
-  const bool has_h = hr != kNoRoot;
-  const bool has_t = tr != kNoRoot && tr != hr;  // a supernode covering the whole range is counted once
-  const uint32_t fh = has_h ? s_bnd[0] / span : 0, lh = has_h ? (s_bnd[1] - 1) / span : 0;
-  const uint32_t lt = has_t ? (s_bnd[2] - 1) / span : 0;
-  const uint32_t gslot = xa.nslots - 1;
-  if (has_h) xacc_add(xa.vals + (size_t)fh * 2 * kWave, s_out[lane], s_out[kWave + lane]);
-  if (has_t) xacc_add(xa.vals + (size_t)blk * 2 * kWave, s_out[2 * kWave + lane], s_out[3 * kWave + lane]);
-  if (giant_tot) xacc_add(xa.vals + (size_t)gslot * 2 * kWave, s_tot[lane], s_tot[kWave + lane]);
-  __threadfence();  // the parts are visible before the arrival is counted
-  bool last = false;
-  if (lane == 0 && has_h) last = atomicAdd(xa.cnt + fh, 1u) == lh - fh;
-  if (lane == 1 && has_t) last = atomicAdd(xa.cnt + blk, 1u) == lt - blk;
-  if (lane == 2 && giant_tot) last = atomicAdd(xa.cnt + gslot, 1u) == nblk - 1;
-  const uint64_t wins = __ballot(last);
-  if (!wins) return;
-  __threadfence();  // every part counted before ours is visible
-  for (uint32_t k = 0; k < 3; ++k) {
-    if (!((wins >> k) & 1)) continue;
-    const uint32_t slot = k == 0 ? fh : k == 1 ? blk : gslot;
-    const uint32_t R = k == 0 ? hr : k == 1 ? tr : giant;
-    uint64_t* sv = xa.vals + (size_t)slot * 2 * kWave;
-    const uint64_t a = ld_acq(sv + lane), gm = ld_acq(sv + kWave + lane);
+    return open >= nw;
+  };
+  auto sample_to = [&](uint32_t R, uint64_t a, uint64_t gm) {
     uint64_t idx;
     const int code = wave_sample<G>(a, (G)gm, g.D, g.chk_bf, &idx);
     if (lane == 0) samp[R] = sample_record(code, idx, g.n, flags);
-    // cleared for the next round: every other part of this slot has been counted
+  };
+  // one of the `parts` workgroups that hold R adds its part to accumulator slot `slot`; the last one
+  // samples the sum and clears the slot for the next round
+  auto cross = [&](uint32_t slot, uint32_t parts, uint32_t R, uint64_t a, uint64_t gm) {
+    uint64_t* sv = xa.vals + (size_t)slot * 2 * kWave;
+    xacc_add(sv, a, gm);
+    __threadfence();  // the part is visible before the arrival is counted
+    uint32_t before = 0;
+    if (lane == 0) before = atomicAdd(xa.cnt + slot, 1u);
+    if (rd_lane_u32(before, 0) != parts - 1) return;
+    __threadfence();  // every part counted before ours is visible
+    sample_to(R, ld_acq(sv + lane), ld_acq(sv + kWave + lane));
     st_rlx(sv + lane, (uint64_t)0);
     st_rlx(sv + kWave + lane, (uint64_t)0);
     if (lane == 0) st_rlx(xa.cnt + slot, 0u);
+  };
+  if (wid < nw) {  // the supernode that starts in this wave and goes on
+    const uint32_t R = rd_lane_u32(tr, (int)wid);
+    if (R != kNoRoot && R != rd_lane_u32(hr, (int)wid)) {
+      const uint64_t* sl = s_vals + (size_t)(2 * wid + 1) * 2 * kWave;
+      uint64_t a = sl[lane], gm = sl[kWave + lane];
+      if (!follow(R, wid + 1, a, gm)) sample_to(R, a, gm);
+      else cross(blk, (s_bnd[2] - 1) / span - blk + 1, R, a, gm);  // it ends where its last entry is
+    }
+  }
+  if (wid == kRedWaves - 1) {  // the supernode that the workgroup's first entry continues
+    const uint32_t R = rd_lane_u32(hr, 0);
+    if (R != kNoRoot) {
+      uint64_t a = 0, gm = 0;
+      (void)follow(R, 0, a, gm);  // one covering the whole range is counted here only
+      const uint32_t fh = s_bnd[0] / span;
+      cross(fh, (s_bnd[1] - 1) / span - fh + 1, R, a, gm);
+    }
+  }
+  if (wid == kRedWaves - 2 && giant_tot) {
+    if (nblk == 1) sample_to(giant, s_tot[lane], s_tot[kWave + lane]);  // the giant's whole sum
+    else cross(xa.nslots - 1, nblk, giant, s_tot[lane], s_tot[kWave + lane]);
   }
 }
 
@@ -1748,7 +1880,7 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
 // It then sets mod[r] for every modified round, as the launched rounds do, and records the last
 // round it ran in mod[nmod - 1] (a word no round uses), so one copy of mod tells the host both.
 //
-// The workgroup reduces its grouped list in chunks of 64 entries (one wave each, reduce_range).  A
+// The workgroup reduces its grouped list in chunks of 64 entries (one wave each, reduce_members).  A
 // supernode continuing past a chunk is accumulated in LDS under the chunk where it starts (only one
 // supernode per chunk can continue past its end) and sampled after a barrier.  DSU and sample
 // loads that an earlier round of this kernel may have changed are device-coherent loads.
@@ -1781,7 +1913,7 @@ __global__ void __launch_bounds__(kRedBlock)
 k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ act0,
             const unsigned char* __restrict__ slab, Geo g, uint32_t r0, uint32_t last_round,
             uint64_t* __restrict__ samp, uint32_t* __restrict__ rstats, const unsigned char* __restrict__ det_cpy,
-            const unsigned char* __restrict__ hint, uint32_t* __restrict__ rep) {
+            const unsigned char* __restrict__ hint, uint32_t* __restrict__ rep, uint32_t deep_skip) {
   __shared__ uint32_t s_key[kFinishTable], s_cnt[kFinishTable];
   __shared__ uint32_t s_mem[kFinishMax], s_mroot[kFinishMax], s_seg[kFinishMax];
   __shared__ uint64_t s_acc[kFinishChunks * 2 * kWave];
@@ -1898,13 +2030,8 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     for (uint32_t c = wid; c < nchunks; c += kRedWaves) {
       const uint32_t p0 = c * cw;
       const uint32_t len = e - p0 < cw ? e - p0 : cw;
-      const uint32_t prev = p0 > 0 ? s_mroot[p0 - 1] : kNoRoot;
-      const uint32_t next = p0 + len < e ? s_mroot[p0 + len] : kNoRoot;
-      uint64_t wa, wg;
-      reduce_range<G, true, true>(p0, len, prev, next, s_mem, nullptr, slab, g, r, nullptr, nullptr, hs, ts, samp, d.flags,
-                            &wa, &wg, det_cpy, nullptr, 0, 0, nullptr, s_mroot);
-      lds_xor(s_tot + lane, wa);
-      lds_xor(s_tot + kWave + lane, wg);
+      reduce_members<G>(p0, len, cw / 4, e, s_mem, s_mroot, slab, g, r, hs, ts, samp, d.flags, det_cpy, deep_skip != 0,
+                        s_tot, nullptr, 0, 0, nullptr);
       const uint32_t hr = *hs.root, tr = *ts.root;
       if (hr != kNoRoot) {  // started in an earlier chunk
         uint64_t* acc = s_acc + (size_t)(s_seg[p0] / cw) * 2 * kWave;
@@ -2320,15 +2447,15 @@ void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const G
 }
 
 bool launch_finish(int gbytes, uint32_t r0, uint32_t last_round, const unsigned char* slab, const Geo& g,
-                   const DsuDev& d, const RoundBufs& rb, hipStream_t s, uint32_t* rep) {
+                   const DsuDev& d, const RoundBufs& rb, hipStream_t s, uint32_t* rep, bool deep_skip) {
   if (r0 < 2 || r0 > last_round) return false;  // round r0 walks round r0 - 1's member list
   const uint32_t* act0 = rb.members[(r0 - 1) & 1];
   if (gbytes == 4)
     hipLaunchKernelGGL(k_bv_finish<uint32_t>, dim3(1), dim3(kRedBlock), 0, s, d, rb.totals, act0, slab, g, r0,
-                       last_round, rb.samp, rb.rstats, rb.det_cpy, rb.hint, rep);
+                       last_round, rb.samp, rb.rstats, rb.det_cpy, rb.hint, rep, deep_skip ? 1u : 0u);
   else
     hipLaunchKernelGGL(k_bv_finish<uint64_t>, dim3(1), dim3(kRedBlock), 0, s, d, rb.totals, act0, slab, g, r0,
-                       last_round, rb.samp, rb.rstats, rb.det_cpy, rb.hint, rep);
+                       last_round, rb.samp, rb.rstats, rb.det_cpy, rb.hint, rep, deep_skip ? 1u : 0u);
   return true;
 }
 uint32_t finish_max() { return kFinishMax; }

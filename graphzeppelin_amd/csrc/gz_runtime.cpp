@@ -748,7 +748,7 @@ void GzAlg::enqueue_query_prefix(bool giant_ok, uint32_t last) {
   launch_dsu_reset(dsu, st, &rb);  // with the root counts and the round state words
   launch_sample_round0(gb, slab.p, geo, dsu, rb, st);
   for (uint32_t r = 1; r <= last; ++r) launch_round(gb, r, slab.p, geo, dsu, rb, giant_ok, st, use_deep_skip);
-  if (giant_ok && use_finish) launch_finish(gb, last + 1, geo.samples - 1, slab.p, geo, dsu, rb, st, rep.d);
+  if (giant_ok && use_finish) launch_finish(gb, last + 1, geo.samples - 1, slab.p, geo, dsu, rb, st, rep.d, use_deep_skip);
 }
 
 hipGraphExec_t GzAlg::get_query_graph(bool giant_ok, uint32_t last) {
@@ -849,7 +849,7 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
         throw GzError(GZ_ERR_OUT_OF_SAMPLES, "Borůvka needs more rounds than the sketches have samples");
       const uint32_t hi = std::min(next + 1, last_round);
       for (uint32_t r = next; r <= hi; ++r) launch_round(gb, r, slab.p, geo, dsu, rb, giant_ok, st, use_deep_skip);
-      reported = giant_ok && use_finish && launch_finish(gb, hi + 1, last_round, slab.p, geo, dsu, rb, st, rep.d);
+      reported = giant_ok && use_finish && launch_finish(gb, hi + 1, last_round, slab.p, geo, dsu, rb, st, rep.d, use_deep_skip);
       GZ_HIP(hipGetLastError());
       fin_r0 = hi + 1;
       next = hi + 1;
