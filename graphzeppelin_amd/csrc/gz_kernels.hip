@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <stdexcept>
+#include <type_traits>
 #include <utility>
 
 #include "gz_kernels.hpp"
@@ -664,174 +665,301 @@ k_make_tiles(const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ off,
   }
 }
 
-// Grouping by vertex without device-scope atomics (vertex counts up to 2^24): a bucket partition
-// over vertex ranges of R = 2^shift vertices (at most kPartBins ranges).
+// Grouping by vertex without device-scope atomics per update (vertex counts up to 2^24): a bucket
+// partition over bins of 2^shift vertices, then one workgroup per bin.
 //   1. k_part_hist: each workgroup takes a contiguous chunk of the pairs and counts the directed
-//      entries per range in LDS; the counts go to hist[range * nblk + block].
-//   2. an exclusive scan of hist (range-major), so each (range, block) owns a slot interval.
-//   3. k_part_scatter: the same chunks again; LDS cursors place the records (vertex, other end)
-//      in range order.
-//   4. k_part_group: one workgroup per range counts its vertices' entries in LDS, scans them, and
-//      writes cnt[v] and each vertex's destinations contiguously (vertex order, the same layout
-//      the vertex-count scan then gives).  The order of one vertex's destinations is arbitrary,
-//      which XOR does not see.
-constexpr uint32_t kPartBins = 4096, kPartBlock = 1024, kPartMaxBlocks = 256, kPartMaxRange = 4096;
+//      entries per bin in LDS; one device atomic per (workgroup, bin) gives its place in the bin.
+//   2. k_part_scatter: the same chunks again; LDS cursors place the records in bin order.
+//   3. k_part_group: one workgroup per bin counts its vertices' entries in LDS, scans them, writes
+//      each vertex's destinations contiguously and its tiles (the bin's share of the tile list taken
+//      with one device atomic).  The order of one vertex's destinations, and of the tiles, is
+//      arbitrary, which XOR does not see.
+// Bound by the scattered record writes (k_part_scatter: a workgroup's run in a bin is a few lines) and,
+// for small flushes, by the launches' latency.  Against contiguous ranges of ids, 8-byte records, a
+// count matrix with two scan launches and a per-vertex scan for the tiles (7 launches): 24M Chung-Lu
+// updates on 2^18 vertices 1025 -> 777 us, 16M R-MAT on 2^20 2190 -> 504 us (one range held 4% of the
+// entries), flushes of about 730k updates of a serving trace 87 -> 35 us.
+// A vertex's place p is its id times an odd number modulo 2^nb (a bijection), and its bin the high
+// bits of p: streams whose busy vertices sit side by side (R-MAT: the 256 lowest of 2^20 ids take 4% of
+// all entries) spread over the bins.  A record holds the place within the bin and the other end in
+// one word when both fit (PACK: nb + shift <= 32), else in two.
+constexpr uint32_t kPartBins = 1024, kPartBlock = 1024, kPartMaxBlocks = 256, kPartMaxShift = 14;
+constexpr uint32_t kPlaceMul = 2654435761u;  // odd, near 2^32 / the golden ratio
+constexpr uint32_t inverse_odd(uint32_t m) {  // Newton: each step doubles the correct low bits
+  uint32_t x = m;
+  for (int k = 0; k < 5; ++k) x *= 2u - m * x;
+  return x;
+}
+constexpr uint32_t kPlaceInv = inverse_odd(kPlaceMul);
+static_assert(kPlaceMul * kPlaceInv == 1u, "inverse modulo 2^32");
+
+template <bool PACK>
+struct PartRec {
+  using T = uint32_t;
+  static __device__ inline T make(uint32_t local, uint32_t other, uint32_t nb) { return (local << nb) | other; }
+  static __device__ inline uint32_t local(T r, uint32_t nb) { return r >> nb; }
+  static __device__ inline uint32_t other(T r, uint32_t nb) { return r & ((1u << nb) - 1); }
+};
+template <>
+struct PartRec<false> {
+  using T = uint2;
+  static __device__ inline T make(uint32_t local, uint32_t other, uint32_t) { return make_uint2(local, other); }
+  static __device__ inline uint32_t local(T r, uint32_t) { return r.x; }
+  static __device__ inline uint32_t other(T r, uint32_t) { return r.y; }
+};
 
 __device__ inline void part_chunk(size_t count, uint32_t nblk, size_t* lo, size_t* hi) {
   const size_t per = (count + nblk - 1) / nblk;
-  *lo = (size_t)blockIdx.x * per;
+  *lo = (size_t)blockIdx.x * per < count ? (size_t)blockIdx.x * per : count;
   *hi = *lo + per < count ? *lo + per : count;
 }
+// Calls f(pair) for the thread's pairs of [lo, hi), four loads in flight.
+template <class F>
+__device__ inline void part_walk(const uint2* __restrict__ pairs, size_t lo, size_t hi, F&& f) {
+  constexpr uint32_t U = 4;
+  size_t k = lo + threadIdx.x;
+  for (; k + (U - 1) * kPartBlock < hi; k += U * kPartBlock) {
+    uint2 p[U];
+#pragma unroll
+    for (uint32_t j = 0; j < U; ++j) p[j] = pairs[k + j * kPartBlock];
+#pragma unroll
+    for (uint32_t j = 0; j < U; ++j) f(p[j]);
+  }
+  for (; k < hi; k += kPartBlock) f(pairs[k]);
+}
+// Exclusive scan over a workgroup of kPartBlock threads.
+__device__ inline uint64_t part_scan(uint64_t x, uint64_t* wsum, uint64_t* total) {
+  const uint32_t lane = lane_id(), wid = threadIdx.x / kWave;
+  const uint64_t incl = wave_incl_scan_u64(x);
+  if (lane == kWave - 1) wsum[wid] = incl;
+  __syncthreads();
+  uint64_t pre = 0, tot = 0;
+  for (uint32_t w = 0; w < kPartBlock / kWave; ++w) {
+    const uint64_t v = wsum[w];
+    if (w < wid) pre += v;
+    tot += v;
+  }
+  *total = tot;
+  return pre + incl - x;
+}
 
+// binned: entries per bin, all zero on entry (k_part_group clears them); place: the workgroup's first
+// slot within each bin.  Also clears the tile count for k_part_group.
 __global__ void __launch_bounds__(kPartBlock)
-k_part_hist(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32_t shift, uint32_t bins, uint32_t nblk,
-            uint32_t* __restrict__ hist, uint32_t* __restrict__ bad_flag) {
+k_part_hist(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32_t nb, uint32_t shift, uint32_t bins,
+            uint32_t nblk, uint32_t* __restrict__ binned, uint32_t* __restrict__ place,
+            uint32_t* __restrict__ totals, uint32_t* __restrict__ bad_flag) {
   __shared__ uint32_t h[kPartBins];
-  for (uint32_t b = threadIdx.x; b < bins; b += kPartBlock) h[b] = 0;
+  if (threadIdx.x < bins) h[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) totals[1] = 0;
   __syncthreads();
   size_t lo, hi;
   part_chunk(count, nblk, &lo, &hi);
-  for (size_t k = lo + threadIdx.x; k < hi; k += kPartBlock) {
-    const uint2 p = pairs[k];
+  const uint32_t mask = (1u << nb) - 1;
+  part_walk(pairs, lo, hi, [&](uint2 p) {
     if (p.x >= n || p.y >= n) {
+      st_rlx(bad_flag, 1u);
+      return;
+    }
+    atomicAdd(h + (((p.x * kPlaceMul) & mask) >> shift), 1u);
+    atomicAdd(h + (((p.y * kPlaceMul) & mask) >> shift), 1u);
+  });
+  __syncthreads();
+  if (threadIdx.x < bins) {
+    const uint32_t c = h[threadIdx.x];
+    place[(size_t)blockIdx.x * bins + threadIdx.x] = c ? atomicAdd(binned + threadIdx.x, c) : 0u;
+  }
+}
+
+// binoff: bins + 1 words, the bins' starts in the record list.
+template <bool PACK>
+__global__ void __launch_bounds__(kPartBlock)
+k_part_scatter(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32_t nb, uint32_t shift, uint32_t bins,
+               uint32_t nblk, const uint32_t* __restrict__ binned, const uint32_t* __restrict__ place,
+               uint32_t* __restrict__ binoff, typename PartRec<PACK>::T* __restrict__ rec) {
+  __shared__ uint32_t cur[kPartBins];
+  __shared__ uint64_t wsum[kPartBlock / kWave];
+  const uint32_t t = threadIdx.x;
+  const uint32_t c = t < bins ? binned[t] : 0u;
+  const uint32_t pl = t < bins ? place[(size_t)blockIdx.x * bins + t] : 0u;
+  uint64_t tot;
+  const uint32_t off = (uint32_t)part_scan(c, wsum, &tot);
+  if (t < bins) cur[t] = off + pl;
+  if (blockIdx.x == 0) {
+    if (t < bins) binoff[t] = off;
+    if (t == 0) binoff[bins] = (uint32_t)tot;
+  }
+  __syncthreads();
+  size_t lo, hi;
+  part_chunk(count, nblk, &lo, &hi);
+  const uint32_t mask = (1u << nb) - 1, lmask = (1u << shift) - 1;
+  part_walk(pairs, lo, hi, [&](uint2 p) {
+    if (p.x >= n || p.y >= n) return;
+    const uint32_t px = (p.x * kPlaceMul) & mask, py = (p.y * kPlaceMul) & mask;
+    const uint32_t a = atomicAdd(cur + (px >> shift), 1u), b = atomicAdd(cur + (py >> shift), 1u);
+    rec[a] = PartRec<PACK>::make(px & lmask, p.y, nb);
+    rec[b] = PartRec<PACK>::make(py & lmask, p.x, nb);
+  });
+}
+
+// Writes the tiles of a vertex with c destinations starting at o, from tile t0 on, and returns their
+// algorithmic bytes (4c + 2 min(S, c * per_update)).
+__device__ inline uint64_t write_tiles(uint32_t v, uint32_t o, uint32_t c, uint32_t tile, Tile* __restrict__ tiles,
+                                       uint32_t t0, uint64_t S, uint64_t per_update) {
+  const uint32_t nt = (c + tile - 1) / tile;
+  for (uint32_t j = 0; j < nt; ++j) {
+    const uint32_t b = j * tile;
+    tiles[t0 + j] = Tile{v, o + b, (c - b) < tile ? (c - b) : tile, nt > 1 ? 1u : 0u};
+  }
+  const uint64_t touched = (uint64_t)c * per_update;
+  return 4ull * c + 2 * (touched < S ? touched : S);
+}
+// Adds a workgroup's profiling bytes to its slot of acc (nullptr: no profiling).
+__device__ inline void add_bytes(uint64_t* acc, uint64_t bytes) {
+  if (!acc) return;
+  for (int o = 32; o > 0; o >>= 1) bytes += shfl_xor_u64(bytes, o);
+  if (lane_id() == 0)
+    atomicAdd(reinterpret_cast<unsigned long long*>(acc + blockIdx.x % kProfSlots), (unsigned long long)bytes);
+}
+
+template <bool PACK>
+__global__ void __launch_bounds__(kPartBlock)
+k_part_group(const typename PartRec<PACK>::T* __restrict__ rec, uint32_t nb, uint32_t shift,
+             uint32_t* __restrict__ binned, const uint32_t* __restrict__ binoff, uint32_t* __restrict__ totals,
+             uint32_t* __restrict__ dst_arr, uint32_t tile, Tile* __restrict__ tiles, uint64_t* __restrict__ acc,
+             uint64_t S, uint64_t per_update) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint32_t* lc = reinterpret_cast<uint32_t*>(smem);  // 2^shift counters, then cursors
+  __shared__ uint64_t wsum[kPartBlock / kWave];
+  __shared__ uint32_t s_tile0;
+  const uint32_t b = blockIdx.x, R = 1u << shift, t = threadIdx.x;
+  const uint32_t s = binoff[b], e = binoff[b + 1];
+  if (t == 0) binned[b] = 0;
+  if (s == e) return;  // uniform over the workgroup
+  for (uint32_t k = t; k < R; k += kPartBlock) lc[k] = 0;
+  // the first kKeep records of every thread stay in registers between the two passes
+  constexpr uint32_t kKeep = 8;
+  typename PartRec<PACK>::T keep[kKeep];
+#pragma unroll
+  for (uint32_t k = 0; k < kKeep; ++k)
+    if (s + k * kPartBlock + t < e) keep[k] = rec[s + k * kPartBlock + t];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kKeep; ++k)
+    if (s + k * kPartBlock + t < e) atomicAdd(lc + PartRec<PACK>::local(keep[k], nb), 1u);
+  const uint32_t rest = s + kKeep * kPartBlock + t;
+  for (uint32_t j = rest; j < e; j += kPartBlock) atomicAdd(lc + PartRec<PACK>::local(rec[j], nb), 1u);
+  __syncthreads();
+  // exclusive scan of the entries and tiles per vertex: a thread owns `per` consecutive vertices
+  const uint32_t per = (R + kPartBlock - 1) / kPartBlock;
+  const uint32_t k0 = t * per;
+  uint64_t mine = 0;
+  for (uint32_t k = 0; k < per; ++k)
+    if (k0 + k < R) mine += pack_ct(lc[k0 + k], tile);
+  uint64_t tot;
+  uint64_t run = part_scan(mine, wsum, &tot);
+  if (t == 0) s_tile0 = atomicAdd(totals + 1, (uint32_t)(tot >> 32));
+  __syncthreads();
+  const uint32_t t0 = s_tile0, pmask = (1u << nb) - 1;
+  uint64_t bytes = 0;
+  for (uint32_t k = 0; k < per; ++k)
+    if (k0 + k < R) {
+      const uint32_t c = lc[k0 + k];
+      const uint32_t o = s + (uint32_t)run;
+      if (c)
+        bytes += write_tiles((((b << shift) | (k0 + k)) * kPlaceInv) & pmask, o, c, tile, tiles,
+                             t0 + (uint32_t)(run >> 32), S, per_update);
+      lc[k0 + k] = o;  // becomes the vertex's cursor
+      run += pack_ct(c, tile);
+    }
+  add_bytes(acc, bytes);
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kKeep; ++k)
+    if (s + k * kPartBlock + t < e)
+      dst_arr[atomicAdd(lc + PartRec<PACK>::local(keep[k], nb), 1u)] = PartRec<PACK>::other(keep[k], nb);
+  for (uint32_t j = rest; j < e; j += kPartBlock) {
+    const auto r = rec[j];
+    dst_arr[atomicAdd(lc + PartRec<PACK>::local(r, nb), 1u)] = PartRec<PACK>::other(r, nb);
+  }
+}
+
+// A flush of at most kSmallPairs updates in one workgroup, one launch instead of three: vertices are
+// counted in an LDS hash table (2^tbits slots, at least 4/3 of the entries), whose scan gives the
+// destinations' places and the tiles.  The limit is what 2^14 slots hold.  5000 updates: 29 us, where
+// the seven launches took 50 us and their gaps; 1000 updates: 8 us against 38.
+constexpr uint32_t kSmallPairs = 6144, kSmallPer = kSmallPairs / kPartBlock;
+__global__ void __launch_bounds__(kPartBlock)
+k_group_small(const uint2* __restrict__ pairs, uint32_t count, uint32_t n, uint32_t tbits, uint32_t* __restrict__ totals,
+              uint32_t* __restrict__ dst_arr, uint32_t tile, Tile* __restrict__ tiles, uint64_t* __restrict__ acc,
+              uint64_t S, uint64_t per_update, uint32_t* __restrict__ bad_flag) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ uint64_t wsum[kPartBlock / kWave];
+  const uint32_t T = 1u << tbits, t = threadIdx.x;
+  uint32_t* key = reinterpret_cast<uint32_t*>(smem);
+  uint32_t* cnt = key + T;
+  uint2 p[kSmallPer];
+#pragma unroll
+  for (uint32_t k = 0; k < kSmallPer; ++k) p[k] = k * kPartBlock + t < count ? pairs[k * kPartBlock + t] : make_uint2(0, 0);
+  for (uint32_t k = t; k < T; k += kPartBlock) {
+    key[k] = 0xFFFFFFFFu;  // no vertex: ids are below 2^31
+    cnt[k] = 0;
+  }
+  __syncthreads();
+  auto slot_of = [&](uint32_t v) -> uint32_t {
+    uint32_t h = (v * kPlaceMul) >> (32 - tbits);
+    while (true) {
+      const uint32_t prev = atomicCAS(key + h, 0xFFFFFFFFu, v);
+      if (prev == 0xFFFFFFFFu || prev == v) return h;
+      h = (h + 1) & (T - 1);
+    }
+  };
+  uint32_t sx[kSmallPer], sy[kSmallPer], ox[kSmallPer], oy[kSmallPer];
+#pragma unroll
+  for (uint32_t k = 0; k < kSmallPer; ++k) {
+    sx[k] = 0xFFFFFFFFu;
+    if (k * kPartBlock + t >= count) continue;
+    if (p[k].x >= n || p[k].y >= n) {
       st_rlx(bad_flag, 1u);
       continue;
     }
-    atomicAdd(h + (p.x >> shift), 1u);
-    atomicAdd(h + (p.y >> shift), 1u);
+    sx[k] = slot_of(p[k].x);
+    sy[k] = slot_of(p[k].y);
+    ox[k] = atomicAdd(cnt + sx[k], 1u);
+    oy[k] = atomicAdd(cnt + sy[k], 1u);
   }
   __syncthreads();
-  for (uint32_t b = threadIdx.x; b < bins; b += kPartBlock) hist[(size_t)b * nblk + blockIdx.x] = h[b];
-}
-
-__global__ void __launch_bounds__(kPartBlock)
-k_part_scatter(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32_t shift, uint32_t bins,
-               uint32_t nblk, const uint32_t* __restrict__ hoff, uint2* __restrict__ rec) {
-  __shared__ uint32_t cur[kPartBins];
-  for (uint32_t b = threadIdx.x; b < bins; b += kPartBlock) cur[b] = hoff[(size_t)b * nblk + blockIdx.x];
-  __syncthreads();
-  size_t lo, hi;
-  part_chunk(count, nblk, &lo, &hi);
-  for (size_t k = lo + threadIdx.x; k < hi; k += kPartBlock) {
-    const uint2 p = pairs[k];
-    if (p.x >= n || p.y >= n) continue;
-    rec[atomicAdd(cur + (p.x >> shift), 1u)] = make_uint2(p.x, p.y);
-    rec[atomicAdd(cur + (p.y >> shift), 1u)] = make_uint2(p.y, p.x);
-  }
-}
-
-__global__ void __launch_bounds__(kPartBlock)
-k_part_group(const uint2* __restrict__ rec, uint32_t n, uint32_t shift, uint32_t bins, uint32_t nblk,
-             const uint32_t* __restrict__ hoff, uint32_t* __restrict__ cnt, uint32_t* __restrict__ dst_arr) {
-  __shared__ uint32_t lc[kPartMaxRange];
-  __shared__ uint32_t wsum[kPartBlock / kWave];
-  const uint32_t b = blockIdx.x;
-  const uint32_t base = b << shift, R = 1u << shift;
-  const uint32_t nv = n - base < R ? n - base : R;
-  const uint32_t s = hoff[(size_t)b * nblk];
-  const uint32_t e = hoff[(size_t)(b + 1) * nblk];  // hoff[bins * nblk] holds the total
-  for (uint32_t k = threadIdx.x; k < R; k += kPartBlock) lc[k] = 0;
-  __syncthreads();
-  for (uint32_t j = s + threadIdx.x; j < e; j += kPartBlock) atomicAdd(lc + (rec[j].x - base), 1u);
-  __syncthreads();
-  // exclusive scan of lc[0..R): each thread owns a run of R / kPartBlock (>= 1) consecutive slots
-  const uint32_t per = (R + kPartBlock - 1) / kPartBlock;
-  const uint32_t k0 = threadIdx.x * per;
-  uint32_t mine = 0;
+  const uint32_t per = (T + kPartBlock - 1) / kPartBlock, k0 = t * per;
+  uint64_t mine = 0;
   for (uint32_t k = 0; k < per; ++k)
-    if (k0 + k < R) {
-      const uint32_t c = lc[k0 + k];
-      if (k0 + k < nv) cnt[base + k0 + k] = c;
-      mine += c;
-    }
-  const uint32_t lane = lane_id(), wid = threadIdx.x / kWave;
-  const uint64_t incl = wave_incl_scan_u64(mine);
-  if (lane == kWave - 1) wsum[wid] = (uint32_t)incl;
-  __syncthreads();
-  uint32_t run = (uint32_t)incl - mine;
-  for (uint32_t w = 0; w < wid; ++w) run += wsum[w];
-  for (uint32_t k = 0; k < per; ++k)
-    if (k0 + k < R) {
-      const uint32_t c = lc[k0 + k];
-      lc[k0 + k] = s + run;  // becomes the vertex's cursor
-      run += c;
-    }
-  __syncthreads();
-  for (uint32_t j = s + threadIdx.x; j < e; j += kPartBlock) {
-    const uint2 r = rec[j];
-    dst_arr[atomicAdd(lc + (r.x - base), 1u)] = r.y;
-  }
-}
-
-// The apply step of the scan when there are at most kScanBlock partials: every block adds up the
-// partials before its own (one per thread), so the separate block-sums launch is not needed, and
-// the last block writes the totals.  tiles != nullptr: each block also writes its vertices' tiles
-// (what k_make_tiles does), with the profiling bytes when acc != nullptr.
-__global__ void __launch_bounds__(kScanBlock)
-k_scan_apply_direct(const uint32_t* __restrict__ cnt, uint32_t n, uint32_t tile, const uint64_t* __restrict__ partials,
-                    uint32_t nparts, uint32_t* __restrict__ off, uint32_t* __restrict__ toff,
-                    uint32_t* __restrict__ cursor, uint32_t* __restrict__ totals, Tile* __restrict__ tiles,
-                    uint64_t* __restrict__ acc, uint64_t S, uint64_t per_update) {
-  uint64_t prefix;
-  block_excl_scan_u64(threadIdx.x < blockIdx.x ? partials[threadIdx.x] : 0, &prefix);
-  const uint32_t base = blockIdx.x * kScanSpan + threadIdx.x * kScanItems;
-  uint32_t c[kScanItems];
-  uint64_t s = 0;
-  for (int k = 0; k < kScanItems; ++k) {
-    const uint32_t i = base + k;
-    c[k] = i < n ? cnt[i] : 0;
-    s += pack_ct(c[k], tile);
-  }
+    if (k0 + k < T) mine += pack_ct(cnt[k0 + k], tile);
   uint64_t tot;
-  uint64_t run = block_excl_scan_u64(s, &tot) + prefix;
+  uint64_t run = part_scan(mine, wsum, &tot);
   uint64_t bytes = 0;
-  for (int k = 0; k < kScanItems; ++k) {
-    const uint32_t i = base + k;
-    if (i < n) {
-      off[i] = (uint32_t)run;
-      if (toff) toff[i] = (uint32_t)(run >> 32);
-      if (cursor) cursor[i] = (uint32_t)run;
-      if (tiles && c[k]) {
-        const uint32_t nt = (c[k] + tile - 1) / tile, o = (uint32_t)run, t0 = (uint32_t)(run >> 32);
-        for (uint32_t j = 0; j < nt; ++j) {
-          const uint32_t b = j * tile;
-          tiles[t0 + j] = Tile{i, o + b, (c[k] - b) < tile ? (c[k] - b) : tile, nt > 1 ? 1u : 0u};
-        }
-        const uint64_t touched = (uint64_t)c[k] * per_update;
-        bytes += 4ull * c[k] + 2 * (touched < S ? touched : S);
-      }
+  for (uint32_t k = 0; k < per; ++k)
+    if (k0 + k < T) {
+      const uint32_t c = cnt[k0 + k];
+      if (c) bytes += write_tiles(key[k0 + k], (uint32_t)run, c, tile, tiles, (uint32_t)(run >> 32), S, per_update);
+      cnt[k0 + k] = (uint32_t)run;
+      run += pack_ct(c, tile);
     }
-    run += pack_ct(c[k], tile);
-  }
-  if (blockIdx.x == nparts - 1 && threadIdx.x == 0) {
-    const uint64_t all = prefix + tot;
-    totals[0] = (uint32_t)all;
-    totals[1] = (uint32_t)(all >> 32);
-    off[n] = (uint32_t)all;
-    if (toff) toff[n] = (uint32_t)(all >> 32);
-  }
-  if (acc) {  // profiling: the block's algorithmic bytes
-    for (int o = 32; o > 0; o >>= 1) bytes += shfl_xor_u64(bytes, o);
-    if (lane_id() == 0)
-      atomicAdd(reinterpret_cast<unsigned long long*>(acc + blockIdx.x % kProfSlots), (unsigned long long)bytes);
+  if (t == 0) totals[1] = (uint32_t)(tot >> 32);
+  add_bytes(acc, bytes);
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kSmallPer; ++k) {
+    if (sx[k] == 0xFFFFFFFFu) continue;
+    dst_arr[cnt[sx[k]] + ox[k]] = p[k].y;
+    dst_arr[cnt[sy[k]] + oy[k]] = p[k].x;
   }
 }
 
-// Returns whether the tile list was written too (only when tiles != nullptr and the one-pass apply
-// was used).
-bool scan_counts(const uint32_t* cnt, uint32_t n, uint32_t tile, uint64_t* partials, uint32_t* off, uint32_t* toff,
-                 uint32_t* cursor, uint32_t* totals, hipStream_t s, Tile* tiles = nullptr,
-                 const FlushBytes* fb = nullptr) {
+void scan_counts(const uint32_t* cnt, uint32_t n, uint32_t tile, uint64_t* partials, uint32_t* off, uint32_t* toff,
+                 uint32_t* cursor, uint32_t* totals, hipStream_t s) {
   const uint32_t nparts = (n + kScanSpan - 1) / kScanSpan;
   hipLaunchKernelGGL(k_scan_partials, dim3(nparts), dim3(kScanBlock), 0, s, cnt, n, tile, partials);
-  if (nparts <= kScanBlock) {
-    hipLaunchKernelGGL(k_scan_apply_direct, dim3(nparts), dim3(kScanBlock), 0, s, cnt, n, tile, partials, nparts, off,
-                       toff, cursor, totals, tiles, fb ? fb->acc : nullptr, fb ? fb->S : 0, fb ? fb->per_update : 0);
-    return tiles != nullptr;
-  }
   hipLaunchKernelGGL(k_scan_block_sums, dim3(1), dim3(kScanBlock), 0, s, partials, nparts, n, off, toff, totals);
   hipLaunchKernelGGL(k_scan_apply, dim3(nparts), dim3(kScanBlock), 0, s, cnt, n, tile, partials, off, toff, cursor);
-  return false;
 }
 
 inline uint32_t grid_for(size_t work, uint32_t block, uint32_t cap = 8192) {
@@ -2301,39 +2429,75 @@ void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_d
 
 size_t group_partials_len(uint32_t n) { return (n + kScanSpan - 1) / kScanSpan + 1; }
 
+// Bits of a vertex's place, and the log2 of a bin's vertices.
+struct PartShape {
+  uint32_t nb, shift;
+};
+uint32_t part_bits(uint32_t n) {
+  uint32_t nb = 5;
+  while (nb < 24 && (1u << nb) < n) ++nb;
+  return nb;
+}
+// One-word records: 1024 bins of 2^(nb - 10) vertices leave nb - 10 bits of place beside nb bits of id.
+bool part_packed(uint32_t n) { return part_bits(n) <= 21; }
+// About 8192 entries a bin (what a workgroup keeps in registers between its passes), at least 64 bins
+// and at most kPartBins, of at most 2^kPartMaxShift vertices (the LDS counters) and at least 8.
+PartShape part_shape(uint32_t n, size_t count) {
+  const uint32_t nb = part_bits(n);
+  uint32_t lb = 6;
+  while (lb < 10 && (size_t(8192) << lb) < 2 * count) ++lb;
+  if (part_packed(n) && 2 * nb > 32 + lb) lb = 2 * nb - 32;
+  if (nb > kPartMaxShift + lb) lb = nb - kPartMaxShift;
+  if (lb + 3 > nb) lb = nb - 3;
+  return PartShape{nb, nb - lb};
+}
+
 void launch_group(const uint32_t* pairs, size_t count, uint32_t n, uint32_t tile, const GroupBufs& b, hipStream_t s,
                   const FlushBytes* fb) {
   const uint2* p2 = reinterpret_cast<const uint2*>(pairs);
-  uint32_t shift = 5;
-  while ((size_t(1) << shift) * kPartBins < n) ++shift;
-  if (b.rec && (1u << shift) <= kPartMaxRange) {
-    const uint32_t bins = (uint32_t)((n + (1u << shift) - 1) >> shift);
-    const uint32_t nblk = (uint32_t)std::max<size_t>(1, std::min<size_t>(kPartMaxBlocks, (count + 4095) / 4096));
-    const uint32_t hn = bins * nblk;
-    if (count) {
-      hipLaunchKernelGGL(k_part_hist, dim3(nblk), dim3(kPartBlock), 0, s, p2, count, n, shift, bins, nblk, b.hist,
-                         b.bad);
-    } else {
-      launch_fill_u32(b.hist, 0, hn, s);
-    }
-    scan_counts(b.hist, hn, 0, b.hpartials, b.hoff, nullptr, nullptr, b.htotals, s);
-    if (count)
-      hipLaunchKernelGGL(k_part_scatter, dim3(nblk), dim3(kPartBlock), 0, s, p2, count, n, shift, bins, nblk, b.hoff,
-                         b.rec);
-    hipLaunchKernelGGL(k_part_group, dim3(bins), dim3(kPartBlock), 0, s, b.rec, n, shift, bins, nblk, b.hoff, b.cnt,
-                       b.dst_arr);
-    if (scan_counts(b.cnt, n, tile, b.partials, b.off, b.toff, nullptr, b.totals, s, b.tiles, fb)) return;
-  } else {
-    launch_fill_u32(b.cnt, 0, n, s);
-    if (count) hipLaunchKernelGGL(k_count_pairs, dim3(grid_for(count, 256)), dim3(256), 0, s, p2, count, n, b.cnt, b.bad);
-    scan_counts(b.cnt, n, tile, b.partials, b.off, b.toff, b.cursor, b.totals, s);
-    if (count) hipLaunchKernelGGL(k_scatter_pairs, dim3(grid_for(count, 256)), dim3(256), 0, s, p2, count, n, b.cursor, b.dst_arr);
+  uint64_t* acc = fb ? fb->acc : nullptr;
+  const uint64_t S = fb ? fb->S : 0, per_update = fb ? fb->per_update : 0;
+  if (!count) {
+    launch_fill_u32(b.totals, 0, 2, s);
+    return;
   }
+  if (count <= kSmallPairs) {
+    uint32_t tbits = 10;
+    while ((2 * count) > (size_t(3) << tbits) / 4) ++tbits;  // at most three quarters full
+    const size_t lds = (size_t(8) << tbits);
+    hipLaunchKernelGGL(k_group_small, dim3(1), dim3(kPartBlock), lds, s, p2, (uint32_t)count, n, tbits, b.totals,
+                       b.dst_arr, tile, b.tiles, acc, S, per_update, b.bad);
+    return;
+  }
+  if (b.rec) {
+    const PartShape sh = part_shape(n, count);
+    const uint32_t nblk = (uint32_t)std::min<size_t>(kPartMaxBlocks, (count + 4095) / 4096);
+    const uint32_t bins = 1u << (sh.nb - sh.shift);
+    const size_t lds = size_t(4) << sh.shift;
+    hipLaunchKernelGGL(k_part_hist, dim3(nblk), dim3(kPartBlock), 0, s, p2, count, n, sh.nb, sh.shift, bins, nblk,
+                       b.binned, b.place, b.totals, b.bad);
+    auto go = [&](auto pack) {
+      constexpr bool PACK = decltype(pack)::value;
+      auto* rec = reinterpret_cast<typename PartRec<PACK>::T*>(b.rec);
+      hipLaunchKernelGGL(k_part_scatter<PACK>, dim3(nblk), dim3(kPartBlock), 0, s, p2, count, n, sh.nb, sh.shift, bins,
+                         nblk, b.binned, b.place, b.binoff, rec);
+      hipLaunchKernelGGL(k_part_group<PACK>, dim3(bins), dim3(kPartBlock), lds, s, rec, sh.nb, sh.shift, b.binned,
+                         b.binoff, b.totals, b.dst_arr, tile, b.tiles, acc, S, per_update);
+    };
+    if (part_packed(n)) go(std::true_type{});
+    else go(std::false_type{});
+    return;
+  }
+  launch_fill_u32(b.cnt, 0, n, s);
+  hipLaunchKernelGGL(k_count_pairs, dim3(grid_for(count, 256)), dim3(256), 0, s, p2, count, n, b.cnt, b.bad);
+  scan_counts(b.cnt, n, tile, b.partials, b.off, b.toff, b.cursor, b.totals, s);
+  hipLaunchKernelGGL(k_scatter_pairs, dim3(grid_for(count, 256)), dim3(256), 0, s, p2, count, n, b.cursor, b.dst_arr);
   hipLaunchKernelGGL(k_make_tiles, dim3(grid_for(n, 256, kProfSlots)), dim3(256), 0, s, b.cnt, b.off, b.toff, n, tile,
-                     b.tiles, fb ? fb->acc : nullptr, fb ? fb->S : 0, fb ? fb->per_update : 0);
+                     b.tiles, acc, S, per_update);
 }
 
-size_t part_hist_len() { return (size_t)kPartBins * kPartMaxBlocks + 1; }
+size_t part_place_len() { return (size_t)kPartBins * kPartMaxBlocks; }
+size_t part_bins_len() { return kPartBins + 1; }
 
 // A large batch on an instance that no query has ranked gets classes first and is merged in launches
 // of doubling size.  The time of the first merges is failed CAS attempts on hubs' words: every update

@@ -49,23 +49,27 @@ size_t update_tiles_lds_bytes(const Geo& g, int gbytes);
 
 // ---- grouping of a device-resident stream of (src,dst) pairs into per-vertex tiles ----
 struct GroupBufs {
+  uint32_t* totals;    // [1] the tile count
+  uint32_t* dst_arr;   // 2 * max_pairs
+  Tile* tiles;         // max tiles
+  uint32_t* bad;       // set to 1 when a pair names a vertex >= n
+  // bucket partition (up to 2^24 vertices; null above)
+  void* rec;           // 2 * max_pairs records (vertex, other end): part_rec_bytes(n) each
+  uint32_t* binned;    // part_bins_len() entries per bin, zero between flushes
+  uint32_t* binoff;    // part_bins_len() starts of the bins
+  uint32_t* place;     // part_place_len() first slot of each workgroup in each bin
+  // counting with device atomics (above 2^24 vertices; null otherwise)
   uint32_t* cnt;       // n      per-vertex directed-update counts (zeroed by launch_group)
   uint32_t* off;       // n + 1  exclusive scan of cnt
   uint32_t* toff;      // n + 1  exclusive scan of per-vertex tile counts
   uint32_t* cursor;    // n      scatter cursors
-  uint64_t* partials;  // scan block partials
-  uint32_t* totals;    // [0] total directed updates, [1] total tiles
-  uint32_t* dst_arr;   // 2 * max_pairs
-  Tile* tiles;         // max tiles
-  uint32_t* bad;       // set to 1 when a pair names a vertex >= n
-  // bucket partition (used when non-null and the vertex count allows it)
-  uint2* rec;          // 2 * max_pairs records (vertex, other end)
-  uint32_t* hist;      // part_hist_len()
-  uint32_t* hoff;      // part_hist_len()
-  uint64_t* hpartials; // group_partials_len(part_hist_len())
-  uint32_t* htotals;   // 4
+  uint64_t* partials;  // group_partials_len(n) scan block partials
 };
-size_t part_hist_len();
+constexpr uint32_t kPartMaxVertices = 1u << 24;
+bool part_packed(uint32_t n);
+inline size_t part_rec_bytes(uint32_t n) { return part_packed(n) ? 4 : 8; }
+size_t part_place_len();
+size_t part_bins_len();
 size_t group_partials_len(uint32_t n);
 // pairs: 2*count u32 (src,dst) in HBM.  Produces tiles of at most `tile` destinations.
 // Profiling: per-block accumulators of a grouped flush's algorithmic bytes (kProfSlots u64,

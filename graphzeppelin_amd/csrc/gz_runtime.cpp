@@ -268,22 +268,31 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   pending.alloc(2 * cap_pairs);
   dst_arr.alloc(2 * cap_pairs);
   merged.alloc(cap_pairs);
-  g_cnt.alloc(n); g_off.alloc(n + 1); g_toff.alloc(n + 1); g_cursor.alloc(n); g_totals.alloc(4);
-  g_partials.alloc(group_partials_len(n));
+  g_totals.alloc(4);
   g_tiles.alloc(2 * cap_pairs / tile + n + 1);
-  gbufs = GroupBufs{g_cnt.p, g_off.p, g_toff.p, g_cursor.p, g_partials.p, g_totals.p, dst_arr.p, g_tiles.p,
-                    flags.p + kFlagBadInput, nullptr, nullptr, nullptr, nullptr, nullptr};
-  if (n <= (1u << 24)) {  // bucket-partition grouping (no device-scope atomics)
-    g_rec.alloc(2 * cap_pairs);
-    g_hist.alloc(part_hist_len());
-    g_hoff.alloc(part_hist_len());
-    g_hpartials.alloc(group_partials_len((uint32_t)part_hist_len()));
-    g_htotals.alloc(4);
+  gbufs = GroupBufs{};
+  gbufs.totals = g_totals.p;
+  gbufs.dst_arr = dst_arr.p;
+  gbufs.tiles = g_tiles.p;
+  gbufs.bad = flags.p + kFlagBadInput;
+  if (n <= kPartMaxVertices) {  // bucket-partition grouping (no device-scope atomics per update)
+    g_rec.alloc(2 * cap_pairs * part_rec_bytes(n));
+    g_place.alloc(part_place_len());
+    g_binned.alloc(part_bins_len());
+    g_binoff.alloc(part_bins_len());
+    launch_fill_u32(g_binned.p, 0, g_binned.n, st);
     gbufs.rec = g_rec.p;
-    gbufs.hist = g_hist.p;
-    gbufs.hoff = g_hoff.p;
-    gbufs.hpartials = g_hpartials.p;
-    gbufs.htotals = g_htotals.p;
+    gbufs.place = g_place.p;
+    gbufs.binned = g_binned.p;
+    gbufs.binoff = g_binoff.p;
+  } else {
+    g_cnt.alloc(n); g_off.alloc(n + 1); g_toff.alloc(n + 1); g_cursor.alloc(n);
+    g_partials.alloc(group_partials_len(n));
+    gbufs.cnt = g_cnt.p;
+    gbufs.off = g_off.p;
+    gbufs.toff = g_toff.p;
+    gbufs.cursor = g_cursor.p;
+    gbufs.partials = g_partials.p;
   }
 
   // host staging

@@ -180,9 +180,8 @@ class GzAlg {
   size_t pending_n = 0;  // pairs copied into `pending`
   const uint32_t* ref_pairs = nullptr;  // pairs referenced in the caller's memory (ingest_device_stable)
   size_t ref_n = 0;
-  DevBuf<uint32_t> pending, dst_arr, g_cnt, g_off, g_toff, g_cursor, g_totals, g_hist, g_hoff, g_htotals;
-  DevBuf<uint2> g_rec;
-  DevBuf<uint64_t> g_hpartials;
+  DevBuf<uint32_t> pending, dst_arr, g_cnt, g_off, g_toff, g_cursor, g_totals, g_place, g_binned, g_binoff;
+  DevBuf<uint8_t> g_rec;
   DevBuf<uint64_t> g_partials;
   DevBuf<Tile> g_tiles;
   DevBuf<uint8_t> merged;
