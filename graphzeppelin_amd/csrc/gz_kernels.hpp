@@ -37,6 +37,12 @@ void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 void launch_fill_u64(uint64_t* p, uint64_t v, size_t n, hipStream_t s);
 
 // ---- sketch update ----
+// Destinations per tile when the configuration names none.  A tile is one wave's work, so the longest
+// tiles set the launch's tail when hubs come last, and each tile of a split vertex writes back with
+// atomics.  Update kernel at 1024 / 512 / 256 / 128: 24M Chung-Lu updates on 2^18 vertices 2521 / 2340 /
+// 2153 / 2670 us, 16M R-MAT on 2^20 2442 / 2329 / 2189 / 3267 us, 3M R-MAT on 2^17 with 8-byte
+// checksums 540 / 473 / 412 / 385 us, flushes of a serving trace 214 / 213 / 206 / 200 us.
+constexpr uint32_t kDefaultTile = 256;
 // Tile kernel (one wave per tile).  `ntiles_dev` (device scalar) bounds the tile index when
 // non-null (persistent grid of grid_cap workgroups), otherwise `ntiles_host` (one workgroup per
 // tile, at most grid_cap when grid_cap > 0).  Workgroups walk tiles grid-stride.

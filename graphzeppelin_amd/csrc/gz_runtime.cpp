@@ -196,7 +196,7 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   require_device();
   geo = make_geo(n, calc_vector_length(n), seed, calc_cc_samples(n, cfg.sketches_factor), 1, gb);
   if (update_tiles_lds_bytes(geo, gb) > 64 * 1024) throw GzError(GZ_ERR_INVALID_ARG, "sketch too large for LDS");
-  tile = cfg.tile ? cfg.tile : 1024;
+  tile = cfg.tile ? cfg.tile : kDefaultTile;
   const size_t lds = update_tiles_lds_bytes(geo, gb);
   // one-wave workgroups: up to 32 per CU (8 waves on each of 4 SIMDs), fewer if LDS runs out
   const size_t per_cu = std::max<size_t>(1, std::min<size_t>(32, (160 * 1024) / lds));
