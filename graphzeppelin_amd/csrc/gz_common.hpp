@@ -33,12 +33,18 @@ __host__ __device__ inline uint64_t xxh3_bitflip(uint64_t seed) {
 // rot32(idx): the input is read as two little-endian 32-bit words and recombined hi + (lo << 32)
 __host__ __device__ inline uint64_t xxh3_prep(uint64_t idx) { return (idx >> 32) | (idx << 32); }
 
-__host__ __device__ inline uint64_t xxh3_mix(uint64_t prepped, uint64_t bitflip) {
-  uint64_t h = prepped ^ bitflip;
-  h ^= rotl64(h, 49) ^ rotl64(h, 24);
+// rrmxmx starts with h ^ rotl(h, 49) ^ rotl(h, 24), which XOR goes through: the index and the bitflip
+// can be spread apart and combined afterwards, spread(a ^ b) = spread(a) ^ spread(b).
+__host__ __device__ inline uint64_t xxh3_spread(uint64_t x) { return x ^ rotl64(x, 49) ^ rotl64(x, 24); }
+// The rest of rrmxmx up to its last step, h ^ (h >> 28).
+__host__ __device__ inline uint64_t xxh3_products(uint64_t h) {
   h *= kPrimeMx2;
   h ^= (h >> 35) + 8;
-  h *= kPrimeMx2;
+  return h * kPrimeMx2;
+}
+
+__host__ __device__ inline uint64_t xxh3_mix(uint64_t prepped, uint64_t bitflip) {
+  const uint64_t h = xxh3_products(xxh3_spread(prepped ^ bitflip));
   return h ^ (h >> 28);
 }
 

@@ -322,7 +322,15 @@ __global__ void k_fill_u64(uint64_t* p, uint64_t v, size_t n) {
 // rare deeper contributions (one pair in 2^kLdsDepth) are XORed straight into the vertex's records
 // with device-scope atomics (setting the column's deep flag when the record lies past the first
 // line of the column's overflow run).  The deterministic bucket is kept in registers and reduced
-// once per tile.  The write-back is a read-xor-write of the touched records, or device-scope
+// once per tile.
+// Long tiles are bound by VALU issue (a pair's hash is two 64-bit products, six quarter-rate
+// multiplies of about 50 instructions before), so everything of the hash that is linear is taken out
+// of the pairs: an update's index and a column's bitflip are spread once (xxh3_spread) and a pair
+// XORs them; the depth is read from the hash's low word, the exact one only where it leaves the LDS
+// delta; indices are rebuilt from the other end, so the pair still costs one 16-byte LDS read.  24M
+// Chung-Lu updates on 2^18 vertices 2153 -> 1653 us (216 SIMD cycles per 64 pairs), 16M R-MAT on 2^20
+// 2189 -> 1627 us, flushes of a serving trace (about 6 updates per vertex, bound by the tiles' memory
+// round trips) 206 -> 199 us.  The write-back is a read-xor-write of the touched records, or device-scope
 // atomic XOR when the vertex is split across tiles of the same launch.  Workgroups walk the tiles
 // grid-stride (no shared counter), so a persistent grid can cover a tile count that only the
 // device knows.
@@ -343,15 +351,19 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
   const uint32_t C = g.C, D = g.D;
   const uint32_t det_slot = C * kLdsPitch;
   const uint32_t lds_n = det_slot + 1;
-  // per chunk: each update's pre-mixed index and checksum, read by the lanes that take its columns
+  // per chunk, read by the lanes that take an update's columns: its spread index, and the other end
+  // and the checksum (kTight: one 16-byte slot), or the index with the checksum in an array of its own
+  constexpr bool kTight = !RAW && sizeof(G) == 4;
   ulonglong2* s_pc = reinterpret_cast<ulonglong2*>(smem);
-  uint64_t* s_bf = reinterpret_cast<uint64_t*>(smem + kWave * sizeof(ulonglong2));
+  uint64_t* s_bf = reinterpret_cast<uint64_t*>(smem + kWave * sizeof(ulonglong2));  // spread bitflips
   uint64_t* s_a = s_bf + C;
   G* s_g = reinterpret_cast<G*>(s_a + lds_n);
-  uint32_t* s_bo = reinterpret_cast<uint32_t*>(s_g + lds_n);  // each delta entry's byte in the row
+  G* s_ck = s_g + lds_n;
+  uint16_t* s_bo = reinterpret_cast<uint16_t*>(s_ck + (kTight ? 0 : kWave));  // each delta entry's word in the row
   const uint32_t lane = threadIdx.x;
 
-  for (uint32_t i = lane; i < C; i += kWave) s_bf[i] = col_bf[i];
+  for (uint32_t i = lane; i < C; i += kWave) s_bf[i] = xxh3_spread(col_bf[i]);
+  const uint64_t chk_sbf = xxh3_spread(g.chk_bf);
   // The delta is zeroed once here; afterwards the write-back clears every entry it reads.  Entries
   // at depth >= D (or at a pitch padding, if the pitch exceeds kLdsDepth) are never written:
   // offset 0.
@@ -359,10 +371,12 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
     s_a[i] = 0;
     s_g[i] = 0;
     const uint32_t cc = i / kLdsPitch, d = i - cc * kLdsPitch;
-    s_bo[i] = i == det_slot ? det_col_off(g) : (d < kLdsDepth && d < D ? rec_col_off<G>(g, cc, d) : 0u);
+    s_bo[i] =
+        (uint16_t)((i == det_slot ? det_col_off(g) : (d < kLdsDepth && d < D ? rec_col_off<G>(g, cc, d) : 0u)) / 4);
   }
   const uint32_t ntiles = ntiles_dev ? *ntiles_dev : ntiles_host;
   const uint64_t depth_cap = 1ull << D;
+  const uint32_t lds_d = D < kLdsDepth ? D : kLdsDepth;
   // pair p = i * C + c: lane starts at pair `lane` and advances 64 pairs (di updates, dc columns)
   const uint32_t i0 = lane / C, c0 = lane % C;
   const uint32_t di = kWave / C, dc = kWave % C;
@@ -387,16 +401,17 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
   G det_g = 0;
   auto hash_chunk = [&](const Tile& tt, uint32_t u0, uint64_t raw) {
     const uint32_t m = tt.count - u0 < kWave ? tt.count - u0 : kWave;
-    uint64_t my_pre = 0;
-    G my_chk = 0;
     if (lane < m) {
       const uint64_t idx = to_idx(tt, raw);
-      my_pre = xxh3_prep(idx);
-      my_chk = (G)xxh3_mix(my_pre, g.chk_bf);
+      const uint64_t sp = xxh3_spread(xxh3_prep(idx));
+      uint64_t ck = xxh3_products(sp ^ chk_sbf);
+      ck ^= ck >> 28;
       det_a ^= idx;
-      det_g ^= my_chk;
+      det_g ^= (G)ck;
+      // the wave's LDS ops stay in order
+      s_pc[lane] = make_ulonglong2(sp, kTight ? (ck << 32) | (uint32_t)raw : idx);
+      if (!kTight) s_ck[lane] = (G)ck;
     }
-    s_pc[lane] = make_ulonglong2(my_pre, (uint64_t)my_chk);  // the wave's LDS ops stay in order
   };
   uint32_t t = blockIdx.x;
   Tile tl{0, 0, 0, 0};
@@ -416,17 +431,22 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
       for (uint32_t it = 0; it < iters; ++it) {
         if (it * kWave + lane < np) {  // q < m here
           const ulonglong2 pc = s_pc[q];
-          const uint64_t pre = pc.x;
-          const G chk = (G)pc.y;
-          const uint64_t idx = (pre << 32) | (pre >> 32);  // xxh3_prep swaps the halves
-          const uint64_t h = xxh3_mix(pre, s_bf[c]);
-          const uint32_t depth = (uint32_t)__builtin_ctzll(h | depth_cap);  // == D: no bucket
-          if (depth < D) {
-            if (depth < kLdsDepth) {
-              const uint32_t li = c * kLdsPitch + depth;
-              lds_xor(s_a + li, idx);
-              lds_xor(s_g + li, chk);
-            } else {
+          const uint64_t h = xxh3_products(pc.x ^ s_bf[c]);
+          const G chk = kTight ? (G)(pc.y >> 32) : s_ck[q];
+          const uint64_t idx = kTight ? concat_pairing(tl.vertex, (uint32_t)pc.y) : pc.y;
+          // the depth from the hash's low word, whose bits decide every depth below kLdsDepth
+          const uint32_t low = (uint32_t)h ^ __builtin_amdgcn_alignbit((uint32_t)(h >> 32), (uint32_t)h, 28);
+          const uint32_t near = (uint32_t)__builtin_ctz(low | (1u << kLdsDepth));
+          if (near < lds_d) {
+            uint32_t c9;  // c * kLdsPitch: the compiler's choice is a quarter-rate multiply
+            asm("v_lshl_add_u32 %0, %1, 3, %1" : "=v"(c9) : "v"(c));
+            static_assert(kLdsPitch == 9, "c9");
+            const uint32_t li = c9 + near;
+            lds_xor(s_a + li, idx);
+            lds_xor(s_g + li, chk);
+          } else {
+            const uint32_t depth = (uint32_t)__builtin_ctzll((h ^ (h >> 28)) | depth_cap);  // == D: no bucket
+            if (depth < D) {
               xor_rec_atomic<G>(row + rec_col_off<G>(g, c, depth), idx, chk);
               if (kDeepFlags<G> && rec_is_deep(g, depth))  // the flag only ever goes from 0 to 1
                 st_rlx(reinterpret_cast<uint32_t*>(row + deep_flag_off(c)), 1u);
@@ -476,7 +496,7 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
         dg[k] = 0;
         bo[k] = 0;
         if (e < lds_n) {
-          bo[k] = s_bo[e];
+          bo[k] = (uint32_t)s_bo[e] * 4u;
           da[k] = s_a[e];
           dg[k] = s_g[e];
           if ((da[k] | (uint64_t)dg[k]) != 0) {
@@ -2402,7 +2422,7 @@ void launch_fill_u64(uint64_t* p, uint64_t v, size_t n, hipStream_t s) {
 
 size_t update_tiles_lds_bytes(const Geo& g, int gbytes) {
   const size_t lds_n = (size_t)g.C * kLdsPitch + 1;
-  return kWave * 16 + g.C * 8 + lds_n * 8 + lds_n * (size_t)gbytes + lds_n * 4;
+  return kWave * 16 + g.C * 8 + lds_n * 8 + (lds_n + kWave) * (size_t)gbytes + lds_n * 2;
 }
 
 void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_dev, uint32_t ntiles_host,
