@@ -296,7 +296,7 @@ class Sketch:
 
     def update_batch_device_noalloc(self, idx_device_ptr: int, count: int):
         """update_batch over `count` uint64 indices in device memory, allocating nothing (at most
-        2^26 indices per call; calls that overlap on one GPU race)."""
+        2^26 indices per call)."""
         _check(lib().gz_sketch_update_batch_device_noalloc(self._h, ctypes.c_void_p(idx_device_ptr), count))
 
     def sample(self):

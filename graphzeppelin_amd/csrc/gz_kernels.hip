@@ -342,18 +342,18 @@ constexpr unsigned kWaitVmcnt0 = 0x0F70;
 // WIDE: more than 28 columns, so the write-back takes more than one pass over the LDS delta (a
 // separate instance keeps the one-pass form free of the loop, whose merged paths would make the
 // compiler wait on this tile's stores at the next tile's first use of the prefetch register).
-template <class G, bool RAW, bool WIDE>
+template <class G, bool WIDE>
 __global__ void __launch_bounds__(kWave, 8)  // 8 waves per SIMD: 32 tiles in flight per CU
 k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntiles_dev, uint32_t ntiles_host,
-               const uint32_t* __restrict__ dsts, const uint64_t* __restrict__ raw_idx,
-               unsigned char* __restrict__ slab, Geo g, const uint64_t* __restrict__ col_bf) {
+               const uint32_t* __restrict__ dsts, unsigned char* __restrict__ slab, Geo g,
+               const uint64_t* __restrict__ col_bf) {
   extern __shared__ __align__(16) unsigned char smem[];
   const uint32_t C = g.C, D = g.D;
   const uint32_t det_slot = C * kLdsPitch;
   const uint32_t lds_n = det_slot + 1;
   // per chunk, read by the lanes that take an update's columns: its spread index, and the other end
   // and the checksum (kTight: one 16-byte slot), or the index with the checksum in an array of its own
-  constexpr bool kTight = !RAW && sizeof(G) == 4;
+  constexpr bool kTight = sizeof(G) == 4;
   ulonglong2* s_pc = reinterpret_cast<ulonglong2*>(smem);
   uint64_t* s_bf = reinterpret_cast<uint64_t*>(smem + kWave * sizeof(ulonglong2));  // spread bitflips
   uint64_t* s_a = s_bf + C;
@@ -385,31 +385,25 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
   // Updates are taken in chunks of 64: lane l loads update u0 + l once and hashes its index and
   // checksum once into a 16-byte LDS slot; the chunk's (update, column) pairs then read their
   // update's slot with one LDS load, so each pair costs one column hash and no memory round trip.
-  // The next tile's descriptor and each lane's first destination (or raw index) are loaded
+  // The next tile's descriptor and each lane's first destination are loaded
   // before the current tile's write-back, and that chunk is hashed between the write-back's
   // record loads and its stores, where the wave waits for those loads anyway.  No tile then
   // starts with a wait, which would also wait for the previous tile's stores (the vector memory
   // counter covers stores too).
-  auto load_raw = [&](const Tile& tt, uint32_t u) -> uint64_t {
-    return RAW ? raw_idx[tt.begin + u] : (uint64_t)dsts[tt.begin + u];
-  };
-  auto to_idx = [&](const Tile& tt, uint64_t w) -> uint64_t {
-    return RAW ? w : concat_pairing(tt.vertex, (uint32_t)w);
-  };
   // per-lane XOR of the tile's indices and checksums: the deterministic bucket's delta
   uint64_t det_a = 0;
   G det_g = 0;
-  auto hash_chunk = [&](const Tile& tt, uint32_t u0, uint64_t raw) {
+  auto hash_chunk = [&](const Tile& tt, uint32_t u0, uint32_t dst) {
     const uint32_t m = tt.count - u0 < kWave ? tt.count - u0 : kWave;
     if (lane < m) {
-      const uint64_t idx = to_idx(tt, raw);
+      const uint64_t idx = concat_pairing(tt.vertex, dst);
       const uint64_t sp = xxh3_spread(xxh3_prep(idx));
       uint64_t ck = xxh3_products(sp ^ chk_sbf);
       ck ^= ck >> 28;
       det_a ^= idx;
       det_g ^= (G)ck;
       // the wave's LDS ops stay in order
-      s_pc[lane] = make_ulonglong2(sp, kTight ? (ck << 32) | (uint32_t)raw : idx);
+      s_pc[lane] = make_ulonglong2(sp, kTight ? (ck << 32) | dst : idx);
       if (!kTight) s_ck[lane] = (G)ck;
     }
   };
@@ -417,14 +411,14 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
   Tile tl{0, 0, 0, 0};
   if (t < ntiles) {
     tl = tiles[t];
-    hash_chunk(tl, 0, lane < tl.count ? load_raw(tl, lane) : 0);
+    hash_chunk(tl, 0, lane < tl.count ? dsts[tl.begin + lane] : 0);
   }
   while (t < ntiles) {
     unsigned char* row = slab + (size_t)tl.vertex * g.row;
 
     for (uint32_t u0 = 0; u0 < tl.count; u0 += kWave) {
       const uint32_t m = tl.count - u0 < kWave ? tl.count - u0 : kWave;
-      if (u0 != 0) hash_chunk(tl, u0, lane < m ? load_raw(tl, u0 + lane) : 0);
+      if (u0 != 0) hash_chunk(tl, u0, lane < m ? dsts[tl.begin + u0 + lane] : 0);
       const uint32_t np = m * C;
       const uint32_t iters = (np + kWave - 1) / kWave;  // uniform over the wave
       uint32_t q = i0, c = c0;
@@ -478,10 +472,10 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
     // them overlap is slower).
     __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
     Tile tl_next{0, 0, 0, 0};
-    uint64_t raw0_next = 0;
+    uint32_t dst_next = 0;
     if (tn < ntiles) {
       tl_next = tiles[tn];
-      if (lane < tl_next.count) raw0_next = load_raw(tl_next, lane);
+      if (lane < tl_next.count) dst_next = dsts[tl_next.begin + lane];
     }
 
     // write-back: read-xor-write of the touched records, four LDS entries per lane in flight
@@ -517,9 +511,8 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
       // stores.  The record loads leave ga/gg unset for entries they skip, so no zero fill of
       // those registers waits on earlier memory operations either.
       if (first) {
-        uint32_t lo = (uint32_t)raw0_next, hi = (uint32_t)(raw0_next >> 32);
-        asm volatile("" : "+v"(lo), "+v"(hi)::"memory");
-        if (tn < ntiles) hash_chunk(tl_next, 0, ((uint64_t)hi << 32) | lo);
+        asm volatile("" : "+v"(dst_next)::"memory");
+        if (tn < ntiles) hash_chunk(tl_next, 0, dst_next);
       }
       if (tl.split) {
 #pragma unroll
@@ -539,6 +532,81 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
     __syncthreads();
     t = tn;
     tl = tl_next;
+  }
+}
+
+// Sketch::update over a batch of indices of one sketch (row 0 of slab).  All waves of a workgroup XOR
+// into one LDS delta of `depth` records per column (odd, so columns start in different banks) and the
+// workgroups add theirs to the row with device-scope atomics, so a record takes one atomic per
+// workgroup where the tiles of 1024 indices, each with its own delta, took one per tile on 2700
+// words and one per deep pair.  A lane keeps its index and takes the columns one after the other from
+// a column of its own on, which spreads a step's 64 lanes over the columns.  VALU-bound like the long
+// tiles of k_update_tiles: 4.19M indices of 25 columns 446 -> 126 us.
+constexpr uint32_t kOneBlock = 1024, kOneGrid = 512;
+constexpr uint32_t kOneDepth = 17, kOneMaxCols = 160;  // deltas of kOneDepth records up to this many columns
+template <class G>
+__global__ void __launch_bounds__(kOneBlock, 8)
+k_sketch_update(const uint64_t* __restrict__ idxs, size_t count, unsigned char* __restrict__ slab, Geo g,
+                const uint64_t* __restrict__ col_bf, uint32_t depth) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const uint32_t C = g.C, D = g.D, lds_n = C * depth + 1, lds_d = D < depth ? D : depth;
+  uint64_t* s_bf = reinterpret_cast<uint64_t*>(smem);  // spread bitflips
+  uint64_t* s_a = s_bf + C;
+  G* s_g = reinterpret_cast<G*>(s_a + lds_n);
+  for (uint32_t i = threadIdx.x; i < C; i += blockDim.x) s_bf[i] = xxh3_spread(col_bf[i]);
+  for (uint32_t i = threadIdx.x; i < lds_n; i += blockDim.x) {
+    s_a[i] = 0;
+    s_g[i] = 0;
+  }
+  __syncthreads();
+  const uint64_t chk_sbf = xxh3_spread(g.chk_bf), depth_cap = 1ull << D;
+  const uint32_t near_cap = 1u << depth;
+  uint64_t det_a = 0;
+  G det_g = 0;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
+    const uint64_t idx = idxs[i];
+    const uint64_t sp = xxh3_spread(xxh3_prep(idx));
+    uint64_t ck = xxh3_products(sp ^ chk_sbf);
+    ck ^= ck >> 28;
+    const G chk = (G)ck;
+    det_a ^= idx;
+    det_g ^= chk;
+    uint32_t c = lane_id() % C, at = c * depth;
+    for (uint32_t k = 0; k < C; ++k) {
+      const uint64_t h = xxh3_products(sp ^ s_bf[c]);
+      const uint32_t low = (uint32_t)h ^ __builtin_amdgcn_alignbit((uint32_t)(h >> 32), (uint32_t)h, 28);
+      const uint32_t near = (uint32_t)__builtin_ctz(low | near_cap);
+      if (near < lds_d) {
+        lds_xor(s_a + at + near, idx);
+        lds_xor(s_g + at + near, chk);
+      } else {
+        const uint32_t d = (uint32_t)__builtin_ctzll((h ^ (h >> 28)) | depth_cap);  // == D: no bucket
+        if (d < D) {
+          xor_rec_atomic<G>(slab + rec_col_off<G>(g, c, d), idx, chk);
+          if (kDeepFlags<G> && rec_is_deep(g, d)) st_rlx(reinterpret_cast<uint32_t*>(slab + deep_flag_off(c)), 1u);
+        }
+      }
+      ++c;
+      at += depth;
+      if (c == C) c = at = 0;
+    }
+  }
+  // lanes past the end hold zeros, and every lane is active again
+  const uint64_t da = wave_xor_dpp_u64(det_a);
+  const G dg = sizeof(G) == 4 ? (G)wave_xor_dpp_u32((uint32_t)det_g) : (G)wave_xor_dpp_u64((uint64_t)det_g);
+  if (lane_id() == 0) {
+    lds_xor(s_a + lds_n - 1, da);
+    lds_xor(s_g + lds_n - 1, dg);
+  }
+  __syncthreads();
+  for (uint32_t e = threadIdx.x; e < lds_n; e += blockDim.x) {
+    const uint64_t a = s_a[e];
+    const G gm = s_g[e];
+    if ((a | (uint64_t)gm) == 0) continue;  // also the entries at depth >= D
+    const uint32_t c = e / depth, d = e - c * depth;
+    const bool det = e == lds_n - 1;
+    xor_rec_atomic<G>(slab + (det ? det_col_off(g) : rec_col_off<G>(g, c, d)), a, gm);
+    if (kDeepFlags<G> && !det && rec_is_deep(g, d)) st_rlx(reinterpret_cast<uint32_t*>(slab + deep_flag_off(c)), 1u);
   }
 }
 
@@ -2426,8 +2494,8 @@ size_t update_tiles_lds_bytes(const Geo& g, int gbytes) {
 }
 
 void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_dev, uint32_t ntiles_host,
-                         uint32_t grid_cap, const uint32_t* dsts, const uint64_t* raw_idx, unsigned char* slab,
-                         const Geo& g, const uint64_t* col_bf, hipStream_t s) {
+                         uint32_t grid_cap, const uint32_t* dsts, unsigned char* slab, const Geo& g,
+                         const uint64_t* col_bf, hipStream_t s) {
   // tile count known on the host: one workgroup per tile (capped, then grid-stride);
   // known only on the device: a persistent grid of grid_cap workgroups
   uint32_t grid = ntiles_dev ? grid_cap : (grid_cap && ntiles_host > grid_cap ? grid_cap : ntiles_host);
@@ -2435,16 +2503,23 @@ void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_d
   const size_t lds = update_tiles_lds_bytes(g, gbytes);
   const bool wide = g.C * kLdsPitch + 1 > 4 * kWave;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kWave), lds, s, tiles, ntiles_dev, ntiles_host, dsts, raw_idx, slab, g,
-                       col_bf);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kWave), lds, s, tiles, ntiles_dev, ntiles_host, dsts, slab, g, col_bf);
   };
-  if (gbytes == 4) {
-    if (raw_idx) wide ? go(k_update_tiles<uint32_t, true, true>) : go(k_update_tiles<uint32_t, true, false>);
-    else wide ? go(k_update_tiles<uint32_t, false, true>) : go(k_update_tiles<uint32_t, false, false>);
-  } else {
-    if (raw_idx) wide ? go(k_update_tiles<uint64_t, true, true>) : go(k_update_tiles<uint64_t, true, false>);
-    else wide ? go(k_update_tiles<uint64_t, false, true>) : go(k_update_tiles<uint64_t, false, false>);
-  }
+  if (gbytes == 4) wide ? go(k_update_tiles<uint32_t, true>) : go(k_update_tiles<uint32_t, false>);
+  else wide ? go(k_update_tiles<uint64_t, true>) : go(k_update_tiles<uint64_t, false>);
+}
+
+void launch_sketch_update(int gbytes, const uint64_t* idx, size_t count, unsigned char* slab, const Geo& g,
+                          const uint64_t* col_bf, hipStream_t s) {
+  if (!count) return;
+  const uint32_t depth = g.C <= kOneMaxCols ? kOneDepth : kLdsDepth;
+  const uint32_t block = (uint32_t)std::min<size_t>(kOneBlock, (count + kWave - 1) / kWave * kWave);
+  const uint32_t grid = (uint32_t)std::min<size_t>(kOneGrid, (count + block - 1) / block);
+  const size_t lds = g.C * size_t(8) + ((size_t)g.C * depth + 1) * (8 + gbytes);
+  if (gbytes == 4)
+    hipLaunchKernelGGL(k_sketch_update<uint32_t>, dim3(grid), dim3(block), lds, s, idx, count, slab, g, col_bf, depth);
+  else
+    hipLaunchKernelGGL(k_sketch_update<uint64_t>, dim3(grid), dim3(block), lds, s, idx, count, slab, g, col_bf, depth);
 }
 
 size_t group_partials_len(uint32_t n) { return (n + kScanSpan - 1) / kScanSpan + 1; }

@@ -46,11 +46,13 @@ constexpr uint32_t kDefaultTile = 256;
 // Tile kernel (one wave per tile).  `ntiles_dev` (device scalar) bounds the tile index when
 // non-null (persistent grid of grid_cap workgroups), otherwise `ntiles_host` (one workgroup per
 // tile, at most grid_cap when grid_cap > 0).  Workgroups walk tiles grid-stride.
-// Exactly one of `dsts` (destination vertex ids; index = concat(vertex, dst)) or `raw_idx`
-// (64-bit indices) is non-null.
+// dsts: destination vertex ids (index = concat(vertex, dst)).
 void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_dev, uint32_t ntiles_host,
-                         uint32_t grid_cap, const uint32_t* dsts, const uint64_t* raw_idx, unsigned char* slab,
-                         const Geo& g, const uint64_t* col_bf, hipStream_t s);
+                         uint32_t grid_cap, const uint32_t* dsts, unsigned char* slab, const Geo& g,
+                         const uint64_t* col_bf, hipStream_t s);
+// Sketch::update over `count` 64-bit indices (device memory) of the one sketch in slab.
+void launch_sketch_update(int gbytes, const uint64_t* idx, size_t count, unsigned char* slab, const Geo& g,
+                          const uint64_t* col_bf, hipStream_t s);
 size_t update_tiles_lds_bytes(const Geo& g, int gbytes);
 
 // ---- grouping of a device-resident stream of (src,dst) pairs into per-vertex tiles ----

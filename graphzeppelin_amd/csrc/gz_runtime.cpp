@@ -93,16 +93,9 @@ void GzSketch::zero() {  // src/sketch.cpp:86-92
 }
 void GzSketch::update_batch(const uint64_t* idx, size_t count) {  // src/sketch.cpp:69-83
   if (!count) return;
-  constexpr size_t kTile = 1024;
   raw.ensure(count);
-  const size_t nt = (count + kTile - 1) / kTile;
-  std::vector<Tile> ht(nt);
-  for (size_t t = 0; t < nt; ++t)
-    ht[t] = Tile{0, (uint32_t)(t * kTile), (uint32_t)std::min(kTile, count - t * kTile), nt > 1 ? 1u : 0u};
-  tiles.ensure(nt);
   GZ_HIP(hipMemcpyAsync(raw.p, idx, count * 8, hipMemcpyHostToDevice, st));
-  GZ_HIP(hipMemcpyAsync(tiles.p, ht.data(), nt * sizeof(Tile), hipMemcpyHostToDevice, st));
-  launch_update_tiles(gb, tiles.p, nullptr, (uint32_t)nt, 0, nullptr, raw.p, slab.p, geo, col_bf.p, st);
+  launch_sketch_update(gb, raw.p, count, slab.p, geo, col_bf.p, st);
   GZ_HIP(hipGetLastError());
   GZ_HIP(hipStreamSynchronize(st));
 }
@@ -433,7 +426,7 @@ void GzAlg::submit_stage_locked() {
   GZ_HIP(hipMemcpyAsync(s.dev.p + doff, s.host.p + doff, s.used * 4, hipMemcpyHostToDevice, st));
   if (prof) prof_begin(0, batch_alg_bytes(s.ent_cnt), false, s.used);
   launch_update_tiles(gb, reinterpret_cast<Tile*>(s.dev.p), nullptr, (uint32_t)nt, 0,
-                      reinterpret_cast<uint32_t*>(s.dev.p + doff), nullptr, slab.p, geo, col_bf.p, st);
+                      reinterpret_cast<uint32_t*>(s.dev.p + doff), slab.p, geo, col_bf.p, st);
   if (prof) prof_end();
   GZ_HIP(hipGetLastError());
   if (!s.ev) GZ_HIP(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming));
@@ -475,7 +468,7 @@ void GzAlg::plain_launch(uint32_t src, const uint32_t* dsts, size_t k) {
   GZ_HIP(hipMemcpyAsync(s.dev.p, s.host.p, need, hipMemcpyHostToDevice, st));
   if (prof) prof_begin(0, batch_alg_bytes(std::vector<uint32_t>{(uint32_t)k}), false, k);
   launch_update_tiles(gb, reinterpret_cast<Tile*>(s.dev.p), nullptr, (uint32_t)nt, 0,
-                      reinterpret_cast<uint32_t*>(s.dev.p + tbytes), nullptr, slab.p, geo, col_bf.p, st);
+                      reinterpret_cast<uint32_t*>(s.dev.p + tbytes), slab.p, geo, col_bf.p, st);
   if (prof) prof_end();
   GZ_HIP(hipGetLastError());
   if (!s.ev) GZ_HIP(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming));
@@ -550,7 +543,7 @@ void GzAlg::flush_pending() {
     pend_wait = true;
   }
   if (prof) prof_begin(0, 0, true, 2 * cnt);
-  launch_update_tiles(gb, g_tiles.p, g_totals.p + 1, 0, grid_cap, dst_arr.p, nullptr, slab.p,
+  launch_update_tiles(gb, g_tiles.p, g_totals.p + 1, 0, grid_cap, dst_arr.p, slab.p,
                       geo, col_bf.p, st);
   if (prof) prof_end();
   GZ_HIP(hipGetLastError());

@@ -126,8 +126,7 @@ class GzSketch {
   hipStream_t st = nullptr;
   DevBuf<uint8_t> slab;  // packed bucket records (see Geo::row)
   DevBuf<uint64_t> col_bf, raw;
-  DevBuf<uint32_t> dsts, out;
-  DevBuf<Tile> tiles;
+  DevBuf<uint32_t> out;
   DevBuf<uint8_t> packed;
 
   GzSketch(uint64_t vector_len, uint64_t seed, size_t samples, size_t cols, int gamma_bytes);

@@ -61,9 +61,8 @@ int gz_sketch_update_batch(gz_sketch* s, const uint64_t* idx, size_t count);
 /* No counterpart in the reference.  For callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): Sketch::update over `count`
  * indices already in device memory, with the kernel and the result of gz_sketch_update_batch, and
- * no allocation or staging.  The kernel's tile descriptors live in a static device array of 1 MiB
- * per GPU, so count is at most 2^26 (GZ_ERR_INVALID_ARG above that).  Every call on a GPU shares
- * that array: calls that overlap on one GPU race.  Returns when the update is done. */
+ * no allocation or staging.  count is at most 2^26 (GZ_ERR_INVALID_ARG above that).  Returns when the
+ * update is done. */
 int gz_sketch_update_batch_device_noalloc(gz_sketch* s, const uint64_t* idx_device, size_t count);
 /* Sketch::sample, src/sketch.cpp:94-116 -> *result is a gz_sample_result */
 int gz_sketch_sample(gz_sketch* s, uint64_t* idx, int* result);
