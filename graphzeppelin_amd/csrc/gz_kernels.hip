@@ -1267,12 +1267,13 @@ constexpr uint32_t kNoRoot = 0xFFFFFFFFu;  // no supernode (unused partial slot,
 //                     The complement sum needs no majority -- any supernode's sum is the XOR of the
 //                     vertices outside it -- so a large one can be left out a round early.
 //   kStSeg + 2(r & 1) + 1  supernodes outside the giant in round r (entries of RoundBufs::segs[r & 1])
+//   kStDropped        vertices of the supernodes taken out of the lists in this query (see k_bv_alloc)
 // The two counts of one round parity share a 64-bit word, so a block takes its share of both with
 // one atomic: entries at kStSeg + 2 * (r & 1), supernodes at kStSeg + 2 * (r & 1) + 1.
 constexpr uint32_t kStGiantRound = 2, kStGiantFirst = 3, kStActMode = 4, kStBest = 6, kStSeg = 8;
-constexpr uint32_t kStWords = 12;
+constexpr uint32_t kStDropped = 12, kStWords = 13;
 constexpr uint32_t kCandidateDiv = 32;
-constexpr uint32_t kMaxStatRounds = 64;
+constexpr uint32_t kMaxStatRounds = 64;  // per round: vertices regrouped and the giant's root, then vertices dropped
 
 // cnt / st (a query's start, or nullptr): the root counts are cleared too, and the round state
 // words are set to their start values (no giant), so a query begins with one launch.
@@ -1435,14 +1436,21 @@ k_bv_find_count(uint32_t* __restrict__ parent, uint32_t n, uint2* __restrict__ n
 // Segments for the roots met in this round's walk (every non-giant root is a member of its own
 // supernode, so it is walked).  cnt is cleared here, its last reader.  Without a giant yet, a root
 // holding more than half of the vertices is elected: at most one can.
+// drop_ok: every update reached both of its ends' sketches, so a supernode without cut edges, which
+// samples ZERO, stays one: no other supernode has an edge into it, and its sums are zero.  A root that
+// was one vertex (rounds >= 2: one supernode) in the last round and sampled ZERO gets no segment
+// (off = kDropped), so finished components are not walked again.  The giant's election comes first.
+// A query on 2^20 R-MAT vertices, a third of them isolated: the rounds' launches 1560 -> 700 us.
 // A root's segment goes into the round's segment list too (block scan of the counts and of the
 // roots, packed in one 64-bit scan: counts in the low 40 bits, roots above).
 constexpr uint32_t kSegShift = 40;
+constexpr uint32_t kDropped = 0xFFFFFFFFu;
 
 __global__ void __launch_bounds__(kAggBlock)
 k_bv_alloc(uint32_t* __restrict__ cnt, uint32_t n, uint32_t* __restrict__ off, uint32_t* __restrict__ cursor,
            uint32_t* __restrict__ st, uint32_t round, const uint32_t* __restrict__ act_list, uint32_t giant_ok,
-           const uint32_t* __restrict__ prev_mod, RoundSeg* __restrict__ segs) {
+           const uint32_t* __restrict__ prev_mod, RoundSeg* __restrict__ segs, const uint64_t* __restrict__ samp,
+           uint32_t drop_ok) {
   const uint32_t live = ld_acq(prev_mod);  // checked after the first reads (see k_bv_find_count)
   __shared__ uint64_t wsum[kAggBlock / kWave];
   __shared__ uint32_t s_base, s_sbase;
@@ -1453,6 +1461,7 @@ k_bv_alloc(uint32_t* __restrict__ cnt, uint32_t n, uint32_t* __restrict__ off, u
   const bool in_walk = i < walk;
   const uint32_t v = in_walk ? walk_vertex(act_list, round, i) : 0;
   uint32_t c = in_walk ? cnt[v] : 0;
+  const uint64_t sv = in_walk && drop_ok ? samp[v] : kSampFail;
   if (!live || blockIdx.x * kAggBlock >= walk) return;  // whole blocks past the walk
   if (c) cnt[v] = 0;
   if (!act && giant_ok && 2ull * c > n) {
@@ -1461,6 +1470,15 @@ k_bv_alloc(uint32_t* __restrict__ cnt, uint32_t n, uint32_t* __restrict__ off, u
     c = 0;
   } else if (!act && giant_ok && c >= 2 && c >= n / kCandidateDiv) {  // at most kCandidateDiv roots
     atomicMax(reinterpret_cast<unsigned long long*>(st + kStBest), ((unsigned long long)c << 32) | v);
+  }
+  const bool drop = c == 1 && sv == kSampZero;
+  if (drop) {
+    c = 0;
+    off[v] = kDropped;
+  }
+  if (drop_ok) {  // uniform
+    const uint32_t d = (uint32_t)__syncthreads_count(drop);
+    if (threadIdx.x == 0 && d) atomicAdd(st + kStDropped, d);
   }
   const uint64_t x = c ? ((uint64_t)1 << kSegShift) | c : 0;
   const uint64_t incl = wave_incl_scan_u64(x);
@@ -1505,8 +1523,8 @@ k_bv_scatter(const uint2* __restrict__ nd, uint32_t n, const uint32_t* __restric
   const uint2 t = in_walk && v < n ? nd[v] : make_uint2(0u, 0u);
   if (!live || !in_walk || v >= n) return;
   if (t.x == gr || t.x >= n) return;  // the giant supernode's members are not regrouped
-  const uint32_t p = off[t.x] + t.y;
-  if (p >= e || p >= n) return;
+  const uint32_t o = off[t.x], p = o + t.y;
+  if (o == kDropped || p >= e || p >= n) return;
   members[p] = v;  // the root beside the member, so the reduce reads both in list order
   mroot[p] = t.x;
 }
@@ -1580,20 +1598,26 @@ k_seg_find(uint32_t* __restrict__ parent, uint32_t n, uint32_t* __restrict__ cnt
 __global__ void __launch_bounds__(kAggBlock)
 k_seg_alloc(uint32_t* __restrict__ cnt, uint32_t n, const uint2* __restrict__ nd, uint32_t* __restrict__ off,
             uint32_t* __restrict__ cursor, RoundSeg* __restrict__ segs_new, uint32_t* __restrict__ st, uint32_t round,
-            const RoundSeg* __restrict__ segs_old, uint32_t giant_ok, const uint32_t* __restrict__ prev_mod) {
+            const RoundSeg* __restrict__ segs_old, uint32_t giant_ok, const uint32_t* __restrict__ prev_mod,
+            const uint64_t* __restrict__ samp, uint32_t drop_ok) {
   const uint32_t live = ld_acq(prev_mod);
   __shared__ uint64_t wsum[kAggBlock / kWave];
-  __shared__ uint32_t s_base, s_sbase;
+  __shared__ uint32_t s_base, s_sbase, s_drop;
   const bool act = st[kStActMode] != 0;
   const uint32_t nseg = st[kStSeg + 2 * ((round - 1) & 1) + 1];
   const uint32_t lane = lane_id(), wid = threadIdx.x / kWave;
   const uint32_t i = blockIdx.x * kAggBlock + threadIdx.x;
   const bool in = i < nseg;
-  const uint32_t v = in ? segs_old[i].root : 0;
+  const uint32_t v = in ? segs_old[i].root : 0, old_len = in ? segs_old[i].len : 0;
   const bool ok = in && v < n;
   const bool is_root = ok && nd[v].x == v;
   uint32_t c = is_root ? cnt[v] : 0;  // zero for the giant's root: its members are not counted
+  const uint64_t sv = ok && drop_ok ? samp[v] : kSampFail;
   if (!live || blockIdx.x * kAggBlock >= nseg) return;  // whole blocks past the segments
+  if (drop_ok) {  // uniform
+    if (threadIdx.x == 0) s_drop = 0;
+    __syncthreads();
+  }
   if (c) cnt[v] = 0;
   if (!act && giant_ok && 2ull * c > n) {
     st[kStGiantFirst] = v;
@@ -1601,6 +1625,10 @@ k_seg_alloc(uint32_t* __restrict__ cnt, uint32_t n, const uint2* __restrict__ nd
     c = 0;
   } else if (!act && giant_ok && c >= 2 && c >= n / kCandidateDiv) {
     atomicMax(reinterpret_cast<unsigned long long*>(st + kStBest), ((unsigned long long)c << 32) | v);
+  } else if (c != 0 && c == old_len && sv == kSampZero) {
+    atomicAdd(&s_drop, c);
+    c = 0;
+    off[v] = kDropped;
   }
   const uint64_t x = c ? ((uint64_t)1 << kSegShift) | c : 0;
   const uint64_t incl = wave_incl_scan_u64(x);
@@ -1613,6 +1641,7 @@ k_seg_alloc(uint32_t* __restrict__ cnt, uint32_t n, const uint2* __restrict__ nd
   }
   constexpr uint64_t kCntMask = ((uint64_t)1 << kSegShift) - 1;
   if (threadIdx.x == 0) {
+    if (drop_ok && s_drop) atomicAdd(st + kStDropped, s_drop);
     // entries and supernodes of the block in one 64-bit atomic (neither sum can reach 2^32)
     const uint64_t add = ((tot >> kSegShift) << 32) | (tot & kCntMask);
     const uint64_t old =
@@ -1652,8 +1681,8 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
   if (!live || !in || R >= n || v >= n) return;
   const uint2 t = nd[R];
   if (t.x == gr || t.x >= n) return;
-  const uint32_t p = off[t.x] + i + t.y;
-  if (p >= e_new || p >= n) return;
+  const uint32_t o = off[t.x], p = o + i + t.y;
+  if (o == kDropped || p >= e_new || p >= n) return;
   members_new[p] = v;
   mroot_new[p] = t.x;
   parent[v] = t.x;
@@ -2009,6 +2038,7 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
   if (rstats && blockIdx.x == 0 && threadIdx.x == 0 && round < kMaxStatRounds) {
     rstats[2 * round] = e1;  // diagnostics: vertices regrouped and the giant's root in this round
     rstats[2 * round + 1] = giant;
+    rstats[2 * kMaxStatRounds + round] = st[kStDropped];
   }
   if (giant != kNoRoot && e1 == 0) {  // every vertex is in the giant: its sum is zero
     if (blockIdx.x == 0 && threadIdx.x == 0) samp[giant] = kSampZero;
@@ -2110,13 +2140,14 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
 }
 
 // ---- the last rounds in one workgroup ----------------------------------------------------------
-// Once a giant supernode exists, a round walks only the vertices outside it, and after a few rounds
-// they are few.  k_bv_finish then runs every remaining round inside one workgroup -- the same
+// Once a giant supernode exists, a round walks only the vertices outside it that are not in a finished
+// component, and after a few rounds they are few; a small graph's are few from the start.  k_bv_finish then runs every remaining round inside one workgroup -- the same
 // regrouping, reduce, sample and merge as k_bv_find_count .. k_apply_samples, with barriers between
 // the steps instead of kernel boundaries -- so a round costs a few round trips instead of five
-// dependent launches.  It takes over at round r0 only when round r0 - 1 changed something, a giant
-// exists (or was recorded as the next round's candidate) and the walk holds at most kFinishMax
-// vertices; otherwise it returns without touching any state and the rounds continue as launches.
+// dependent launches.  It takes over at round r0 only when round r0 - 1 changed something and the walk
+// holds at most kFinishMax vertices; otherwise it returns without touching any state and the rounds
+// continue as launches.  A giant is elected in it as in the launched rounds, so both regroup the same
+// vertices.
 // It then sets mod[r] for every modified round, as the launched rounds do, and records the last
 // round it ran in mod[nmod - 1] (a word no round uses), so one copy of mod tells the host both.
 //
@@ -2162,7 +2193,8 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
   __shared__ uint32_t s_slotroot[kRedWaves * 2];
   __shared__ uint64_t s_tot[2 * kWave];
   __shared__ uint32_t s_wsum[kRedWaves];
-  __shared__ uint32_t s_take, s_gfirst, s_walk, s_gcur, s_e;
+  __shared__ uint32_t s_take, s_gfirst, s_walk, s_gcur, s_e, s_elect;
+  __shared__ unsigned long long s_best;
   const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
   if (tid == 0) {
     const uint32_t live = ld_acq(d.mod + (r0 - 1));
@@ -2170,8 +2202,9 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     const uint64_t best = *reinterpret_cast<const uint64_t*>(st + kStBest);
     if (gfirst == kNoRoot && best) gfirst = (uint32_t)best;  // as k_bv_find_count takes the candidate
     const uint32_t walk = st[kStSeg + 2 * ((r0 - 1) & 1)];
-    s_take = (live && gfirst != kNoRoot && walk <= kFinishMax) ? 1u : 0u;
+    s_take = (live && walk <= kFinishMax) ? 1u : 0u;
     s_gfirst = gfirst;
+    s_best = 0;
     s_walk = walk;
   }
   // The last kernel of every group of rounds: on exit it copies the round flags and the per-round
@@ -2180,7 +2213,7 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
   auto report = [&]() {
     __syncthreads();
     for (uint32_t t = tid; t < d.nmod; t += kRedBlock) rep[t] = ld_acq(d.mod + t);
-    for (uint32_t t = tid; t < 2 * kMaxStatRounds; t += kRedBlock) rep[d.nmod + t] = ld_acq(rstats + t);
+    for (uint32_t t = tid; t < 3 * kMaxStatRounds; t += kRedBlock) rep[d.nmod + t] = ld_acq(rstats + t);
     __threadfence_system();
   };
   __syncthreads();
@@ -2201,9 +2234,13 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
       s_cnt[k] = 0;
     }
     if (tid < 2 * kWave) s_tot[tid] = 0;
-    if (tid == 0) s_gcur = dsu_find_coherent(d.parent, s_gfirst);  // the giant only grows
+    if (tid == 0) {
+      if (s_gfirst == kNoRoot && s_best) s_gfirst = (uint32_t)s_best;
+      s_gcur = s_gfirst == kNoRoot ? kNoRoot : dsu_find_coherent(d.parent, s_gfirst);  // the giant only grows
+      s_elect = kNoRoot;
+    }
     __syncthreads();
-    const uint32_t gcur = s_gcur;
+    uint32_t gcur = s_gcur;
     // roots of the walked vertices, full path compression, members per root (k_bv_find_count)
     uint32_t rr[kFinishPer], slot[kFinishPer], pos[kFinishPer];
 #pragma unroll
@@ -2219,13 +2256,22 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
       }
     }
     __syncthreads();
+    if (gcur == kNoRoot) {  // the giant's election and candidates, as in k_bv_alloc
+      for (uint32_t k = tid; k < kFinishTable; k += kRedBlock) {
+        const uint32_t c = s_cnt[k];
+        if (2ull * c > d.n) s_elect = s_gfirst = s_key[k];  // at most one
+        else if (c >= 2 && c >= d.n / kCandidateDiv) atomicMax(&s_best, ((unsigned long long)c << 32) | s_key[k]);
+      }
+      __syncthreads();
+      gcur = s_elect;
+    }
     // segment starts: exclusive scan of the counts over the table (4 slots per thread)
     {
       constexpr uint32_t per = kFinishTable / kRedBlock;
       uint32_t c[per], sum = 0;
 #pragma unroll
       for (uint32_t k = 0; k < per; ++k) {
-        c[k] = s_cnt[tid * per + k];
+        c[k] = s_key[tid * per + k] == gcur ? 0u : s_cnt[tid * per + k];
         sum += c[k];
       }
       const uint32_t incl = (uint32_t)wave_incl_scan_u64(sum);
@@ -2257,6 +2303,7 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     if (tid == 0 && rstats && r < kMaxStatRounds) {
       rstats[2 * r] = e;
       rstats[2 * r + 1] = gcur;
+      rstats[2 * kMaxStatRounds + r] = st[kStDropped];
     }
     __syncthreads();
     // reduce + sample (k_bv_reduce): one wave per chunk of cw <= 64 entries, the entries spread
@@ -2271,7 +2318,7 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
       const uint32_t p0 = c * cw;
       const uint32_t len = e - p0 < cw ? e - p0 : cw;
       reduce_members<G>(p0, len, cw / 4, e, s_mem, s_mroot, slab, g, r, hs, ts, samp, d.flags, det_cpy, deep_skip != 0,
-                        s_tot, nullptr, 0, 0, nullptr);
+                        gcur != kNoRoot ? s_tot : nullptr, nullptr, 0, 0, nullptr);
       const uint32_t hr = *hs.root, tr = *ts.root;
       if (hr != kNoRoot) {  // started in an earlier chunk
         uint64_t* acc = s_acc + (size_t)(s_seg[p0] / cw) * 2 * kWave;
@@ -2297,7 +2344,7 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
       acc[kWave + lane] = 0;
       if (lane == 0) s_accroot[c] = kNoRoot;
     }
-    if (wid == kRedWaves - 1) {  // the giant, from the complement
+    if (wid == kRedWaves - 1 && gcur != kNoRoot) {  // the giant, from the complement
       uint64_t idx;
       const int code = wave_sample<G>(s_tot[lane], (G)s_tot[kWave + lane], g.D, g.chk_bf, &idx);
       if (lane == 0) samp[gcur] = e == 0 ? kSampZero : sample_record(code, idx, g.n, d.flags);
@@ -2310,7 +2357,7 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     bool modified = false;
     for (uint32_t k = tid; k < kFinishTable; k += kRedBlock)
       if (s_key[k] != kEmptyKey && apply_sample(d, ld_acq(samp + s_key[k]), hint)) modified = true;
-    if (tid == 0 && apply_sample(d, ld_acq(samp + gcur), hint)) modified = true;
+    if (tid == 0 && gcur != kNoRoot && apply_sample(d, ld_acq(samp + gcur), hint)) modified = true;
     const bool any = __syncthreads_or(modified);
     if (tid == 0 && any) st_rlx(d.mod + r, 1u);
     if (!any || r >= last_round) {
@@ -2689,7 +2736,7 @@ uint32_t reduce_blocks(uint32_t n) { return 2 * std::max(1u, (n + kRedBlock - 1)
 constexpr uint32_t kSmallWalkDiv = 2;  // rounds regrouping at most n / kSmallWalkDiv entries use 32 per wave
 
 void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const Geo& g,
-                  const DsuDev& d, const RoundBufs& rb, bool giant_ok, hipStream_t s, bool deep_skip) {
+                  const DsuDev& d, const RoundBufs& rb, bool giant_ok, bool drop_ok, hipStream_t s, bool deep_skip) {
   const uint32_t n = g.n;
   const uint32_t* prev = d.mod + (round - 1);
   uint32_t* cur = d.mod + round;
@@ -2702,14 +2749,14 @@ void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const G
     hipLaunchKernelGGL(k_bv_find_count, dim3(grid), dim3(kAggBlock), 0, s, d.parent, n, rb.nd, rb.cnt, st, round,
                        act_list, prev);
     hipLaunchKernelGGL(k_bv_alloc, dim3(grid), dim3(kAggBlock), 0, s, rb.cnt, n, rb.off, rb.cursor, st, round,
-                       act_list, giant_ok ? 1u : 0u, prev, rb.segs[par]);
+                       act_list, giant_ok ? 1u : 0u, prev, rb.segs[par], rb.samp, drop_ok ? 1u : 0u);
     hipLaunchKernelGGL(k_bv_scatter, dim3(grid), dim3(kAggBlock), 0, s, rb.nd, n, rb.off, members, rb.mroot[par],
                        st, round, act_list, prev);
   } else {  // whole runs of the previous round's member list
     hipLaunchKernelGGL(k_seg_find, dim3(grid), dim3(kAggBlock), 0, s, d.parent, n, rb.cnt, rb.nd, st, round,
                        rb.segs[opar], prev);
     hipLaunchKernelGGL(k_seg_alloc, dim3(grid), dim3(kAggBlock), 0, s, rb.cnt, n, rb.nd, rb.off, rb.cursor,
-                       rb.segs[par], st, round, rb.segs[opar], giant_ok ? 1u : 0u, prev);
+                       rb.segs[par], st, round, rb.segs[opar], giant_ok ? 1u : 0u, prev, rb.samp, drop_ok ? 1u : 0u);
     hipLaunchKernelGGL(k_seg_copy, dim3(grid_for(n, 256)), dim3(256), 0, s, n, rb.nd, rb.off, d.parent, rb.members[opar],
                        rb.mroot[opar], members, rb.mroot[par], st, round, prev);
   }

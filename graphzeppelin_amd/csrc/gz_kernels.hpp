@@ -108,6 +108,7 @@ void launch_dsu_reset(const DsuDev& d, hipStream_t s, const RoundBufs* rb = null
 struct RoundSeg {
   uint32_t root, start, len, pad;
 };
+constexpr uint32_t kRoundStats = 192;
 struct RoundBufs {
   uint32_t* cnt;         // n      members per root (zero between rounds)
   uint32_t* off;         // n      segment start per root
@@ -123,7 +124,8 @@ struct RoundBufs {
   uint32_t* xcnt;        // xslots arrival counters, zero between rounds
   uint32_t xslots;       // >= reduce_blocks(n) + 1 (one per reduce workgroup, one for the giant)
   uint64_t* samp;        // n      sample record per supernode root
-  uint32_t* rstats;      // 2 * 64 per round: vertices regrouped, giant root (diagnostics)
+  uint32_t* rstats;      // kRoundStats: per round, vertices regrouped and giant root (2 * 64), then vertices
+                         // of finished components dropped from the lists so far (64)
   unsigned char* det_cpy;  // n records: every vertex's deterministic bucket, copied in round 0
   unsigned char* hint;     // n      round 0: each vertex's degree class, the first key of its merge order
 };
@@ -135,21 +137,24 @@ void launch_sample_round0(int gbytes, const unsigned char* slab, const Geo& g, c
                           hipStream_t s);
 // Workgroups of a round's reduce over n vertices (enough for 512 member entries each).
 uint32_t reduce_blocks(uint32_t n);
-// Rounds r0, r0 + 1, ... up to last_round in one workgroup, when round r0 - 1 changed something, a
-// giant supernode exists and round r0 walks at most finish_max() vertices; otherwise a no-op.
+// Rounds r0, r0 + 1, ... up to last_round in one workgroup, when round r0 - 1 changed something and
+// round r0 walks at most finish_max() vertices; otherwise a no-op.  Only for sketches known to XOR to
+// zero (it may elect a giant).
 // d.mod[d.nmod - 1] gets the last round it ran (it stays 0 when the finish did not take over).
-// rep (mapped host memory, or nullptr): on exit the kernel copies d.mod[0..nmod) and the 128
+// rep (mapped host memory, or nullptr): on exit the kernel copies d.mod[0..nmod) and the kRoundStats
 // per-round diagnostic words there.  Returns whether it launched (2 <= r0 <= last_round).
 bool launch_finish(int gbytes, uint32_t r0, uint32_t last_round, const unsigned char* slab, const Geo& g,
                    const DsuDev& d, const RoundBufs& rb, hipStream_t s, uint32_t* rep = nullptr, bool deep_skip = true);
 uint32_t finish_max();
 // Queue round `round` (>= 1); every kernel of it is a no-op when d.mod[round - 1] == 0.
 // giant_ok: the vertex sketches are known to XOR to zero, so a supernode holding more than half of
-// the vertices may be summed from its complement.  deep_skip: the reduce reads a member's records
+// the vertices may be summed from its complement.  drop_ok: the sketches were built from updates that
+// reached both ends, so supernodes that sample ZERO are finished and leave the lists.  deep_skip: the reduce reads a member's records
 // past the first overflow line of the round's column only when its deep flag is set (rows of
 // 12-byte records); false reads them all (same result).
 void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const Geo& g,
-                  const DsuDev& d, const RoundBufs& rb, bool giant_ok, hipStream_t s, bool deep_skip = true);
+                  const DsuDev& d, const RoundBufs& rb, bool giant_ok, bool drop_ok, hipStream_t s,
+                  bool deep_skip = true);
 void launch_labels(const DsuDev& d, uint32_t* labels, uint32_t* ncc, hipStream_t s);
 // A query group's answers in place in mapped host memory: q[0..nq) and q[nq..2nq) are the pairs;
 // out gets the kNumFlags error flags, then one byte per pair (1: connected).

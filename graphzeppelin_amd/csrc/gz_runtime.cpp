@@ -235,11 +235,11 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   r_members[0].alloc(n); r_members[1].alloc(n); r_mroot[0].alloc(n); r_mroot[1].alloc(n);
   r_segs[0].alloc(n); r_segs[1].alloc(n); r_nd.alloc(n);
   r_totals.alloc(16);
-  r_stats.alloc(128);
+  r_stats.alloc(kRoundStats);
   r_det.alloc((size_t)n * (8 + gb));
   r_hint.alloc(((size_t)n + 3) & ~size_t(3));
   launch_fill_u32(reinterpret_cast<uint32_t*>(r_hint.p), 0, r_hint.n / 4, st);  // no classes before the first query
-  launch_fill_u32(r_stats.p, 0, 128, st);
+  launch_fill_u32(r_stats.p, 0, kRoundStats, st);
   // cross-workgroup accumulators of the reduce: one slot per workgroup and one for the giant
   const size_t xslots = (size_t)reduce_blocks(n) + 1;
   r_xacc.alloc(xslots * 128);
@@ -296,8 +296,8 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   eager_cap = size_t(1) << 20;
   hflags.alloc(std::max<size_t>(kNumFlags, geo.samples + 2));
   hsmall.alloc(16);
-  hround.alloc(128);
-  rep.ensure(dsu.nmod + 128);
+  hround.alloc(kRoundStats);
+  rep.ensure(dsu.nmod + kRoundStats);
   GZ_HIP(hipEventCreateWithFlags(&hround_ev, hipEventDisableTiming));
   GZ_HIP(hipEventCreateWithFlags(&eager_ev, hipEventDisableTiming));
   GZ_HIP(hipStreamSynchronize(st));
@@ -366,6 +366,7 @@ void GzAlg::apply_update_batch(uint32_t src, const uint32_t* dsts, size_t k) {
   if (k > 0xffffffffull) throw GzError(GZ_ERR_INVALID_ARG, "batch too large");
   std::lock_guard<std::mutex> lk(stage_mtx);
   zero_sum = 0;  // one direction of an edge alone would break the zero sum
+  paired = false;
   if (!cfg.batched) {
     plain_launch(src, dsts, k);
     return;
@@ -487,6 +488,7 @@ void GzAlg::apply_raw(uint32_t src, const void* rawb) {
   launch_merge_packed(gb, slab.p, geo, src, 1, tmp.p, st);
   GZ_HIP(hipStreamSynchronize(st));
   zero_sum = 0;  // a raw delta on one vertex may break the zero sum
+  paired = false;
 }
 
 // ---- kernel timing ----
@@ -746,19 +748,20 @@ bool GzAlg::sketches_sum_to_zero() {
 // DSU reset, round 0, rounds 1..last and (with a giant allowed) the single-workgroup finish from
 // round last + 1, as one stream sequence (captured into a graph or launched directly).  Fills are
 // kernels, so the sequence holds no memset nodes.
-void GzAlg::enqueue_query_prefix(bool giant_ok, uint32_t last) {
+void GzAlg::enqueue_query_prefix(bool giant_ok, bool drop_ok, uint32_t last) {
   launch_dsu_reset(dsu, st, &rb);  // with the root counts and the round state words
   launch_sample_round0(gb, slab.p, geo, dsu, rb, st);
-  for (uint32_t r = 1; r <= last; ++r) launch_round(gb, r, slab.p, geo, dsu, rb, giant_ok, st, use_deep_skip);
+  for (uint32_t r = 1; r <= last; ++r) launch_round(gb, r, slab.p, geo, dsu, rb, giant_ok, drop_ok, st, use_deep_skip);
   if (giant_ok && use_finish) launch_finish(gb, last + 1, geo.samples - 1, slab.p, geo, dsu, rb, st, rep.d, use_deep_skip);
 }
 
-hipGraphExec_t GzAlg::get_query_graph(bool giant_ok, uint32_t last) {
-  const uint32_t key = ((last * 2 + (giant_ok ? 1 : 0)) * 2 + (use_finish ? 1 : 0)) * 2 + (use_deep_skip ? 1 : 0);
+hipGraphExec_t GzAlg::get_query_graph(bool giant_ok, bool drop_ok, uint32_t last) {
+  const uint32_t key = (((last * 2 + (giant_ok ? 1 : 0)) * 2 + (drop_ok ? 1 : 0)) * 2 + (use_finish ? 1 : 0)) * 2 +
+                       (use_deep_skip ? 1 : 0);
   hipGraphExec_t& slot = query_graphs[key];
   if (slot) return slot;
   GZ_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  enqueue_query_prefix(giant_ok, last);
+  enqueue_query_prefix(giant_ok, drop_ok, last);
   hipGraph_t graph = nullptr;
   const hipError_t cap = hipStreamEndCapture(st, &graph);
   if (cap != hipSuccess || !graph) {
@@ -788,27 +791,28 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
   update_locked = true;
   try {
     const bool giant_ok = sketches_sum_to_zero();
+    const bool drop_ok = giant_ok && paired;
+    const bool fin_ok = giant_ok && use_finish;
     const uint32_t last_round = geo.samples - 1;  // round index `samples` would be out of samples
     if (hround_pending) {
-      // The launched rounds of this query: up to the first round of the previous query after which
-      // a giant existed and at most finish_max() vertices remained outside it (diagnostics: vertices
-      // regrouped and the giant's root per round).
+      // The launched rounds of this query: up to the first round of the previous query that regrouped
+      // at most finish_max() vertices.
       if (hround_on_event) GZ_HIP(hipEventSynchronize(hround_ev));
       hround_pending = false;
       next_prefix = (uint32_t)last_rounds + 1;
-      for (uint32_t r = 1; r < (uint32_t)last_rounds && r < 64; ++r)
-        if (hround.p[2 * r + 1] != 0xFFFFFFFFu && hround.p[2 * r] <= finish_max()) {
+      for (uint32_t r = 1; fin_ok && r < (uint32_t)last_rounds && r < 64; ++r)
+        if (hround.p[2 * r] <= finish_max()) {
           next_prefix = r;
           break;
         }
     }
-    const uint32_t want = next_prefix ? next_prefix : kFirstGraphRounds;
+    const uint32_t want = next_prefix ? next_prefix : fin_ok && n <= finish_max() ? 1u : kFirstGraphRounds;
     const uint32_t first = std::max(1u, std::min(want, last_round));
     const bool sf_was_pending = sf_pending;
     sf_pending = false;  // the DSU reset clears the set
     if (prof) prof_begin(1, 0, false, 0);
-    if (use_graphs) GZ_HIP(hipGraphLaunch(get_query_graph(giant_ok, first), st));
-    else enqueue_query_prefix(giant_ok, first);
+    if (use_graphs) GZ_HIP(hipGraphLaunch(get_query_graph(giant_ok, drop_ok, first), st));
+    else enqueue_query_prefix(giant_ok, drop_ok, first);
     GZ_HIP(hipGetLastError());
     uint32_t next = first + 1;
     uint32_t fin_r0 = first + 1;  // first round of the last finish attempt queued
@@ -850,7 +854,7 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
       if (upto >= last_round)
         throw GzError(GZ_ERR_OUT_OF_SAMPLES, "Borůvka needs more rounds than the sketches have samples");
       const uint32_t hi = std::min(next + 1, last_round);
-      for (uint32_t r = next; r <= hi; ++r) launch_round(gb, r, slab.p, geo, dsu, rb, giant_ok, st, use_deep_skip);
+      for (uint32_t r = next; r <= hi; ++r) launch_round(gb, r, slab.p, geo, dsu, rb, giant_ok, drop_ok, st, use_deep_skip);
       reported = giant_ok && use_finish && launch_finish(gb, hi + 1, last_round, slab.p, geo, dsu, rb, st, rep.d, use_deep_skip);
       GZ_HIP(hipGetLastError());
       fin_r0 = hi + 1;
@@ -860,10 +864,10 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
     last_rounds = (size_t)rounds;
     last_finish_start = hf[dsu.nmod - 1] ? fin_r0 : 0;
     if (reported) {
-      std::memcpy(hround.p, rep.p + dsu.nmod, 128 * 4);
+      std::memcpy(hround.p, rep.p + dsu.nmod, kRoundStats * 4);
       hround_on_event = false;
     } else {
-      GZ_HIP(hipMemcpyAsync(hround.p, r_stats.p, 128 * 4, hipMemcpyDeviceToHost, st));
+      GZ_HIP(hipMemcpyAsync(hround.p, r_stats.p, kRoundStats * 4, hipMemcpyDeviceToHost, st));
       GZ_HIP(hipEventRecord(hround_ev, st));
       hround_on_event = true;
     }
@@ -1053,6 +1057,7 @@ void GzAlg::load_packed(uint32_t v0, uint32_t count, const void* in) {
     GZ_HIP(hipStreamSynchronize(st));
   }
   zero_sum = 0;
+  paired = false;
 }
 
 }  // namespace gz
@@ -1390,12 +1395,12 @@ size_t gz_alg_last_query_round_sizes(gz_alg* a, uint32_t* entries, uint32_t* gia
     GZ_REQUIRE(a, "null alg");
     GzAlg& A = *a->a;
     std::lock_guard<std::mutex> lk(A.query_mtx);
-    uint32_t h[128];
+    uint32_t h[gz::kRoundStats];
     GZ_HIP(hipMemcpyAsync(h, A.r_stats.p, sizeof(h), hipMemcpyDeviceToHost, A.st));
     GZ_HIP(hipStreamSynchronize(A.st));
     const size_t rounds = std::min<size_t>(A.last_rounds, 63);
     for (size_t r = 1; r <= rounds && k < cap; ++r, ++k) {
-      if (entries) entries[k] = h[2 * r];
+      if (entries) entries[k] = h[2 * r] + h[128 + r];  // finished components included
       if (giant_root) giant_root[k] = h[2 * r + 1];
     }
   });

@@ -256,6 +256,9 @@ class GzAlg {
   // Whether the vertex sketches XOR to zero (true for sketches built from edge updates only):
   // 1 known zero, 0 unknown (checked at the next query), -1 known not zero.
   std::atomic<int> zero_sum{1};
+  // Whether every update so far was applied to both of its ends (ingested pairs); not known after
+  // apply_update_batch, raw buckets or a load.
+  std::atomic<bool> paired{true};
   bool sketches_sum_to_zero();
   std::atomic<uint64_t> total_updates{0};
   std::mutex query_mtx;
@@ -318,9 +321,9 @@ class GzAlg {
   // Query prefix (DSU reset, round 0, rounds 1..K and a single-workgroup finish of the remaining
   // rounds) replayed from a HIP graph: every parameter is fixed per instance (round state lives on
   // the device), so one graph launch replaces ~5 kernel launches per round.  K is the last round
-  // the previous query needed launched rounds for: the first round after which a giant existed and
-  // at most finish_max() vertices remained outside it (queries on one stream need similar counts),
-  // else its round count plus one.  Graphs are built on first use and kept per (K, giant_ok).
+  // the previous query needed launched rounds for: the first round that regrouped at most
+  // finish_max() vertices (queries on one stream need similar counts), else its round count plus one.
+  // Graphs are built on first use and kept per (K, giant_ok, drop_ok, switches).
  public:
   bool use_graphs = true;
   bool use_finish = true;           // the single-workgroup finish of the last rounds
@@ -333,7 +336,7 @@ class GzAlg {
   hipEvent_t hround_ev = nullptr;  // that copy has landed
   bool hround_pending = false;      // hround holds the last query's diagnostics, not yet used
   bool hround_on_event = false;     // ... once hround_ev has completed
-  MapBuf<uint32_t> rep;             // the finish kernel's report: round flags, then 128 diagnostic words
+  MapBuf<uint32_t> rep;             // the finish kernel's report: round flags, then the diagnostic words
   uint32_t next_prefix = 0;  // K of the next query's prefix (0: none chosen yet)
   // The spanning-forest membership set that the eager DSU's deletion check reads is built from the
   // forest edges after a query, but only before the first eager batch that needs it.
@@ -344,8 +347,8 @@ class GzAlg {
   uint64_t unranked_seen = 0;
   // src != pairs: the batch is copied from src into pairs (device memory) by the same launch
   void eager_batch(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged);
-  void enqueue_query_prefix(bool giant_ok, uint32_t last);
-  hipGraphExec_t get_query_graph(bool giant_ok, uint32_t last);
+  void enqueue_query_prefix(bool giant_ok, bool drop_ok, uint32_t last);
+  hipGraphExec_t get_query_graph(bool giant_ok, bool drop_ok, uint32_t last);
 };
 
 // Runs f, converting exceptions to a gz_status and the thread's last-error message.
