@@ -178,7 +178,148 @@ uint64_t GzAlg::footprint(uint32_t n, const gz_alg_config& c) {
   return slab + ingest + rounds;
 }
 
-GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(seed_), cfg(c) {
+// ---- instance memory ----
+Block allocate_block(size_t dev_bytes, size_t host_bytes) {
+  Block b;
+  GZ_HIP(hipGetDevice(&b.device));
+  GZ_HIP(hipMalloc(&b.dev, dev_bytes));
+  b.dev_bytes = dev_bytes;
+  try {
+    GZ_HIP(hipHostMalloc(&b.host, host_bytes, hipHostMallocMapped | hipHostMallocCoherent));
+    b.host_bytes = host_bytes;
+    GZ_HIP(hipHostGetDevicePointer(&b.host_dev, b.host, 0));
+  } catch (...) {
+    free_block(b);
+    throw;
+  }
+  return b;
+}
+void free_block(const Block& b) {
+  if (b.dev) (void)hipFree(b.dev);
+  if (b.host) (void)hipHostFree(b.host);
+}
+
+Block BlockCache::take(size_t dev_bytes, size_t host_bytes, size_t keep) {
+  int device = 0;
+  GZ_HIP(hipGetDevice(&device));
+  {
+    std::lock_guard<std::mutex> lk(mtx_);
+    // the smallest block that is large enough and at most 1/32 larger than asked for
+    auto best = blocks_.end();
+    for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
+      if (it->device == device && it->dev_bytes >= dev_bytes && it->dev_bytes <= dev_bytes + dev_bytes / 32 &&
+          it->host_bytes >= host_bytes && (best == blocks_.end() || it->dev_bytes < best->dev_bytes))
+        best = it;
+    if (best != blocks_.end()) {
+      const Block b = *best;
+      blocks_.erase(best);
+      held_ -= b.dev_bytes;
+      return b;
+    }
+  }
+  trim(keep);
+  try {
+    return allocate_block(dev_bytes, host_bytes);
+  } catch (const GzError& e) {
+    if (e.code != GZ_ERR_OOM) throw;
+  }
+  (void)hipGetLastError();
+  trim(0);
+  return allocate_block(dev_bytes, host_bytes);
+}
+void BlockCache::put(const Block& b) {
+  if (!b.dev) return;
+  {
+    std::lock_guard<std::mutex> lk(mtx_);
+    if (held_ + b.dev_bytes <= bound_) {
+      blocks_.push_back(b);
+      held_ += b.dev_bytes;
+      return;
+    }
+  }
+  free_block(b);
+}
+void BlockCache::trim(size_t keep) {
+  std::vector<Block> out;
+  {
+    std::lock_guard<std::mutex> lk(mtx_);
+    while (held_ > keep) {
+      held_ -= blocks_.front().dev_bytes;
+      out.push_back(blocks_.front());
+      blocks_.erase(blocks_.begin());
+    }
+  }
+  for (const Block& b : out) free_block(b);
+}
+
+GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c, BlockCache* cache, size_t keep)
+    : n(n_), seed(seed_), cfg(c) {
+  try {
+    init(cache, keep);
+  } catch (...) {  // the members are about to give memory back that queued work may still use
+    if (st) {
+      (void)hipStreamSynchronize(st);
+      (void)hipStreamDestroy(st);
+    }
+    if (hround_ev) (void)hipEventDestroy(hround_ev);
+    if (eager_ev) (void)hipEventDestroy(eager_ev);
+    throw;
+  }
+}
+
+// Every buffer of fixed size; dev and host only count until they have memory.
+void GzAlg::place_buffers(Arena& dev, Arena& host) {
+  slab.place(dev, (size_t)n * geo.row);
+  col_bf.place(dev, geo.C);
+  // DSU + forest
+  parent.place(dev, n);
+  uint64_t cap = 1;
+  while (cap < 2ull * n) cap <<= 1;
+  sf_hash.place(dev, cap);
+  sf_edge.place(dev, n);
+  flags.place(dev, kNumFlags);
+  mod.place(dev, geo.samples + 2);
+  labels.place(dev, n + 1);
+  scratch.place(dev, 2 * (size_t)geo.nb);
+  // Borůvka round buffers
+  r_cnt.place(dev, n); r_off.place(dev, n); r_cursor.place(dev, n); r_samp.place(dev, n);
+  r_members[0].place(dev, n); r_members[1].place(dev, n); r_mroot[0].place(dev, n); r_mroot[1].place(dev, n);
+  r_segs[0].place(dev, n); r_segs[1].place(dev, n); r_nd.place(dev, n);
+  r_totals.place(dev, 16);
+  r_stats.place(dev, kRoundStats);
+  r_det.place(dev, (size_t)n * (8 + gb));
+  r_hint.place(dev, ((size_t)n + 3) & ~size_t(3));
+  // cross-workgroup accumulators of the reduce: one slot per workgroup and one for the giant
+  const size_t xslots = (size_t)reduce_blocks(n) + 1;
+  r_xacc.place(dev, xslots * 128);
+  r_xcnt.place(dev, xslots);
+  // device ingest
+  pending.place(dev, 2 * cap_pairs);
+  dst_arr.place(dev, 2 * cap_pairs);
+  merged.place(dev, cap_pairs);
+  g_totals.place(dev, 4);
+  g_tiles.place(dev, 2 * cap_pairs / tile + n + 1);
+  if (n <= kPartMaxVertices) {  // bucket-partition grouping (no device-scope atomics per update)
+    g_rec.place(dev, 2 * cap_pairs * part_rec_bytes(n));
+    g_place.place(dev, part_place_len());
+    g_binned.place(dev, part_bins_len());
+    g_binoff.place(dev, part_bins_len());
+  } else {
+    g_cnt.place(dev, n); g_off.place(dev, n + 1); g_toff.place(dev, n + 1); g_cursor.place(dev, n);
+    g_partials.place(dev, group_partials_len(n));
+  }
+  // words shared with the host
+  eager_inv.place(host, 1);
+  qforce.place(host, 1);
+  hflags.place(host, std::max<size_t>(kNumFlags, geo.samples + 2));
+  hsmall.place(host, 16);
+  hround.place(host, kRoundStats);
+  rep.place(host, geo.samples + 2 + kRoundStats);
+  aq_in.place(host, 2 * kAnswerPoints);
+  aq_out.place(host, kNumFlags + kAnswerPoints / 4);
+}
+
+void GzAlg::init(BlockCache* cache, size_t keep) {
   if (n < 2) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices must be >= 2");
   if (n > (1u << 31)) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices above 2^31 is not supported");
   if (cfg.sketches_factor <= 0) cfg.sketches_factor = 1;  // cc_alg_configuration.cpp:15-23
@@ -196,56 +337,45 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   grid_cap = (uint32_t)(device_cu_count() * per_cu);
   GZ_HIP(hipStreamCreate(&st));
 
-  // sketch slab
-  slab.alloc((size_t)n * geo.row);
+  cap_pairs = cfg.flush_threshold ? (size_t)cfg.flush_threshold : default_cap_pairs(n, desired_updates_per_batch());
+  if (cap_pairs > (size_t(1) << 30)) cap_pairs = size_t(1) << 30;
+
+  Arena dev, host;
+  place_buffers(dev, host);
+  auto round_up = [](size_t x, size_t to) { return (x + to - 1) / to * to; };
+  const size_t dev_bytes = round_up(dev.used, size_t(2) << 20), host_bytes = round_up(host.used, size_t(32) << 10);
+  mem.b = cache ? cache->take(dev_bytes, host_bytes, keep) : allocate_block(dev_bytes, host_bytes);
+  mem.cache = cache;
+  dev = Arena{nullptr, static_cast<uint8_t*>(mem.b.dev), 0};
+  host = Arena{static_cast<uint8_t*>(mem.b.host), static_cast<uint8_t*>(mem.b.host_dev), 0};
+  place_buffers(dev, host);
+
+  // Nothing is assumed about the memory's contents.
   launch_fill_u32(reinterpret_cast<uint32_t*>(slab.p), 0, slab.n / 4, st);
   auto bf = column_bitflips(geo);
-  col_bf.alloc(bf.size());
   GZ_HIP(hipMemcpyAsync(col_bf.p, bf.data(), bf.size() * 8, hipMemcpyHostToDevice, st));
 
-  // DSU + forest
-  parent.alloc(n);
-  uint64_t cap = 1;
-  while (cap < 2ull * n) cap <<= 1;
-  sf_hash.alloc(cap);
-  sf_edge.alloc(n);
-  flags.alloc(kNumFlags);
-  mod.alloc(geo.samples + 2);
-  labels.alloc(n + 1);
   dsu.parent = parent.p;
   dsu.sf_hash = sf_hash.p;
-  dsu.sf_mask = cap - 1;
+  dsu.sf_mask = sf_hash.n - 1;
   dsu.sf_edge = sf_edge.p;
   dsu.flags = flags.p;
   dsu.mod = mod.p;
   dsu.nmod = geo.samples + 2;
   dsu.prio_seed = (uint32_t)(seed * 0x9E3779B97F4A7C15ULL >> 32);
   dsu.n = n;
-  eager_inv.ensure(1);
   eager_inv.p[0] = 0;
   dsu.inv_mirror = eager_inv.d;
-  qforce.ensure(1);
   qforce.p[0] = 1;
   dsu.query_force = qforce.d;
   launch_fill_u32(flags.p, 0, kNumFlags, st);  // the reset below keeps the bad-input flag
   launch_dsu_reset(dsu, st);
 
-  // Borůvka round buffers
-  r_cnt.alloc(n); r_off.alloc(n); r_cursor.alloc(n); r_samp.alloc(n);
-  r_members[0].alloc(n); r_members[1].alloc(n); r_mroot[0].alloc(n); r_mroot[1].alloc(n);
-  r_segs[0].alloc(n); r_segs[1].alloc(n); r_nd.alloc(n);
-  r_totals.alloc(16);
-  r_stats.alloc(kRoundStats);
-  r_det.alloc((size_t)n * (8 + gb));
-  r_hint.alloc(((size_t)n + 3) & ~size_t(3));
   launch_fill_u32(reinterpret_cast<uint32_t*>(r_hint.p), 0, r_hint.n / 4, st);  // no classes before the first query
   launch_fill_u32(r_stats.p, 0, kRoundStats, st);
-  // cross-workgroup accumulators of the reduce: one slot per workgroup and one for the giant
-  const size_t xslots = (size_t)reduce_blocks(n) + 1;
-  r_xacc.alloc(xslots * 128);
-  r_xcnt.alloc(xslots);
-  launch_fill_u64(r_xacc.p, 0, xslots * 128, st);
-  launch_fill_u32(r_xcnt.p, 0, xslots, st);
+  launch_fill_u64(r_xacc.p, 0, r_xacc.n, st);
+  launch_fill_u32(r_xcnt.p, 0, r_xcnt.n, st);
+  const size_t xslots = r_xcnt.n;
   rb = RoundBufs{r_cnt.p, r_off.p, r_cursor.p, {r_members[0].p, r_members[1].p},
                  {r_mroot[0].p, r_mroot[1].p}, {r_segs[0].p, r_segs[1].p}, r_nd.p, r_totals.p,
                  r_xacc.p, r_xcnt.p, (uint32_t)xslots, r_samp.p, r_stats.p, r_det.p, r_hint.p};
@@ -255,32 +385,18 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   // sets the state words again.
   launch_round_state_init(rb, n, st);
 
-  // device ingest
-  cap_pairs = cfg.flush_threshold ? (size_t)cfg.flush_threshold : default_cap_pairs(n, desired_updates_per_batch());
-  if (cap_pairs > (size_t(1) << 30)) cap_pairs = size_t(1) << 30;
-  pending.alloc(2 * cap_pairs);
-  dst_arr.alloc(2 * cap_pairs);
-  merged.alloc(cap_pairs);
-  g_totals.alloc(4);
-  g_tiles.alloc(2 * cap_pairs / tile + n + 1);
   gbufs = GroupBufs{};
   gbufs.totals = g_totals.p;
   gbufs.dst_arr = dst_arr.p;
   gbufs.tiles = g_tiles.p;
   gbufs.bad = flags.p + kFlagBadInput;
-  if (n <= kPartMaxVertices) {  // bucket-partition grouping (no device-scope atomics per update)
-    g_rec.alloc(2 * cap_pairs * part_rec_bytes(n));
-    g_place.alloc(part_place_len());
-    g_binned.alloc(part_bins_len());
-    g_binoff.alloc(part_bins_len());
+  if (n <= kPartMaxVertices) {
     launch_fill_u32(g_binned.p, 0, g_binned.n, st);
     gbufs.rec = g_rec.p;
     gbufs.place = g_place.p;
     gbufs.binned = g_binned.p;
     gbufs.binoff = g_binoff.p;
   } else {
-    g_cnt.alloc(n); g_off.alloc(n + 1); g_toff.alloc(n + 1); g_cursor.alloc(n);
-    g_partials.alloc(group_partials_len(n));
     gbufs.cnt = g_cnt.p;
     gbufs.off = g_off.p;
     gbufs.toff = g_toff.p;
@@ -291,13 +407,7 @@ GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c) : n(n_), seed(
   // host staging
   stage_cap = std::max<size_t>(desired_updates_per_batch(), cfg.batched ? (size_t(1) << 22) : 0);
   stages.resize(cfg.batched ? 2 : 4);
-  vstamp.assign(n, 0);
-  vtiles.assign(n, 0);
   eager_cap = size_t(1) << 20;
-  hflags.alloc(std::max<size_t>(kNumFlags, geo.samples + 2));
-  hsmall.alloc(16);
-  hround.alloc(kRoundStats);
-  rep.ensure(dsu.nmod + kRoundStats);
   GZ_HIP(hipEventCreateWithFlags(&hround_ev, hipEventDisableTiming));
   GZ_HIP(hipEventCreateWithFlags(&eager_ev, hipEventDisableTiming));
   GZ_HIP(hipStreamSynchronize(st));
@@ -402,6 +512,10 @@ void GzAlg::apply_update_batch(uint32_t src, const uint32_t* dsts, size_t k) {
 void GzAlg::submit_stage_locked() {
   Stage& s = stages[cur_stage];
   if (!s.used) return;
+  if (vstamp.empty()) {
+    vstamp.assign(n, 0);
+    vtiles.assign(n, 0);
+  }
   ++epoch;
   if (epoch == 0) {
     std::fill(vstamp.begin(), vstamp.end(), 0u);
@@ -728,13 +842,11 @@ void GzAlg::ensure_answer() {
 // may not, so after those the sum is checked once (one pass over the sketches).
 bool GzAlg::sketches_sum_to_zero() {
   if (zero_sum == 0) {
-    DevBuf<uint64_t> sa, sg;
-    sa.alloc(geo.nb);
-    sg.alloc(geo.nb);
-    launch_sum_all(gb, slab.p, geo, sa.p, sg.p, st);
+    uint64_t *sa = scratch.p, *sg = scratch.p + geo.nb;
+    launch_sum_all(gb, slab.p, geo, sa, sg, st);
     std::vector<uint64_t> ha(geo.nb), hg(geo.nb);
-    GZ_HIP(hipMemcpyAsync(ha.data(), sa.p, geo.nb * 8, hipMemcpyDeviceToHost, st));
-    GZ_HIP(hipMemcpyAsync(hg.data(), sg.p, geo.nb * (size_t)gb, hipMemcpyDeviceToHost, st));
+    GZ_HIP(hipMemcpyAsync(ha.data(), sa, geo.nb * 8, hipMemcpyDeviceToHost, st));
+    GZ_HIP(hipMemcpyAsync(hg.data(), sg, geo.nb * (size_t)gb, hipMemcpyDeviceToHost, st));
     GZ_HIP(hipStreamSynchronize(st));
     bool zero = true;
     for (uint32_t b = 0; b < geo.nb && zero; ++b) zero = ha[b] == 0;
@@ -1036,11 +1148,9 @@ void GzAlg::dump(uint32_t v0, uint32_t count, void* outp) {
 
 uint64_t GzAlg::digest() {
   flush_all();
-  DevBuf<uint64_t> d;
-  d.alloc(1);
-  launch_digest(gb, slab.p, geo, d.p, st);
+  launch_digest(gb, slab.p, geo, scratch.p, st);
   uint64_t h = 0;
-  GZ_HIP(hipMemcpyAsync(&h, d.p, 8, hipMemcpyDeviceToHost, st));
+  GZ_HIP(hipMemcpyAsync(&h, scratch.p, 8, hipMemcpyDeviceToHost, st));
   GZ_HIP(hipStreamSynchronize(st));
   return h;
 }

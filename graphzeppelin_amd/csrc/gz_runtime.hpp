@@ -30,15 +30,29 @@ struct GzError : std::runtime_error {
                           std::string(#x) + " failed: " + hipGetErrorString(e_));                   \
   } while (0)
 
-// Owning device buffer.
+// One allocation cut into buffers on 256-byte boundaries.  The same sequence of place() calls runs
+// twice: without memory, which only adds up the size, then on the memory.
+struct Arena {
+  uint8_t* host = nullptr;    // address the host uses (host memory only)
+  uint8_t* device = nullptr;  // address the device uses
+  size_t used = 0;
+  size_t take(size_t bytes) {
+    const size_t at = used;
+    used = (used + bytes + 255) & ~size_t(255);
+    return at;
+  }
+};
+
+// Device buffer: owned (alloc), or part of an arena (place).
 template <class T>
 struct DevBuf {
   T* p = nullptr;
   size_t n = 0;
+  bool own = true;
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n) {
+  DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n), own(o.own) {
     o.p = nullptr;
     o.n = 0;
   }
@@ -52,10 +66,19 @@ struct DevBuf {
   void ensure(size_t count) {
     if (count > n) alloc(count);
   }
+  void place(Arena& a, size_t count) {
+    release();
+    const size_t at = a.take(count * sizeof(T));
+    if (!a.device) return;
+    p = reinterpret_cast<T*>(a.device + at);
+    n = count;
+    own = false;
+  }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && own) (void)hipFree(p);
     p = nullptr;
     n = 0;
+    own = true;
   }
 };
 
@@ -88,13 +111,14 @@ struct PinBuf {
   }
 };
 
-// Owning pinned host buffer that kernels read and write in place (fine-grained, mapped): for a
-// few words per query, a kernel access over the bus replaces a copy launch.
+// Pinned host buffer that kernels read and write in place (fine-grained, mapped): for a few words per
+// query, a kernel access over the bus replaces a copy launch.  Owned (ensure), or part of an arena.
 template <class T>
 struct MapBuf {
   T* p = nullptr;  // host address
   T* d = nullptr;  // device address
   size_t n = 0;
+  bool own = true;
   MapBuf() = default;
   MapBuf(const MapBuf&) = delete;
   MapBuf& operator=(const MapBuf&) = delete;
@@ -106,10 +130,66 @@ struct MapBuf {
     GZ_HIP(hipHostGetDevicePointer((void**)&d, p, 0));
     n = count;
   }
+  void place(Arena& a, size_t count) {
+    release();
+    const size_t at = a.take(count * sizeof(T));
+    if (!a.host) return;
+    p = reinterpret_cast<T*>(a.host + at);
+    d = reinterpret_cast<T*>(a.device + at);
+    n = count;
+    own = false;
+  }
   void release() {
-    if (p) (void)hipHostFree(p);
+    if (p && own) (void)hipHostFree(p);
     p = d = nullptr;
     n = 0;
+    own = true;
+  }
+};
+
+// The memory of one instance: a device block and a few KB of pinned host memory.
+struct Block {
+  void* dev = nullptr;
+  size_t dev_bytes = 0;
+  void* host = nullptr;
+  void* host_dev = nullptr;  // the device's address of host
+  size_t host_bytes = 0;
+  int device = 0;  // the device dev is on
+};
+// Blocks of released instances, kept for later ones: the driver hands out tens of GB/s at most, so a
+// server that admits and releases streams spends most of its time in allocation otherwise.  Holds at
+// most `bound` bytes; what does not fit, and everything at the end, goes back to the device.  Safe
+// with several threads; a block is put back once its instance's streams are idle.
+class BlockCache {
+ public:
+  explicit BlockCache(size_t bound) : bound_(bound) {}
+  BlockCache(const BlockCache&) = delete;
+  BlockCache& operator=(const BlockCache&) = delete;
+  ~BlockCache() { trim(0); }
+  // A block of at least these sizes, with at most `keep` bytes held besides it.
+  Block take(size_t dev_bytes, size_t host_bytes, size_t keep);
+  void put(const Block& b);
+  void trim(size_t keep);
+
+ private:
+  std::mutex mtx_;
+  std::vector<Block> blocks_;  // oldest first
+  size_t held_ = 0;
+  const size_t bound_;
+};
+Block allocate_block(size_t dev_bytes, size_t host_bytes);
+void free_block(const Block& b);
+
+// An instance's block, given back when the instance ends.
+struct Memory {
+  Block b;
+  BlockCache* cache = nullptr;
+  Memory() = default;
+  Memory(const Memory&) = delete;
+  Memory& operator=(const Memory&) = delete;
+  ~Memory() {
+    if (cache) cache->put(b);
+    else free_block(b);
   }
 };
 
@@ -145,9 +225,12 @@ class GzSketch {
 // CCSketchAlg (include/cc_sketch_alg.h) with every vertex sketch resident in HBM.
 class GzAlg {
  public:
-  GzAlg(uint32_t n, uint64_t seed, const gz_alg_config& cfg);
+  // cache (or nullptr): where the instance's memory comes from and goes back to, with at most `keep`
+  // bytes left in it meanwhile; it outlives the instance.
+  GzAlg(uint32_t n, uint64_t seed, const gz_alg_config& cfg, BlockCache* cache = nullptr, size_t keep = 0);
   ~GzAlg();
 
+  Memory mem;  // declared before the buffers placed in it
   uint32_t n;
   uint64_t seed;
   gz_alg_config cfg;
@@ -224,11 +307,12 @@ class GzAlg {
   DevBuf<uint8_t> eager_merged;
   hipEvent_t eager_ev = nullptr;
   size_t eager_used = 0, eager_cap;
-  PinBuf<uint32_t> hflags;  // device flags, or a query's round flags
-  PinBuf<uint32_t> hsmall;
+  MapBuf<uint32_t> hflags;  // device flags, or a query's round flags
+  MapBuf<uint32_t> hsmall;
   MapBuf<uint32_t> eager_inv;  // mapped mirror of kFlagEagerInvalid, cleared after each query
   MapBuf<uint32_t> qforce;     // DsuDev::query_force: 1 runs the next query whatever the eager DSU's state
   bool eager_live() const { return !(eager_inv.p && *reinterpret_cast<const volatile uint32_t*>(eager_inv.p)); }
+  static constexpr size_t kAnswerPoints = 1024;  // pairs a group holds without growing these two
   MapBuf<uint32_t> aq_in;  // a query group's point queries: us then vs, read by the answer kernel
   MapBuf<uint32_t> aq_out;  // the error flags, then one answer byte per point query, written by it
 
@@ -243,6 +327,7 @@ class GzAlg {
   bool prof = false;
   std::vector<Timed> timed;
   std::vector<hipEvent_t> ev_pool;
+  DevBuf<uint64_t> scratch;     // results read back by the host: the digest, or the sketches' sum
   DevBuf<uint64_t> prof_bytes;  // device accumulator for grouped-flush bytes
   gz_alg_profile profile{};
   hipEvent_t prof_begin(int kind, double host_bytes, bool dev_bytes, uint64_t items);
@@ -332,7 +417,7 @@ class GzAlg {
   static constexpr uint32_t kFirstGraphRounds = 12;
  private:
   std::map<uint32_t, hipGraphExec_t> query_graphs;
-  PinBuf<uint32_t> hround;  // per-round diagnostics of the last query (copied when it ends)
+  MapBuf<uint32_t> hround;  // per-round diagnostics of the last query (copied when it ends)
   hipEvent_t hround_ev = nullptr;  // that copy has landed
   bool hround_pending = false;      // hround holds the last query's diagnostics, not yet used
   bool hround_on_event = false;     // ... once hround_ev has completed
@@ -347,6 +432,8 @@ class GzAlg {
   uint64_t unranked_seen = 0;
   // src != pairs: the batch is copied from src into pairs (device memory) by the same launch
   void eager_batch(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged);
+  void init(BlockCache* cache, size_t keep);
+  void place_buffers(Arena& dev, Arena& host);
   void enqueue_query_prefix(bool giant_ok, bool drop_ok, uint32_t last);
   hipGraphExec_t get_query_graph(bool giant_ok, bool drop_ok, uint32_t last);
 };

@@ -174,25 +174,31 @@ class Server {
   };
   uint64_t budget;
   uint64_t reserved = 0;
+  // Memory of released tenants, within the part of the budget that no tenant has reserved.  Declared
+  // before the tenants, whose memory goes back to it.
+  static constexpr uint64_t kKeepMax = uint64_t(16) << 30;
+  BlockCache kept;
   int workers;
   std::mutex mtx;
   std::map<int, Tenant> tenants;
   int next_id = 0;
 
-  Server(uint64_t b, int w) : budget(b), workers(std::max(1, w)) {}
+  Server(uint64_t b, int w) : budget(b), kept(std::min<uint64_t>(b / 4, kKeepMax)), workers(std::max(1, w)) {}
 
   int admit(uint32_t n, uint64_t seed, const gz_alg_config& cfg) {
     const uint64_t fp = GzAlg::footprint(n, cfg);
+    uint64_t unreserved;
     {
       std::lock_guard<std::mutex> lk(mtx);
       if (reserved + fp > budget)
         throw GzError(GZ_ERR_ADMISSION, "tenant footprint " + std::to_string(fp) + " B exceeds the unreserved budget " +
                                             std::to_string(budget - reserved) + " B");
       reserved += fp;
+      unreserved = budget - reserved;
     }
     std::unique_ptr<GzAlg> a;
     try {
-      a.reset(new GzAlg(n, seed, cfg));
+      a.reset(new GzAlg(n, seed, cfg, &kept, unreserved));
     } catch (...) {
       std::lock_guard<std::mutex> lk(mtx);
       reserved -= fp;
