@@ -2373,21 +2373,21 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
   }
 }
 
-// ConnectedComponents (src/return_types.cpp:5-19): root of every vertex and the root count.
-__global__ void k_labels(uint32_t* __restrict__ parent, uint32_t n, uint32_t* __restrict__ labels,
-                         uint32_t* __restrict__ ncc) {
-  const uint32_t lane = lane_id();
-  for (uint32_t v0 = (blockIdx.x * blockDim.x + threadIdx.x) - lane; v0 < n; v0 += gridDim.x * blockDim.x) {
-    const uint32_t v = v0 + lane;
-    bool is_root = false;
-    if (v < n) {
-      const uint32_t r = dsu_find(parent, v);
-      labels[v] = r;
-      is_root = r == v;
-    }
-    const uint64_t m = __ballot(is_root);
-    if (lane == 0 && m) atomicAdd(ncc, (uint32_t)__popcll(m));
+// ConnectedComponents (src/return_types.cpp:5-19): root of every vertex and the root count.  The count
+// takes one atomic per workgroup of 1024: one per wave with a root, on one address at 11 ns each, was
+// the kernel's time on graphs with many components (2^20 R-MAT vertices, a third isolated: 169 us).
+constexpr uint32_t kLabelBlock = 1024;
+__global__ void __launch_bounds__(kLabelBlock)
+k_labels(uint32_t* __restrict__ parent, uint32_t n, uint32_t* __restrict__ labels, uint32_t* __restrict__ ncc) {
+  const uint32_t v = blockIdx.x * kLabelBlock + threadIdx.x;
+  bool is_root = false;
+  if (v < n) {
+    const uint32_t r = dsu_find(parent, v);
+    labels[v] = r;
+    is_root = r == v;
   }
+  const uint32_t roots = (uint32_t)__syncthreads_count(is_root);
+  if (threadIdx.x == 0 && roots) atomicAdd(ncc, roots);
 }
 __global__ void k_point_queries(uint32_t* __restrict__ parent, const uint32_t* __restrict__ qa,
                                 const uint32_t* __restrict__ qb, uint32_t nq, uint8_t* __restrict__ out) {
@@ -2814,7 +2814,7 @@ void launch_digest(int gbytes, const unsigned char* slab, const Geo& g, uint64_t
 
 void launch_labels(const DsuDev& d, uint32_t* labels, uint32_t* ncc, hipStream_t s) {
   launch_fill_u32(ncc, 0, 1, s);
-  hipLaunchKernelGGL(k_labels, dim3(grid_for(d.n, 256)), dim3(256), 0, s, d.parent, d.n, labels, ncc);
+  hipLaunchKernelGGL(k_labels, dim3((d.n + kLabelBlock - 1) / kLabelBlock), dim3(kLabelBlock), 0, s, d.parent, d.n, labels, ncc);
 }
 void launch_answer_points(const DsuDev& d, const uint32_t* q, uint32_t nq, uint32_t* out, hipStream_t s) {
   hipLaunchKernelGGL(k_answer_points, dim3(grid_for(nq > kNumFlags ? nq : kNumFlags, 256)), dim3(256), 0, s, d.parent,
