@@ -2498,15 +2498,21 @@ __global__ void k_packed(unsigned char* __restrict__ slab, Geo g, uint32_t v0, u
 }
 
 // Bucket-wise XOR of every vertex sketch into out_a / out_g (nb entries each, zero on entry): one
-// thread per (bucket, chunk of kSumChunk vertices), one device-scope atomic per thread.
-constexpr uint32_t kSumChunk = 1024;
+// thread per (bucket, chunk of vertices), one device-scope atomic per thread.  The chunks are cut so
+// that a small graph still fills the chip: 1024 vertices in one chunk took 290 us.
+constexpr uint32_t kSumChunkMax = 1024, kSumChunks = 512;
+uint32_t sum_chunk(uint32_t n) {
+  const uint32_t c = (n + kSumChunks - 1) / kSumChunks;
+  return c < 4 ? 4 : c > kSumChunkMax ? kSumChunkMax : c;
+}
 template <class G>
 __global__ void __launch_bounds__(256)
-k_sum_all(const unsigned char* __restrict__ slab, Geo g, uint64_t* __restrict__ out_a, G* __restrict__ out_g) {
+k_sum_all(const unsigned char* __restrict__ slab, Geo g, uint32_t chunk, uint64_t* __restrict__ out_a,
+          G* __restrict__ out_g) {
   const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= g.nb) return;
-  const uint32_t v0 = blockIdx.y * kSumChunk;
-  const uint32_t v1 = v0 + kSumChunk < g.n ? v0 + kSumChunk : g.n;
+  const uint32_t v0 = blockIdx.y * chunk;
+  const uint32_t v1 = v0 + chunk < g.n ? v0 + chunk : g.n;
   uint64_t a = 0;
   G gm = 0;
   for (uint32_t v = v0; v < v1; ++v) {
@@ -2795,11 +2801,12 @@ void launch_sum_all(int gbytes, const unsigned char* slab, const Geo& g, uint64_
   launch_fill_u64(out_a, 0, g.nb, s);
   if (gbytes == 4) launch_fill_u32((uint32_t*)out_g, 0, g.nb, s);
   else launch_fill_u64((uint64_t*)out_g, 0, g.nb, s);
-  const dim3 grid((g.nb + 255) / 256, (g.n + kSumChunk - 1) / kSumChunk);
+  const uint32_t chunk = sum_chunk(g.n);
+  const dim3 grid((g.nb + 255) / 256, (g.n + chunk - 1) / chunk);
   if (gbytes == 4)
-    hipLaunchKernelGGL(k_sum_all<uint32_t>, grid, dim3(256), 0, s, slab, g, out_a, (uint32_t*)out_g);
+    hipLaunchKernelGGL(k_sum_all<uint32_t>, grid, dim3(256), 0, s, slab, g, chunk, out_a, (uint32_t*)out_g);
   else
-    hipLaunchKernelGGL(k_sum_all<uint64_t>, grid, dim3(256), 0, s, slab, g, out_a, (uint64_t*)out_g);
+    hipLaunchKernelGGL(k_sum_all<uint64_t>, grid, dim3(256), 0, s, slab, g, chunk, out_a, (uint64_t*)out_g);
 }
 
 void launch_digest(int gbytes, const unsigned char* slab, const Geo& g, uint64_t* out, hipStream_t s) {
