@@ -669,10 +669,12 @@ constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;
 constexpr uint32_t kScanSpan = kScanBlock * kScanItems;
 
-__device__ inline uint64_t pack_ct(uint32_t c, uint32_t tile) {
-  const uint64_t nt = tile ? (c + tile - 1) / tile : 0;
-  return (nt << 32) | c;
+// Tiles of c destinations; almost every vertex has at most one, which spares the division's ~40
+// instructions.
+__device__ inline uint32_t tile_count(uint32_t c, uint32_t tile) {
+  return c <= tile ? (c != 0 ? 1u : 0u) : (c - 1) / tile + 1;
 }
+__device__ inline uint64_t pack_ct(uint32_t c, uint32_t tile) { return ((uint64_t)tile_count(c, tile) << 32) | c; }
 __device__ inline uint64_t block_excl_scan_u64(uint64_t x, uint64_t* total) {
   __shared__ uint64_t wsum[kScanBlock / kWave];
   const uint32_t lane = lane_id(), wid = threadIdx.x / kWave;
@@ -918,7 +920,7 @@ k_part_scatter(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32
 // algorithmic bytes (4c + 2 min(S, c * per_update)).
 __device__ inline uint64_t write_tiles(uint32_t v, uint32_t o, uint32_t c, uint32_t tile, Tile* __restrict__ tiles,
                                        uint32_t t0, uint64_t S, uint64_t per_update) {
-  const uint32_t nt = (c + tile - 1) / tile;
+  const uint32_t nt = tile_count(c, tile);
   for (uint32_t j = 0; j < nt; ++j) {
     const uint32_t b = j * tile;
     tiles[t0 + j] = Tile{v, o + b, (c - b) < tile ? (c - b) : tile, nt > 1 ? 1u : 0u};
@@ -962,28 +964,25 @@ k_part_group(const typename PartRec<PACK>::T* __restrict__ rec, uint32_t nb, uin
   const uint32_t rest = s + kKeep * kPartBlock + t;
   for (uint32_t j = rest; j < e; j += kPartBlock) atomicAdd(lc + PartRec<PACK>::local(rec[j], nb), 1u);
   __syncthreads();
-  // exclusive scan of the entries and tiles per vertex: a thread owns `per` consecutive vertices
-  const uint32_t per = (R + kPartBlock - 1) / kPartBlock;
-  const uint32_t k0 = t * per;
+  // exclusive scan of the entries and tiles per vertex: thread t owns vertices t, t + 1024, ... (their
+  // runs' order is free, and consecutive lanes read consecutive banks)
   uint64_t mine = 0;
-  for (uint32_t k = 0; k < per; ++k)
-    if (k0 + k < R) mine += pack_ct(lc[k0 + k], tile);
+  for (uint32_t k = t; k < R; k += kPartBlock) mine += pack_ct(lc[k], tile);
   uint64_t tot;
   uint64_t run = part_scan(mine, wsum, &tot);
   if (t == 0) s_tile0 = atomicAdd(totals + 1, (uint32_t)(tot >> 32));
   __syncthreads();
   const uint32_t t0 = s_tile0, pmask = (1u << nb) - 1;
   uint64_t bytes = 0;
-  for (uint32_t k = 0; k < per; ++k)
-    if (k0 + k < R) {
-      const uint32_t c = lc[k0 + k];
-      const uint32_t o = s + (uint32_t)run;
-      if (c)
-        bytes += write_tiles((((b << shift) | (k0 + k)) * kPlaceInv) & pmask, o, c, tile, tiles,
-                             t0 + (uint32_t)(run >> 32), S, per_update);
-      lc[k0 + k] = o;  // becomes the vertex's cursor
-      run += pack_ct(c, tile);
-    }
+  for (uint32_t k = t; k < R; k += kPartBlock) {
+    const uint32_t c = lc[k];
+    const uint32_t o = s + (uint32_t)run;
+    if (c)
+      bytes += write_tiles((((b << shift) | k) * kPlaceInv) & pmask, o, c, tile, tiles, t0 + (uint32_t)(run >> 32), S,
+                           per_update);
+    lc[k] = o;  // becomes the vertex's cursor
+    run += pack_ct(c, tile);
+  }
   add_bytes(acc, bytes);
   __syncthreads();
 #pragma unroll
@@ -1041,20 +1040,17 @@ k_group_small(const uint2* __restrict__ pairs, uint32_t count, uint32_t n, uint3
     oy[k] = atomicAdd(cnt + sy[k], 1u);
   }
   __syncthreads();
-  const uint32_t per = (T + kPartBlock - 1) / kPartBlock, k0 = t * per;
   uint64_t mine = 0;
-  for (uint32_t k = 0; k < per; ++k)
-    if (k0 + k < T) mine += pack_ct(cnt[k0 + k], tile);
+  for (uint32_t k = t; k < T; k += kPartBlock) mine += pack_ct(cnt[k], tile);
   uint64_t tot;
   uint64_t run = part_scan(mine, wsum, &tot);
   uint64_t bytes = 0;
-  for (uint32_t k = 0; k < per; ++k)
-    if (k0 + k < T) {
-      const uint32_t c = cnt[k0 + k];
-      if (c) bytes += write_tiles(key[k0 + k], (uint32_t)run, c, tile, tiles, (uint32_t)(run >> 32), S, per_update);
-      cnt[k0 + k] = (uint32_t)run;
-      run += pack_ct(c, tile);
-    }
+  for (uint32_t k = t; k < T; k += kPartBlock) {
+    const uint32_t c = cnt[k];
+    if (c) bytes += write_tiles(key[k], (uint32_t)run, c, tile, tiles, (uint32_t)(run >> 32), S, per_update);
+    cnt[k] = (uint32_t)run;
+    run += pack_ct(c, tile);
+  }
   if (t == 0) totals[1] = (uint32_t)(tot >> 32);
   add_bytes(acc, bytes);
   __syncthreads();
