@@ -789,7 +789,7 @@ k_make_tiles(const uint32_t* __restrict__ cnt, const uint32_t* __restrict__ off,
 //      with one device atomic).  The order of one vertex's destinations, and of the tiles, is
 //      arbitrary, which XOR does not see.
 // Bound by the scattered record writes (k_part_scatter: a workgroup's run in a bin is a few lines) and,
-// for small flushes, by the launches' latency.  Against contiguous ranges of ids, 8-byte records, a
+// for small flushes, by the launches' latency.  With the direct writes alone, against contiguous ranges of ids, 8-byte records, a
 // count matrix with two scan launches and a per-vertex scan for the tiles (7 launches): 24M Chung-Lu
 // updates on 2^18 vertices 1025 -> 777 us, 16M R-MAT on 2^20 2190 -> 504 us (one range held 4% of the
 // entries), flushes of about 730k updates of a serving trace 87 -> 35 us.
@@ -864,7 +864,7 @@ k_part_hist(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32_t 
             uint32_t nblk, uint32_t* __restrict__ binned, uint32_t* __restrict__ place,
             uint32_t* __restrict__ totals, uint32_t* __restrict__ bad_flag) {
   __shared__ uint32_t h[kPartBins];
-  if (threadIdx.x < bins) h[threadIdx.x] = 0;
+  for (uint32_t b = threadIdx.x; b < bins; b += kPartBlock) h[b] = 0;
   if (blockIdx.x == 0 && threadIdx.x == 0) totals[1] = 0;
   __syncthreads();
   size_t lo, hi;
@@ -879,34 +879,131 @@ k_part_hist(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32_t 
     atomicAdd(h + (((p.y * kPlaceMul) & mask) >> shift), 1u);
   });
   __syncthreads();
-  if (threadIdx.x < bins) {
-    const uint32_t c = h[threadIdx.x];
-    place[(size_t)blockIdx.x * bins + threadIdx.x] = c ? atomicAdd(binned + threadIdx.x, c) : 0u;
+  for (uint32_t b = threadIdx.x; b < bins; b += kPartBlock) {
+    const uint32_t c = h[b];
+    place[(size_t)blockIdx.x * bins + b] = c ? atomicAdd(binned + b, c) : 0u;
   }
 }
 
-// binoff: bins + 1 words, the bins' starts in the record list.
-template <bool PACK>
+// Large flushes move their records through LDS: a workgroup sorts a tile of up to kTile records by
+// bin there and writes each bin's records as one run, where single records written straight to their
+// places kept 256 * 1024 partly filled lines open, which were evicted from the L2s before they filled.
+// 24M Chung-Lu updates on 2^18 vertices 450 -> 168 us, 16M R-MAT on 2^20 298 -> 115 us.  (2048 bins: 215
+// and 154, which the group kernel wins back on the first only, 293 -> 231 and 178 -> 187 us.)
+template <class T>
+struct StageLds {
+  static constexpr uint32_t kTile = sizeof(T) == 4 ? 16384 : 8192, kPer = kTile / kPartBlock;
+  uint32_t* cnt;    // kPartBins: records per key in the tile
+  uint32_t* first;  // kPartBins: a key's first record in the sorted tile
+  T* item;          // kTile
+  uint16_t* key;    // kTile
+  uint64_t* wsum;
+  static constexpr size_t bytes() { return 2 * 4 * kPartBins + kTile * (sizeof(T) + 2); }
+  __device__ StageLds(unsigned char* p, uint64_t* w) : wsum(w) {
+    cnt = reinterpret_cast<uint32_t*>(p);
+    first = cnt + kPartBins;
+    item = reinterpret_cast<T*>(first + kPartBins);
+    key = reinterpret_cast<uint16_t*>(item + kTile);
+  }
+  // Writes the workgroup's records r[j] with k[j] < kPartBins (others are left out) to out[cur[key]...]
+  // and moves the cursors on.  cur: kPartBins words in LDS.
+  __device__ void write(const T* r, const uint32_t* k, uint32_t* cur, T* __restrict__ out) {
+    constexpr uint32_t M = kPartBins / kPartBlock;  // keys of a thread
+    const uint32_t t = threadIdx.x;
+    __syncthreads();  // the previous tile's reads are done, and cur is written
+#pragma unroll
+    for (uint32_t j = 0; j < M; ++j) cnt[M * t + j] = 0;
+    __syncthreads();
+    uint32_t rank[kPer];
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) rank[j] = k[j] < kPartBins ? atomicAdd(cnt + k[j], 1u) : 0u;
+    __syncthreads();
+    uint32_t c[M], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < M; ++j) {
+      c[j] = cnt[M * t + j];
+      sum += c[j];
+    }
+    uint64_t total;
+    const uint32_t f = (uint32_t)part_scan(sum, wsum, &total);
+    for (uint32_t j = 0, at = f; j < M; at += c[j], ++j) first[M * t + j] = at;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j)
+      if (k[j] < kPartBins) {
+        const uint32_t at = first[k[j]] + rank[j];
+        item[at] = r[j];
+        key[at] = (uint16_t)k[j];
+      }
+    __syncthreads();
+    for (uint32_t j = 0, at = f; j < M; at += c[j], ++j) {
+      first[M * t + j] = cur[M * t + j] - at;  // a record's place is its place in the tile plus its key's base
+      cur[M * t + j] += c[j];
+    }
+    __syncthreads();
+    for (uint32_t i = t; i < (uint32_t)total; i += kPartBlock) out[first[key[i]] + i] = item[i];
+  }
+};
+
+// binoff: bins + 1 words, the bins' starts in the record list.  STAGED: through LDS (StageLds).
+template <bool PACK, bool STAGED>
 __global__ void __launch_bounds__(kPartBlock)
 k_part_scatter(const uint2* __restrict__ pairs, size_t count, uint32_t n, uint32_t nb, uint32_t shift, uint32_t bins,
                uint32_t nblk, const uint32_t* __restrict__ binned, const uint32_t* __restrict__ place,
                uint32_t* __restrict__ binoff, typename PartRec<PACK>::T* __restrict__ rec) {
   __shared__ uint32_t cur[kPartBins];
   __shared__ uint64_t wsum[kPartBlock / kWave];
+  constexpr uint32_t M = kPartBins / kPartBlock;  // bins of a thread
   const uint32_t t = threadIdx.x;
-  const uint32_t c = t < bins ? binned[t] : 0u;
-  const uint32_t pl = t < bins ? place[(size_t)blockIdx.x * bins + t] : 0u;
-  uint64_t tot;
-  const uint32_t off = (uint32_t)part_scan(c, wsum, &tot);
-  if (t < bins) cur[t] = off + pl;
-  if (blockIdx.x == 0) {
-    if (t < bins) binoff[t] = off;
-    if (t == 0) binoff[bins] = (uint32_t)tot;
+  uint32_t c[M], pl[M], sum = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < M; ++j) {
+    const uint32_t b = M * t + j;
+    c[j] = b < bins ? binned[b] : 0u;
+    pl[j] = b < bins ? place[(size_t)blockIdx.x * bins + b] : 0u;
+    sum += c[j];
   }
+  uint64_t tot;
+  uint32_t off = (uint32_t)part_scan(sum, wsum, &tot);
+#pragma unroll
+  for (uint32_t j = 0; j < M; ++j) {
+    const uint32_t b = M * t + j;
+    cur[b] = off + pl[j];
+    if (blockIdx.x == 0 && b < bins) binoff[b] = off;
+    off += c[j];
+  }
+  if (blockIdx.x == 0 && t == 0) binoff[bins] = (uint32_t)tot;
   __syncthreads();
   size_t lo, hi;
   part_chunk(count, nblk, &lo, &hi);
   const uint32_t mask = (1u << nb) - 1, lmask = (1u << shift) - 1;
+  if constexpr (STAGED) {
+    using R = typename PartRec<PACK>::T;
+    extern __shared__ __align__(16) unsigned char smem[];
+    StageLds<R> stage(smem, wsum);
+    constexpr uint32_t P = StageLds<R>::kPer / 2;
+    for (size_t k0 = lo; k0 < hi; k0 += P * kPartBlock) {  // uniform over the workgroup
+      uint2 p[P];
+#pragma unroll
+      for (uint32_t j = 0; j < P; ++j) {
+        const size_t k = k0 + j * kPartBlock + t;
+        p[j] = k < hi ? pairs[k] : make_uint2(0xFFFFFFFFu, 0);
+      }
+      R r[2 * P];
+      uint32_t key[2 * P];
+#pragma unroll
+      for (uint32_t j = 0; j < P; ++j) {
+        const bool ok = p[j].x < n && p[j].y < n;
+        const uint32_t px = (p[j].x * kPlaceMul) & mask, py = (p[j].y * kPlaceMul) & mask;
+        r[2 * j] = PartRec<PACK>::make(px & lmask, p[j].y, nb);
+        r[2 * j + 1] = PartRec<PACK>::make(py & lmask, p[j].x, nb);
+        key[2 * j] = ok ? px >> shift : kPartBins;
+        key[2 * j + 1] = ok ? py >> shift : kPartBins;
+      }
+      stage.write(r, key, cur, rec);
+    }
+    return;
+  }
   part_walk(pairs, lo, hi, [&](uint2 p) {
     if (p.x >= n || p.y >= n) return;
     const uint32_t px = (p.x * kPlaceMul) & mask, py = (p.y * kPlaceMul) & mask;
@@ -2597,6 +2694,9 @@ void launch_sketch_update(int gbytes, const uint64_t* idx, size_t count, unsigne
 
 size_t group_partials_len(uint32_t n) { return (n + kScanSpan - 1) / kScanSpan + 1; }
 
+// Entries from which records move through LDS: with fewer than 1024 bins of 8192 entries, the open
+// lines fit the L2s, and the direct writes (12 us for 730k updates) take no sorting.
+constexpr size_t kStagedMin = size_t(1) << 23;
 // Bits of a vertex's place, and the log2 of a bin's vertices.
 struct PartShape {
   uint32_t nb, shift;
@@ -2606,7 +2706,7 @@ uint32_t part_bits(uint32_t n) {
   while (nb < 24 && (1u << nb) < n) ++nb;
   return nb;
 }
-// One-word records: 1024 bins of 2^(nb - 10) vertices leave nb - 10 bits of place beside nb bits of id.
+// One-word records: with at least 1024 bins, at most nb - 10 bits of place stand beside nb bits of id.
 bool part_packed(uint32_t n) { return part_bits(n) <= 21; }
 // About 8192 entries a bin (what a workgroup keeps in registers between its passes), at least 64 bins
 // and at most kPartBins, of at most 2^kPartMaxShift vertices (the LDS counters) and at least 8.
@@ -2644,16 +2744,20 @@ void launch_group(const uint32_t* pairs, size_t count, uint32_t n, uint32_t tile
     const size_t lds = size_t(4) << sh.shift;
     hipLaunchKernelGGL(k_part_hist, dim3(nblk), dim3(kPartBlock), 0, s, p2, count, n, sh.nb, sh.shift, bins, nblk,
                        b.binned, b.place, b.totals, b.bad);
-    auto go = [&](auto pack) {
-      constexpr bool PACK = decltype(pack)::value;
-      auto* rec = reinterpret_cast<typename PartRec<PACK>::T*>(b.rec);
-      hipLaunchKernelGGL(k_part_scatter<PACK>, dim3(nblk), dim3(kPartBlock), 0, s, p2, count, n, sh.nb, sh.shift, bins,
-                         nblk, b.binned, b.place, b.binoff, rec);
+    auto go = [&](auto pack, auto staged) {
+      constexpr bool PACK = decltype(pack)::value, STAGED = decltype(staged)::value;
+      using R = typename PartRec<PACK>::T;
+      R* rec = reinterpret_cast<R*>(b.rec);
+      hipLaunchKernelGGL((k_part_scatter<PACK, STAGED>), dim3(nblk), dim3(kPartBlock), STAGED ? StageLds<R>::bytes() : 0,
+                         s, p2, count, n, sh.nb, sh.shift, bins, nblk, b.binned, b.place, b.binoff, rec);
       hipLaunchKernelGGL(k_part_group<PACK>, dim3(bins), dim3(kPartBlock), lds, s, rec, sh.nb, sh.shift, b.binned,
                          b.binoff, b.totals, b.dst_arr, tile, b.tiles, acc, S, per_update);
     };
-    if (part_packed(n)) go(std::true_type{});
-    else go(std::false_type{});
+    const std::true_type yes{};
+    const std::false_type no{};
+    const bool large = 2 * count >= kStagedMin;
+    if (part_packed(n)) large ? go(yes, yes) : go(yes, no);
+    else large ? go(no, yes) : go(no, no);
     return;
   }
   launch_fill_u32(b.cnt, 0, n, s);
