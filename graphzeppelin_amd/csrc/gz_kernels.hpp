@@ -95,9 +95,9 @@ void launch_group(const uint32_t* pairs, size_t count, uint32_t n, uint32_t tile
 // src != pairs: the batch is copied from src into pairs by the same launch.
 // build_sf: the same launch first fills the forest membership set from d.sf_edge (the first
 // batch after a query).  hint: n rank classes (RoundBufs::hint); ranked: false while no query
-// has written them and the instance is new.
+// has written them and the instance is new.  map: scratch of (n + 63) / 64 words.
 void launch_eager(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged, const DsuDev& d,
-                  hipStream_t s, bool build_sf, unsigned char* hint, bool ranked);
+                  hipStream_t s, bool build_sf, unsigned char* hint, bool ranked, uint64_t* map);
 
 // ---- Borůvka ----
 struct RoundBufs;

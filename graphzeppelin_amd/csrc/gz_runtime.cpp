@@ -277,6 +277,7 @@ void GzAlg::place_buffers(Arena& dev, Arena& host) {
   while (cap < 2ull * n) cap <<= 1;
   sf_hash.place(dev, cap);
   sf_edge.place(dev, n);
+  dsu_map.place(dev, ((size_t)n + 63) / 64);
   flags.place(dev, kNumFlags);
   mod.place(dev, geo.samples + 2);
   labels.place(dev, n + 1);
@@ -1014,7 +1015,8 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
 
 void GzAlg::eager_batch(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged) {
   if (!count) return;
-  launch_eager(src, pairs, count, merged, dsu, st, sf_pending, rb.hint, unranked_seen >= 4ull * n);
+  launch_eager(src, pairs, count, merged, dsu, st, sf_pending, rb.hint, unranked_seen >= 4ull * n,
+               dsu_map.p);
   unranked_seen += count;  // builds the forest set when pending
   sf_pending = false;
 }

@@ -245,7 +245,7 @@ class GzAlg {
   DevBuf<uint64_t> col_bf;
   // DSU / forest
   DevBuf<uint32_t> parent, flags, labels, qa, qb;
-  DevBuf<uint64_t> sf_edge;
+  DevBuf<uint64_t> sf_edge, dsu_map;
   DevBuf<uint64_t> sf_hash;
   DevBuf<uint8_t> qout;
   DsuDev dsu{};
