@@ -205,31 +205,60 @@ constexpr uint32_t kNoLink = 0xFFFFFFFFu;
 // the hub's.  Returns the root that was linked under the other one, or kNoLink when a and b were
 // already connected.
 // LATE: the hints are loaded once the roots are known to differ (a batch whose edges are mostly
-// connected already); otherwise with the first parents (Borůvka's samples, which mostly link).
+// connected already); otherwise with the parents (Borůvka's samples, which mostly link).
+//
+// The first walk takes its parents through the caches: a stale parent is still an ancestor, so equal
+// roots are connected, and the CAS finds out whether the lower root is one still; a winner that was
+// linked meanwhile ranks higher all the same.  After a lost CAS the walk goes on from the parent the
+// CAS returned, with device-coherent loads.
+template <class T>
+__device__ inline T ld_cached(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
 template <bool LATE = false>
 __device__ inline uint32_t dsu_link(uint32_t* parent, uint32_t a, uint32_t b, uint32_t pseed,
                                     const unsigned char* hint) {
+  // both first parents (and hints) in one round trip; a root (the common case) needs no more
+  uint32_t pa = ld_cached(parent + a), pb = ld_cached(parent + b);
+  uint32_t ha = 0, hb = 0;
+  if (!LATE) {
+    ha = hint[a];
+    hb = hint[b];
+  }
+  // one step of both walks per round trip, splitting the paths
+  while (pa != a || pb != b) {
+    const uint32_t ga = pa != a ? ld_cached(parent + pa) : pa, gb = pb != b ? ld_cached(parent + pb) : pb;
+    if (!LATE && pa != a) ha = hint[pa];
+    if (!LATE && pb != b) hb = hint[pb];
+    if (pa != a && ga != pa) st_rlx(parent + a, ga);
+    if (pb != b && gb != pb) st_rlx(parent + b, gb);
+    a = pa;
+    pa = ga;
+    b = pb;
+    pb = gb;
+  }
   while (true) {
-    // both first parents (and hints) in one round trip; a root (the common case) needs no more
-    const uint32_t a_up = ld_acq(parent + a), b_up = ld_acq(parent + b);
-    uint32_t ha = 0, hb = 0;
-    if (!LATE) {
+    if (a == b) return kNoLink;
+    if (LATE) {
       ha = hint[a];
       hb = hint[b];
     }
-    const uint32_t ra = dsu_find_from(parent, a, a_up), rb = dsu_find_from(parent, b, b_up);
-    if (ra == rb) return kNoLink;
-    if (LATE || ra != a) ha = hint[ra];
-    if (LATE || rb != b) hb = hint[rb];
-    a = ra;
-    b = rb;
-    const uint32_t pa = dsu_prio(a, pseed), pb = dsu_prio(b, pseed);
-    const bool a_wins = ha != hb ? ha > hb : pa != pb ? pa > pb : a < b;
-    if (!a_wins) { uint32_t t = a; a = b; b = t; }
+    const uint32_t wa = dsu_prio(a, pseed), wb = dsu_prio(b, pseed);
+    const bool a_wins = ha != hb ? ha > hb : wa != wb ? wa > wb : a < b;
+    if (!a_wins) {
+      uint32_t t = a; a = b; b = t;
+      t = ha; ha = hb; hb = t;
+    }
     uint32_t expected = b;
     if (__hip_atomic_compare_exchange_strong(parent + b, &expected, a, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT))
       return b;
+    const uint32_t a_up = ld_acq(parent + a);
+    const uint32_t rb = dsu_find_from(parent, b, expected), ra = dsu_find_from(parent, a, a_up);
+    if (!LATE && rb != b) hb = hint[rb];
+    if (!LATE && ra != a) ha = hint[ra];
+    a = ra;
+    b = rb;
   }
 }
 
@@ -1374,11 +1403,10 @@ k_sample_round0(const unsigned char* __restrict__ slab, Geo g, uint64_t* __restr
   if (__ballot(hooked) && lane_id() == 0) d.mod[0] = 1;  // round 0 merged something
 }
 
-// The merges of a round (sample_supernode, src/cc_sketch_alg.cpp:137-166), one thread per
-// supernode: every vertex that was a root when the round began (root == nullptr: every vertex, as
-// in round 0) acts on its sample record.  The round is modified by a FAIL or a merge.  Links rank
-// roots by the degree class round 0 recorded (hint), so hubs stay roots and absorb their
-// neighbours without contention.
+// The merge of a supernode's sample (sample_supernode, src/cc_sketch_alg.cpp:137-166): round 0's in
+// k_apply_samples, one thread per vertex, the later rounds' where the sample is taken (k_bv_reduce,
+// k_bv_finish).  The round is modified by a FAIL or a merge.  Links rank roots by the degree class
+// round 0 recorded (hint), so hubs stay roots and absorb their neighbours without contention.
 constexpr uint32_t kNoRoot = 0xFFFFFFFFu;  // no supernode (unused partial slot, no giant)
 
 // Round state words (RoundBufs::totals).  A query starts with kStGiantFirst = kNoRoot.
@@ -1461,29 +1489,16 @@ __device__ inline bool apply_sample(const DsuDev& d, uint64_t s, const unsigned 
   return true;
 }
 
-// st == nullptr (round 0): every vertex is a root.  Otherwise the round's supernodes: its segment
-// list (every root outside the giant) and the giant's root.
+// The merges of round 0 that k_sample_round0 left in samp.  Nothing to do when the query keeps the
+// eager DSU; else the DSU restarts valid.
 __global__ void __launch_bounds__(256)
-k_apply_samples(const uint64_t* __restrict__ samp, const RoundSeg* __restrict__ segs, DsuDev d,
-                const uint32_t* __restrict__ st, uint32_t round, const uint32_t* __restrict__ prev_mod,
-                uint32_t* __restrict__ cur_mod, const unsigned char* __restrict__ hint) {
-  uint32_t live = prev_mod ? ld_acq(prev_mod) : 1u;  // checked after the first reads
-  if (!st) {  // round 0: nothing to do when the query keeps the eager DSU; else the DSU restarts valid
-    if (ld_acq(d.flags + kFlagSkip)) live = 0;
-    else if (blockIdx.x == 0 && threadIdx.x == 0) d.flags[kFlagEagerInvalid] = 0;
-  }
-  const bool act = st && st[kStActMode] != 0;
-  const uint32_t gr = act ? st[kStGiantRound] : kNoRoot;
-  const uint32_t count = st ? st[kStSeg + 2 * (round & 1) + 1] : d.n;
-  if (!live) return;
+k_apply_samples(const uint64_t* __restrict__ samp, DsuDev d, const unsigned char* __restrict__ hint) {
+  if (ld_acq(d.flags + kFlagSkip)) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) d.flags[kFlagEagerInvalid] = 0;
   bool modified = false;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-    const uint32_t v = st ? segs[i].root : i;
-    if (v == gr) continue;  // handled once below
+  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < d.n; v += gridDim.x * blockDim.x)
     if (apply_sample(d, samp[v], hint)) modified = true;
-  }
-  if (gr != kNoRoot && blockIdx.x == 0 && threadIdx.x == 0 && apply_sample(d, samp[gr], hint)) modified = true;
-  if (__syncthreads_or(modified) && threadIdx.x == 0) *cur_mod = 1;  // one plain store per block
+  if (__syncthreads_or(modified) && threadIdx.x == 0) d.mod[0] = 1;  // one plain store per block
 }
 
 // ---- rounds >= 1 (perform_boruvka_round 246-380 + create_merge_instructions 382-462) ----------
@@ -1821,8 +1836,7 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
 // Segmented XOR-reduce + sample (range_merge of column `round` + the deterministic bucket over
 // every member of a supernode, then sample_supernode).  Entries are the member list, grouped by
 // root.  A wave takes 64 consecutive entries (reduce_members).  A supernode whose entries all lie
-// inside the range is sampled from registers; its sample record goes to samp[root] for
-// k_apply_samples.  A supernode that crosses the range's first (head) or last (tail) boundary leaves
+// inside the range is sampled from registers; its sample record goes to samp[root].  A supernode that crosses the range's first (head) or last (tail) boundary leaves
 // its partial XOR in the range's head or tail slot under its root; a slot left unused gets root
 // kNoRoot and a zero value.
 //
@@ -1830,6 +1844,13 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
 // which a crossing supernode starts adds up that supernode's slots, so at most two supernodes of a
 // workgroup are unfinished: the one continuing from the previous workgroup and the one continuing
 // into the next.
+//
+// The round's merges are made here too: a wave keeps the samples of its supernodes one to a lane and
+// links them all at once at its end (no kernel of the round reads the parents beside this one).  Taken
+// in the loop that samples them, one by one, the links cost three times the launch that they spare;
+// before the workgroup's barrier, 2 us a round more than after it.  Against a launch of their own
+// (5 to 11 us a round), a query over 32k vertices in 64 components went from 579 to 537 us with its
+// updates, a point query on 2^18 vertices from 600 to 570 us; full rounds of 2^18 gain nothing.
 //
 // A full round over 2^18 members reads three lines per member (122 MB) and is bound by them: a
 // workgroup's records arrive over 7..20 us of its 28 and the sampling runs behind.  Before the rows of
@@ -1901,7 +1922,8 @@ __device__ inline uint64_t low_bits(uint32_t k) { return k >= 64 ? ~0ull : (1ull
 // same root in the tail slot, so the supernode's entries stay contiguous in the next reduce.  A slot
 // left unused gets root kNoRoot and a zero value.  s_tot, if given, gets the XOR of every entry.  With
 // s_bnd, the wave holding the workgroup's first entry [blk_b0] loads that entry's segment bounds into
-// s_bnd[0..1], the one holding its last entry the end of that entry's segment into s_bnd[2].
+// s_bnd[0..1], the one holding its last entry the end of that entry's segment into s_bnd[2].  pend, if
+// given, gets in each lane the sample record of the run that begins at the lane's entry, or ZERO.
 constexpr uint32_t kRow = 16, kRowDet = kRow - 1;  // lanes of a row; the lane of the deterministic bucket
 typedef uint32_t Words __attribute__((ext_vector_type(16)));  // one word of a row's 16 entries per lane
 template <class G>
@@ -1910,7 +1932,8 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
                                       const unsigned char* __restrict__ slab, const Geo& g, uint32_t round, Slot head,
                                       Slot tail, uint64_t* __restrict__ samp, uint32_t* __restrict__ flags,
                                       const unsigned char* __restrict__ det_cpy, bool deep_on, uint64_t* s_tot,
-                                      const XAcc* xa, uint32_t blk_b0, uint32_t blk_b1, uint32_t* s_bnd) {
+                                      const XAcc* xa, uint32_t blk_b0, uint32_t blk_b1, uint32_t* s_bnd,
+                                      uint64_t* pend = nullptr) {
   constexpr uint32_t RB = 8 + sizeof(G);
   const uint32_t lane = lane_id(), i = lane % kRow, base = lane - i, row = lane / kRow;
   // lane base + k holds entry k of its row
@@ -1960,6 +1983,14 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
   if (kDeepFlags<G> && deep_on && mine)
     flag = *reinterpret_cast<const uint32_t*>(slab + (size_t)m * g.row + deep_flag_off(round));
 
+  // The sample record of the run whose first entry is lane l's, besides samp[], at recs[l] (in the
+  // head slot, which is written last).
+  uint64_t* recs = pend ? head.vals : nullptr;
+  if (recs) recs[lane] = kSampZero;
+  auto leave = [&](uint32_t R, uint32_t first, uint64_t rec) {
+    samp[R] = rec;
+    if (recs) recs[first] = rec;
+  };
   uint64_t again = 0;  // first lanes of the runs inside the wave whose sample is left to the deep records
   // Sample the runs of the rows with `done` set (the same in all lanes of a row); first: the run's first lane.
   auto emit = [&](bool done, uint64_t a, G gm, uint32_t R, uint32_t first) {
@@ -1973,10 +2004,10 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
     if (done) {
       if (i == kRowDet) {
         if (zero) samp[R] = kSampZero;
-        else if (det) samp[R] = sample_record(kGood, a, g.n, flags);
+        else if (det) leave(R, first, sample_record(kGood, a, g.n, flags));
         else left = col == 0;
       } else if (!zero && !det && col && i == (uint32_t)__builtin_ctz(col)) {
-        samp[R] = sample_record(kGood, a, g.n, flags);
+        leave(R, first, sample_record(kGood, a, g.n, flags));
       }
     }
     for (uint64_t b = __ballot(left); b; b &= b - 1) again |= 1ull << rd_lane_u32(first, __builtin_ctzll(b));
@@ -2092,7 +2123,14 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
         __ballot(lane >= kRowDet && lane < g.D && (G)xxh3_mix(xxh3_prep(a), g.chk_bf) == gm);
     const uint32_t R = rd_lane_u32(rt, (int)f);
     if (good ? lane == (uint32_t)__builtin_ctzll(good) : lane == 0)
-      samp[R] = sample_record(good ? kGood : kFail, a, g.n, flags);
+      leave(R, f, sample_record(good ? kGood : kFail, a, g.n, flags));
+  }
+  if (recs) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    *pend = recs[lane];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
 
   // Every lane stores the root (the same value), so every lane of this wave may read it back
@@ -2157,9 +2195,10 @@ template <class G>
 __global__ void __launch_bounds__(kRedBlock)
 k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ members,
             const uint32_t* __restrict__ mroot, const unsigned char* __restrict__ slab, Geo g, uint32_t round,
-            XAcc xa, uint64_t* __restrict__ samp, uint32_t* __restrict__ flags,
-            const uint32_t* __restrict__ prev_mod, uint32_t* __restrict__ rstats,
-            const unsigned char* __restrict__ det_cpy, uint32_t small_walk, uint32_t deep_skip) {
+            XAcc xa, uint64_t* __restrict__ samp, DsuDev d,
+            const uint32_t* __restrict__ prev_mod, uint32_t* __restrict__ cur_mod, uint32_t* __restrict__ rstats,
+            const unsigned char* __restrict__ det_cpy, const unsigned char* __restrict__ hint, uint32_t small_walk,
+            uint32_t deep_skip) {
   const uint32_t live = ld_acq(prev_mod);  // checked after the first reads
   GZ_REDUCE_LDS
   const uint32_t giant = st[kStGiantRound];
@@ -2193,10 +2232,11 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
   const uint32_t p0 = b0 + wid * W;
   Slot hs{s_vals + (size_t)(2 * wid) * 2 * kWave, s_root + 2 * wid};
   Slot ts{s_vals + (size_t)(2 * wid + 1) * 2 * kWave, s_root + 2 * wid + 1};
+  uint64_t pend = kSampZero;  // lane l: the sample record of a supernode still to be merged
   if (p0 < b1) {
     const uint32_t len = b1 - p0 < W ? b1 - p0 : W;
-    reduce_members<G>(p0, len, W / 4, e1, members, mroot, slab, g, round, hs, ts, samp, flags, det_cpy, deep_skip != 0,
-                      giant_tot ? s_tot : nullptr, &xa, b0, b1, s_bnd);
+    reduce_members<G>(p0, len, W / 4, e1, members, mroot, slab, g, round, hs, ts, samp, d.flags, det_cpy,
+                      deep_skip != 0, giant_tot ? s_tot : nullptr, &xa, b0, b1, s_bnd, &pend);
   } else {
     hs.vals[lane] = 0;
     hs.vals[kWave + lane] = 0;
@@ -2225,10 +2265,15 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
     }
     return open >= nw;
   };
+  bool modified = false;
   auto sample_to = [&](uint32_t R, uint64_t a, uint64_t gm) {
     uint64_t idx;
     const int code = wave_sample<G>(a, (G)gm, g.D, g.chk_bf, &idx);
-    if (lane == 0) samp[R] = sample_record(code, idx, g.n, flags);
+    const uint64_t rec = sample_record(code, idx, g.n, d.flags);
+    if (lane == 0) samp[R] = rec;
+    const uint64_t idle = __ballot(pend == kSampZero);
+    if (!idle) modified |= lane == 0 && apply_sample(d, rec, hint);
+    else if (lane == (uint32_t)__builtin_ctzll(idle)) pend = rec;
   };
   // one of the `parts` workgroups that hold R adds its part to accumulator slot `slot`; the last one
   // samples the sum and clears the slot for the next round
@@ -2267,13 +2312,15 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
     if (nblk == 1) sample_to(giant, s_tot[lane], s_tot[kWave + lane]);  // the giant's whole sum
     else cross(xa.nslots - 1, nblk, giant, s_tot[lane], s_tot[kWave + lane]);
   }
+  if (apply_sample(d, pend, hint)) modified = true;
+  if (__ballot(modified) && lane == 0) *cur_mod = 1;  // one plain store per wave
 }
 
 // ---- the last rounds in one workgroup ----------------------------------------------------------
 // Once a giant supernode exists, a round walks only the vertices outside it that are not in a finished
 // component, and after a few rounds they are few; a small graph's are few from the start.  k_bv_finish then runs every remaining round inside one workgroup -- the same
-// regrouping, reduce, sample and merge as k_bv_find_count .. k_apply_samples, with barriers between
-// the steps instead of kernel boundaries -- so a round costs a few round trips instead of five
+// regrouping, reduce, sample and merge as k_bv_find_count .. k_bv_reduce, with barriers between
+// the steps instead of kernel boundaries -- so a round costs a few round trips instead of four
 // dependent launches.  It takes over at round r0 only when round r0 - 1 changed something and the walk
 // holds at most kFinishMax vertices; otherwise it returns without touching any state and the rounds
 // continue as launches.  A giant is elected in it as in the launched rounds, so both regroup the same
@@ -2483,7 +2530,7 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     // which a workgroup barrier alone does not order after those stores.
     __threadfence();
     __syncthreads();
-    // merges (k_apply_samples): every supernode root of the walk, and the giant
+    // merges: every supernode root of the walk, and the giant
     bool modified = false;
     for (uint32_t k = tid; k < kFinishTable; k += kRedBlock)
       if (s_key[k] != kEmptyKey && apply_sample(d, ld_acq(samp + s_key[k]), hint)) modified = true;
@@ -2881,8 +2928,7 @@ void launch_sample_round0(int gbytes, const unsigned char* slab, const Geo& g, c
   else
     hipLaunchKernelGGL(k_sample_round0<uint64_t>, dim3(grid), dim3(256), 0, s, slab, g, samp, d.flags, rb.det_cpy,
                        rb.hint, d);
-  hipLaunchKernelGGL(k_apply_samples, dim3(grid_for(g.n, 256, 4096)), dim3(256), 0, s, samp, nullptr, d, nullptr, 0u,
-                     nullptr, d.mod, rb.hint);
+  hipLaunchKernelGGL(k_apply_samples, dim3(grid_for(g.n, 256, 4096)), dim3(256), 0, s, samp, d, rb.hint);
 }
 
 // Host bound on each level's entry count (the kernels compute the exact counts on the device):
@@ -2922,14 +2968,12 @@ void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const G
   const XAcc xa{rb.xacc, rb.xcnt, rb.xslots, rb.off, rb.cursor};
   if (gbytes == 4)
     hipLaunchKernelGGL(k_bv_reduce<uint32_t>, dim3(rgrid), dim3(kRedBlock), 0, s, st, members, rb.mroot[par],
-                       slab, g, round, xa, rb.samp, d.flags, prev, rb.rstats, rb.det_cpy, n / kSmallWalkDiv,
+                       slab, g, round, xa, rb.samp, d, prev, cur, rb.rstats, rb.det_cpy, rb.hint, n / kSmallWalkDiv,
                        deep_skip ? 1u : 0u);
   else
     hipLaunchKernelGGL(k_bv_reduce<uint64_t>, dim3(rgrid), dim3(kRedBlock), 0, s, st, members, rb.mroot[par],
-                       slab, g, round, xa, rb.samp, d.flags, prev, rb.rstats, rb.det_cpy, n / kSmallWalkDiv,
+                       slab, g, round, xa, rb.samp, d, prev, cur, rb.rstats, rb.det_cpy, rb.hint, n / kSmallWalkDiv,
                        deep_skip ? 1u : 0u);
-  hipLaunchKernelGGL(k_apply_samples, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, rb.samp, rb.segs[par], d, st,
-                     round, prev, cur, rb.hint);
 }
 
 bool launch_finish(int gbytes, uint32_t r0, uint32_t last_round, const unsigned char* slab, const Geo& g,
