@@ -367,25 +367,59 @@ __global__ void k_fill_u64(uint64_t* p, uint64_t v, size_t n) {
 // One wave (a 64-thread workgroup) per tile of <= tile-size destinations of one vertex, so a CU
 // keeps up to 32 tiles in flight: most tiles of a flush hold a handful of updates, and a tile's
 // time is the latency of its few dependent memory round trips, not bandwidth.  Lanes take
-// (update, column) pairs; the tile's delta for depths 0..kLdsDepth-1 of every column lives in LDS
-// (column pitch kLdsPitch = 9, odd, so lanes on consecutive columns hit different banks), and the
-// rare deeper contributions (one pair in 2^kLdsDepth) are XORed straight into the vertex's records
+// (update, column) pairs; the tile's delta for the lower depths of every column lives in LDS
+// (lds_depth), and the rare deeper contributions are XORed straight into the vertex's records
 // with device-scope atomics (setting the column's deep flag when the record lies past the first
 // line of the column's overflow run).  The deterministic bucket is kept in registers and reduced
 // once per tile.
 // Long tiles are bound by VALU issue (a pair's hash is two 64-bit products, six quarter-rate
 // multiplies of about 50 instructions before), so everything of the hash that is linear is taken out
 // of the pairs: an update's index and a column's bitflip are spread once (xxh3_spread) and a pair
-// XORs them; the depth is read from the hash's low word, the exact one only where it leaves the LDS
-// delta; indices are rebuilt from the other end, so the pair still costs one 16-byte LDS read.  24M
-// Chung-Lu updates on 2^18 vertices 2153 -> 1653 us (216 SIMD cycles per 64 pairs), 16M R-MAT on 2^20
-// 2189 -> 1627 us, flushes of a serving trace (about 6 updates per vertex, bound by the tiles' memory
-// round trips) 206 -> 199 us.  The write-back is a read-xor-write of the touched records, or device-scope
+// XORs them; the depth is read from the hash's low word, whose second product then needs two 24-bit
+// multiplies instead of two of the quarter-rate ones (hash_low28), and a pair's two LDS addresses come
+// from one multiply-add; indices are rebuilt from the other end, so the pair still costs one 16-byte LDS
+// read.  24M Chung-Lu updates on 2^18 vertices 2153 -> 1290 us in all (hash_low28 and the addresses 1530
+// -> 1415), 16M R-MAT on 2^20 2189 -> 1550 us, flushes of a serving trace (about 6 updates per vertex,
+// bound by the tiles' memory round trips) 206 -> 193 us.  The write-back is a read-xor-write of the touched records, or device-scope
 // atomic XOR when the vertex is split across tiles of the same launch.  Workgroups walk the tiles
 // grid-stride (no shared counter), so a persistent grid can cover a tile count that only the
 // device knows.
 // ================================================================================================
-constexpr uint32_t kLdsDepth = 9, kLdsPitch = 9;  // depths 0..8 per column; 9 is odd
+// Entries of the LDS delta that a lane writes back in one pass, and the depths of a column held there.
+// With 4-byte checksums as many as one pass takes, 9 (28 columns, a deep pair in 512) to 14 (18 columns),
+// and a CU still has LDS for its 32 tiles: 24M Chung-Lu updates on 2^18 vertices (25 columns, 10 depths
+// against 9) 1415 -> 1290 us.  With 8-byte checksums the larger delta would take tiles from a CU, which
+// costs flushes of a few updates per vertex 3% (dense ones would gain 8%), and where a pass does not hold
+// 9 depths there are several.  Deep records that need a flag begin at depth 15.
+constexpr uint32_t kPerLane = 4, kLdsDepthMin = 9, kLdsDepthMax = 14;
+uint32_t lds_depth(uint32_t C, int gbytes) {
+  const uint32_t d = gbytes == 4 ? (kPerLane * kWave - 1) / C : 0;
+  return d < kLdsDepthMin ? kLdsDepthMin : d > kLdsDepthMax ? kLdsDepthMax : d;
+}
+// (a mod 2^24) * (b mod 2^24) + c; from plain C the compiler takes the quarter-rate 32-bit multiply.
+__device__ inline uint32_t mad24(uint32_t a, uint32_t b, uint32_t c) {
+  uint32_t r;
+  asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "Is"(b), "v"(c));
+  return r;
+}
+// Low word of the hash of x, a spread index ^ bitflip (xxh3_products and the last step), exact in its low
+// 28 bits.  They need the second product only up to bit 55, so its cross terms are taken modulo 2^24:
+// full-rate 24-bit multiplies instead of quarter-rate 32-bit ones.
+__device__ inline uint32_t hash_low28(uint64_t x) {
+  x *= kPrimeMx2;
+  const uint32_t hi = (uint32_t)(x >> 32), lo = (uint32_t)x ^ ((hi >> 3) + 8);
+  const uint64_t p = (uint64_t)lo * (uint32_t)kPrimeMx2;
+  uint32_t ph = mad24(lo, (uint32_t)(kPrimeMx2 >> 32), (uint32_t)(p >> 32));
+  ph = mad24(hi, (uint32_t)kPrimeMx2, ph);
+  return (uint32_t)p ^ __builtin_amdgcn_alignbit(ph, (uint32_t)p, 28);
+}
+// Depth of a bucket from x, the spread index ^ bitflip, and low, hash_low28 of it; at least D: no bucket.
+__device__ inline uint32_t bucket_depth(uint32_t low, uint64_t x, uint64_t depth_cap) {
+  low &= (1u << 28) - 1;
+  if (low) return (uint32_t)__builtin_ctz(low);
+  const uint64_t h = xxh3_products(x);
+  return (uint32_t)__builtin_ctzll((h ^ (h >> 28)) | depth_cap);
+}
 // Updates of a chunk from which each lane takes its own one: C steps against m * C / 64 longer ones.
 // 24M Chung-Lu updates on 2^18 vertices 1667 -> 1567 us, 3M R-MAT on 2^17 with 8-byte checksums 343 ->
 // 307 us, a serving trace's flushes 192 -> 189 us.
@@ -400,10 +434,10 @@ template <class G, bool WIDE>
 __global__ void __launch_bounds__(kWave, 8)  // 8 waves per SIMD: 32 tiles in flight per CU
 k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntiles_dev, uint32_t ntiles_host,
                const uint32_t* __restrict__ dsts, unsigned char* __restrict__ slab, Geo g,
-               const uint64_t* __restrict__ col_bf) {
+               const uint64_t* __restrict__ col_bf, uint32_t ldepth, uint32_t ldepth_inv) {
   extern __shared__ __align__(16) unsigned char smem[];
   const uint32_t C = g.C, D = g.D;
-  const uint32_t det_slot = C * kLdsPitch;
+  const uint32_t det_slot = C * ldepth;
   const uint32_t lds_n = det_slot + 1;
   // per chunk, read by the lanes that take an update's columns: its spread index, and the other end
   // and the checksum (kTight: one 16-byte slot), or the index with the checksum in an array of its own
@@ -419,18 +453,17 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
   for (uint32_t i = lane; i < C; i += kWave) s_bf[i] = xxh3_spread(col_bf[i]);
   const uint64_t chk_sbf = xxh3_spread(g.chk_bf);
   // The delta is zeroed once here; afterwards the write-back clears every entry it reads.  Entries
-  // at depth >= D (or at a pitch padding, if the pitch exceeds kLdsDepth) are never written:
-  // offset 0.
+  // at depth >= D are never written: offset 0.
   for (uint32_t i = lane; i < lds_n; i += kWave) {
     s_a[i] = 0;
     s_g[i] = 0;
-    const uint32_t cc = i / kLdsPitch, d = i - cc * kLdsPitch;
+    const uint32_t cc = (i * ldepth_inv) >> 16, d = i - cc * ldepth;  // i / ldepth
     s_bo[i] =
-        (uint16_t)((i == det_slot ? det_col_off(g) : (d < kLdsDepth && d < D ? rec_col_off<G>(g, cc, d) : 0u)) / 4);
+        (uint16_t)((i == det_slot ? det_col_off(g) : (d < D ? rec_col_off<G>(g, cc, d) : 0u)) / 4);
   }
   const uint32_t ntiles = ntiles_dev ? *ntiles_dev : ntiles_host;
   const uint64_t depth_cap = 1ull << D;
-  const uint32_t lds_d = D < kLdsDepth ? D : kLdsDepth;
+  const uint32_t lds_d = D < ldepth ? D : ldepth, near_cap = 1u << ldepth;
   // pair p = i * C + c: lane starts at pair `lane` and advances 64 pairs (di updates, dc columns)
   const uint32_t i0 = lane / C, c0 = lane % C;
   const uint32_t di = kWave / C, dc = kWave % C;
@@ -473,16 +506,16 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
     for (uint32_t u0 = 0; u0 < tl.count; u0 += kWave) {
       const uint32_t m = tl.count - u0 < kWave ? tl.count - u0 : kWave;
       if (u0 != 0) hash_chunk(tl, u0, lane < m ? dsts[tl.begin + u0 + lane] : 0);
-      // one column's bucket of one update; the depth from the hash's low word, whose bits decide every
-      // depth below kLdsDepth
-      auto add = [&](uint64_t h, uint32_t c, uint32_t c9, uint64_t idx, G chk) {
-        const uint32_t low = (uint32_t)h ^ __builtin_amdgcn_alignbit((uint32_t)(h >> 32), (uint32_t)h, 28);
-        const uint32_t near = (uint32_t)__builtin_ctz(low | (1u << kLdsDepth));
+      // one column's bucket of one update
+      auto add = [&](uint64_t x, uint32_t c, uint64_t idx, G chk) {
+        const uint32_t low = hash_low28(x);
+        const uint32_t near = (uint32_t)__builtin_ctz(low | near_cap);
         if (near < lds_d) {
-          lds_xor(s_a + c9 + near, idx);
-          lds_xor(s_g + c9 + near, chk);
+          const uint32_t e = mad24(c, ldepth, near);  // one full-rate step, and one for either address
+          lds_xor(s_a + e, idx);
+          lds_xor(s_g + e, chk);
         } else {
-          const uint32_t depth = (uint32_t)__builtin_ctzll((h ^ (h >> 28)) | depth_cap);  // == D: no bucket
+          const uint32_t depth = bucket_depth(low, x, depth_cap);
           if (depth < D) {
             xor_rec_atomic<G>(row + rec_col_off<G>(g, c, depth), idx, chk);
             if (kDeepFlags<G> && rec_is_deep(g, depth))  // the flag only ever goes from 0 to 1
@@ -497,12 +530,11 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
           const ulonglong2 pc = s_pc[lane];
           const G chk = kTight ? (G)(pc.y >> 32) : s_ck[lane];
           const uint64_t idx = kTight ? concat_pairing(tl.vertex, (uint32_t)pc.y) : pc.y;
-          uint32_t c = c0, c9 = c0 * kLdsPitch;
+          uint32_t c = c0;
           for (uint32_t k = 0; k < C; ++k) {
-            add(xxh3_products(pc.x ^ s_bf[c]), c, c9, idx, chk);
+            add(pc.x ^ s_bf[c], c, idx, chk);
             ++c;
-            c9 += kLdsPitch;
-            if (c == C) c = c9 = 0;
+            c = c < c - C ? c : c - C;  // C - C, or c - C below zero
           }
         }
         continue;
@@ -513,13 +545,10 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
       for (uint32_t it = 0; it < iters; ++it) {
         if (it * kWave + lane < np) {  // q < m here
           const ulonglong2 pc = s_pc[q];
-          const uint64_t h = xxh3_products(pc.x ^ s_bf[c]);
+          const uint64_t x = pc.x ^ s_bf[c];
           const G chk = kTight ? (G)(pc.y >> 32) : s_ck[q];
           const uint64_t idx = kTight ? concat_pairing(tl.vertex, (uint32_t)pc.y) : pc.y;
-          uint32_t c9;  // c * kLdsPitch: the compiler's choice is a quarter-rate multiply
-          asm("v_lshl_add_u32 %0, %1, 3, %1" : "=v"(c9) : "v"(c));
-          static_assert(kLdsPitch == 9, "c9");
-          add(h, c, c9, idx, chk);
+          add(x, c, idx, chk);
         }
         q += di;
         c += dc;
@@ -554,11 +583,11 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
 
     // write-back: read-xor-write of the touched records, four LDS entries per lane in flight
     auto write_back = [&](uint32_t e0, bool first) {
-      uint64_t da[4], ga[4];
-      G dg[4], gg[4];
-      uint32_t bo[4];
+      uint64_t da[kPerLane], ga[kPerLane];
+      G dg[kPerLane], gg[kPerLane];
+      uint32_t bo[kPerLane];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (uint32_t k = 0; k < kPerLane; ++k) {
         const uint32_t e = e0 + k * kWave + lane;
         da[k] = 0;
         dg[k] = 0;
@@ -575,7 +604,7 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
       }
       if (!tl.split) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (uint32_t k = 0; k < kPerLane; ++k)
           if ((da[k] | (uint64_t)dg[k]) != 0) ld_rec<G>(row + bo[k], &ga[k], &gg[k]);
       }
       // The next tile's first chunk, hashed while this tile's record loads are in flight.  The
@@ -590,16 +619,16 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
       }
       if (tl.split) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (uint32_t k = 0; k < kPerLane; ++k)
           if ((da[k] | (uint64_t)dg[k]) != 0) xor_rec_atomic<G>(row + bo[k], da[k], dg[k]);
       } else {
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (uint32_t k = 0; k < kPerLane; ++k)
           if ((da[k] | (uint64_t)dg[k]) != 0) st_rec<G>(row + bo[k], ga[k] ^ da[k], (G)(gg[k] ^ dg[k]));
       }
     };
     write_back(0, true);  // the delta holds at least the deterministic bucket's entry
-    for (uint32_t e0 = 4 * kWave; WIDE && e0 < lds_n; e0 += 4 * kWave) {
+    for (uint32_t e0 = kPerLane * kWave; WIDE && e0 < lds_n; e0 += kPerLane * kWave) {
       write_back(e0, false);
       __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // none of these passes' loads stays pending into the next tile
     }
@@ -615,7 +644,7 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
 // workgroup where the tiles of 1024 indices, each with its own delta, took one per tile on 2700
 // words and one per deep pair.  A lane keeps its index and takes the columns one after the other from
 // a column of its own on, which spreads a step's 64 lanes over the columns.  VALU-bound like the long
-// tiles of k_update_tiles: 4.19M indices of 25 columns 446 -> 126 us.
+// tiles of k_update_tiles: 4.19M indices of 25 columns 446 -> 113 us.
 constexpr uint32_t kOneBlock = 1024, kOneGrid = 512;
 constexpr uint32_t kOneDepth = 17, kOneMaxCols = 160;  // deltas of kOneDepth records up to this many columns
 template <class G>
@@ -645,24 +674,24 @@ k_sketch_update(const uint64_t* __restrict__ idxs, size_t count, unsigned char* 
     const G chk = (G)ck;
     det_a ^= idx;
     det_g ^= chk;
-    uint32_t c = lane_id() % C, at = c * depth;
+    uint32_t c = lane_id() % C;
     for (uint32_t k = 0; k < C; ++k) {
-      const uint64_t h = xxh3_products(sp ^ s_bf[c]);
-      const uint32_t low = (uint32_t)h ^ __builtin_amdgcn_alignbit((uint32_t)(h >> 32), (uint32_t)h, 28);
+      const uint64_t x = sp ^ s_bf[c];
+      const uint32_t low = hash_low28(x);
       const uint32_t near = (uint32_t)__builtin_ctz(low | near_cap);
       if (near < lds_d) {
-        lds_xor(s_a + at + near, idx);
-        lds_xor(s_g + at + near, chk);
+        const uint32_t e = mad24(c, depth, near);
+        lds_xor(s_a + e, idx);
+        lds_xor(s_g + e, chk);
       } else {
-        const uint32_t d = (uint32_t)__builtin_ctzll((h ^ (h >> 28)) | depth_cap);  // == D: no bucket
+        const uint32_t d = bucket_depth(low, x, depth_cap);
         if (d < D) {
           xor_rec_atomic<G>(slab + rec_col_off<G>(g, c, d), idx, chk);
           if (kDeepFlags<G> && rec_is_deep(g, d)) st_rlx(reinterpret_cast<uint32_t*>(slab + deep_flag_off(c)), 1u);
         }
       }
       ++c;
-      at += depth;
-      if (c == C) c = at = 0;
+      c = c < c - C ? c : c - C;  // C - C, or c - C below zero
     }
   }
   // lanes past the end hold zeros, and every lane is active again
@@ -2784,7 +2813,7 @@ void launch_fill_u64(uint64_t* p, uint64_t v, size_t n, hipStream_t s) {
 }
 
 size_t update_tiles_lds_bytes(const Geo& g, int gbytes) {
-  const size_t lds_n = (size_t)g.C * kLdsPitch + 1;
+  const size_t lds_n = (size_t)g.C * lds_depth(g.C, gbytes) + 1;
   return kWave * 16 + g.C * 8 + lds_n * 8 + (lds_n + kWave) * (size_t)gbytes + lds_n * 2;
 }
 
@@ -2796,9 +2825,11 @@ void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_d
   uint32_t grid = ntiles_dev ? grid_cap : (grid_cap && ntiles_host > grid_cap ? grid_cap : ntiles_host);
   if (grid == 0) return;
   const size_t lds = update_tiles_lds_bytes(g, gbytes);
-  const bool wide = g.C * kLdsPitch + 1 > 4 * kWave;
+  const uint32_t ldepth = lds_depth(g.C, gbytes);
+  const bool wide = g.C * ldepth + 1 > kPerLane * kWave;
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kWave), lds, s, tiles, ntiles_dev, ntiles_host, dsts, slab, g, col_bf);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kWave), lds, s, tiles, ntiles_dev, ntiles_host, dsts, slab, g, col_bf,
+                       ldepth, 65536 / ldepth + 1);
   };
   if (gbytes == 4) wide ? go(k_update_tiles<uint32_t, true>) : go(k_update_tiles<uint32_t, false>);
   else wide ? go(k_update_tiles<uint64_t, true>) : go(k_update_tiles<uint64_t, false>);
@@ -2807,7 +2838,7 @@ void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_d
 void launch_sketch_update(int gbytes, const uint64_t* idx, size_t count, unsigned char* slab, const Geo& g,
                           const uint64_t* col_bf, hipStream_t s) {
   if (!count) return;
-  const uint32_t depth = g.C <= kOneMaxCols ? kOneDepth : kLdsDepth;
+  const uint32_t depth = g.C <= kOneMaxCols ? kOneDepth : kLdsDepthMin;
   const uint32_t block = (uint32_t)std::min<size_t>(kOneBlock, (count + kWave - 1) / kWave * kWave);
   const uint32_t grid = (uint32_t)std::min<size_t>(kOneGrid, (count + block - 1) / block);
   const size_t lds = g.C * size_t(8) + ((size_t)g.C * depth + 1) * (8 + gbytes);
