@@ -2033,34 +2033,25 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
   if (kDeepFlags<G> && deep_on && mine)
     flag = *reinterpret_cast<const uint32_t*>(slab + (size_t)m * g.row + deep_flag_off(round));
 
-  // The sample record of the run whose first entry is lane l's, besides samp[], at recs[l] (in the
-  // head slot, which is written last).
-  uint64_t* recs = pend ? head.vals : nullptr;
-  if (recs) recs[lane] = kSampZero;
-  auto leave = [&](uint32_t R, uint32_t first, uint64_t rec) {
-    samp[R] = rec;
-    if (recs) recs[first] = rec;
-  };
-  uint64_t again = 0;  // first lanes of the runs inside the wave whose sample is left to the deep records
+  // What was sampled of the run whose first entry is lane l's, at recs[l] (in the head slot, which is
+  // written last): its index or one of these.  The runs leave no more than that here; their records are
+  // written by one step for the wave, each by its first lane.
+  constexpr uint64_t kRecBad = kSampFail - 1, kRecLeft = kSampFail - 2, kRecNone = kSampFail - 3;
+  uint64_t* recs = head.vals;
+  recs[lane] = kRecNone;
+  // lanes that go before this one where several buckets of a run are good: the deterministic bucket, then
+  // the lower depths
+  const uint32_t before_me = i == kRowDet ? 0u : (1u << kRowDet) | ((1u << i) - 1);
   // Sample the runs of the rows with `done` set (the same in all lanes of a row); first: the run's first lane.
-  auto emit = [&](bool done, uint64_t a, G gm, uint32_t R, uint32_t first) {
-    const uint32_t good =
-        (uint32_t)(__ballot(done && live && (G)xxh3_mix(xxh3_prep(a), g.chk_bf) == gm) >> base) & 0xffffu;
-    const bool zero =
-        ((uint32_t)(__ballot(done && i == kRowDet && (a | (uint64_t)gm) == 0) >> base) >> kRowDet) & 1u;
-    const uint32_t col = good & ((1u << kRowDet) - 1);
-    const bool det = (good >> kRowDet) & 1u;
-    bool left = false;
-    if (done) {
-      if (i == kRowDet) {
-        if (zero) samp[R] = kSampZero;
-        else if (det) leave(R, first, sample_record(kGood, a, g.n, flags));
-        else left = col == 0;
-      } else if (!zero && !det && col && i == (uint32_t)__builtin_ctz(col)) {
-        leave(R, first, sample_record(kGood, a, g.n, flags));
-      }
+  auto emit = [&](bool done, uint64_t a, G gm, uint32_t first) {
+    const bool zero = i == kRowDet && (a | (uint64_t)gm) == 0;
+    const bool ok = done && live && (zero || (G)xxh3_mix(xxh3_prep(a), g.chk_bf) == gm);
+    const uint32_t good = (uint32_t)(__ballot(ok) >> base) & 0xffffu;
+    const bool left = done && i == kRowDet && good == 0;
+    if (left || (ok && (good & before_me) == 0)) {
+      const uint32_t x = (uint32_t)(a >> 32), y = (uint32_t)a;
+      recs[first] = left ? kRecLeft : zero ? kSampZero : (x > y ? x : y) < g.n ? a : kRecBad;
     }
-    for (uint64_t b = __ballot(left); b; b &= b - 1) again |= 1ull << rd_lane_u32(first, __builtin_ctzll(b));
   };
 
   // The XOR of every prefix of the row's entries; a run is the XOR of two of them.  The runs are then
@@ -2094,8 +2085,7 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
       h_a = pa;
       h_g = pg;
     }
-    emit(ends && earlier, pa ^ done_a, (G)(pg ^ done_g), __shfl((unsigned)rt, (int)(base + k - 1)),
-         base + 31u - (uint32_t)__builtin_clz(earlier | 1u));
+    emit(ends && earlier, pa ^ done_a, (G)(pg ^ done_g), base + 31u - (uint32_t)__builtin_clz(earlier | 1u));
     if (ends) {
       done_a = pa;
       done_g = pg;
@@ -2125,12 +2115,24 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
   const bool ends_x = row == 3 ? !tail_open : ((starts >> (base + kRow)) & 1) != 0;
   if (__ballot(has_h && st_h)) {
     const uint32_t f = 63u - (uint32_t)__builtin_clzll(st_h | 1ull);
-    emit(has_h && st_h, h_a, h_g, __shfl((unsigned)rt, (int)f), f);
+    emit(has_h && st_h, h_a, h_g, f);
   }
   if (__ballot(ends_x && st_x)) {
     const uint32_t f = 63u - (uint32_t)__builtin_clzll(st_x | 1ull);
-    emit(ends_x && st_x, acc, accg, __shfl((unsigned)rt, (int)f), f);
+    emit(ends_x && st_x, acc, accg, f);
   }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  uint64_t rec = recs[lane];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  uint64_t again = __ballot(rec == kRecLeft);  // first lanes of the runs left to the deep records
+  if (rec == kRecBad) {  // an index out of range, as in sample_record
+    flags[kFlagBad] = 1;
+    rec = kSampFail;
+  }
+  if (rec != kRecNone && rec != kRecLeft) samp[rt] = rec;
+  else rec = kSampZero;
 
   // deep records: lane d < D of depths >= kRowDet; the XOR over the entries in lanes `of`
   const uint64_t deep = g.D > kRowDet ? __ballot(mine && flag != 0) : 0;
@@ -2171,17 +2173,11 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
     deep_sum(low_bits(end) & ~low_bits(f), &a, &gm);
     const uint64_t good =
         __ballot(lane >= kRowDet && lane < g.D && (G)xxh3_mix(xxh3_prep(a), g.chk_bf) == gm);
-    const uint32_t R = rd_lane_u32(rt, (int)f);
-    if (good ? lane == (uint32_t)__builtin_ctzll(good) : lane == 0)
-      leave(R, f, sample_record(good ? kGood : kFail, a, g.n, flags));
+    const uint64_t idx = good ? rd_lane_u64(a, __builtin_ctzll(good)) : 0;
+    const uint64_t deep_rec = sample_record(good ? kGood : kFail, idx, g.n, flags);
+    if (lane == f) samp[rt] = rec = deep_rec;
   }
-  if (recs) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    *pend = recs[lane];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
+  if (pend) *pend = rec;
 
   // Every lane stores the root (the same value), so every lane of this wave may read it back
   // without a barrier.  Slots are ordered by depth, the deterministic bucket at D.
