@@ -1983,7 +1983,7 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
                                       Slot tail, uint64_t* __restrict__ samp, uint32_t* __restrict__ flags,
                                       const unsigned char* __restrict__ det_cpy, bool deep_on, uint64_t* s_tot,
                                       const XAcc* xa, uint32_t blk_b0, uint32_t blk_b1, uint32_t* s_bnd,
-                                      uint64_t* pend = nullptr) {
+                                      uint64_t* pend, bool ahead = false) {
   constexpr uint32_t RB = 8 + sizeof(G);
   const uint32_t lane = lane_id(), i = lane % kRow, base = lane - i, row = lane / kRow;
   // lane base + k holds entry k of its row
@@ -2029,6 +2029,15 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
         if constexpr (kWide) ghi[k] = (uint32_t)((uint64_t)gm >> 32);
       },
       std::make_integer_sequence<uint32_t, kRow>{});
+  // ahead: the entries' lines of the next column, touched here so that the next round finds them in the L2
+  uint32_t near_line = 0, far_line = 0, last_line = 0;
+  if (ahead && mine) {
+    const unsigned char* nrow = slab + (size_t)m * g.row;
+    near_line = *reinterpret_cast<const uint32_t*>(nrow + rec_col_off<G>(g, round + 1, 0));
+    if (g.D > g.low) far_line = *reinterpret_cast<const uint32_t*>(nrow + rec_col_off<G>(g, round + 1, g.low));
+    if (kWide && g.D > g.low + 8)
+      last_line = *reinterpret_cast<const uint32_t*>(nrow + rec_col_off<G>(g, round + 1, g.low + 8));
+  }
   uint32_t flag = 1;
   if (kDeepFlags<G> && deep_on && mine)
     flag = *reinterpret_cast<const uint32_t*>(slab + (size_t)m * g.row + deep_flag_off(round));
@@ -2216,6 +2225,7 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
       lds_xor(s_tot + kWave + pos, (uint64_t)totg);
     }
   }
+  if (ahead) asm volatile("" ::"v"(near_line), "v"(far_line), "v"(last_line));
   if (holds_first && lane < 2) s_bnd[lane] = bnd;
   if (holds_last && lane == 2) s_bnd[2] = bnd;
 }
@@ -2376,8 +2386,16 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
 //
 // The workgroup reduces its grouped list in chunks of 64 entries (one wave each, reduce_members).  A
 // supernode continuing past a chunk is accumulated in LDS under the chunk where it starts (only one
-// supernode per chunk can continue past its end) and sampled after a barrier.  DSU and sample
-// loads that an earlier round of this kernel may have changed are device-coherent loads.
+// supernode per chunk can continue past its end) and sampled after a barrier.  Parents that an earlier
+// round of this kernel may have changed are read with device-coherent loads.
+//
+// A round is a chain of about eight steps between barriers, 15 to 45 thousand cycles with everything it
+// reads at hand, so the steps are few: roots are looked up from the old roots, the giant's beside them;
+// segments are taken from a cursor by each supernode's first member, without a scan of the table; a wave
+// links its samples as soon as it has them, without a pass over the table behind a device-wide fence
+// (each of the two a fifth of a round); the next round's lines are touched while this round's arrive.
+// 1000 vertices (5 rounds) 88 -> 61 us, the last 400 vertices of 2^18 44 -> 30, of a serving trace 23.6
+// -> 17.2, 8-byte checksums 38 -> 25.
 constexpr uint32_t kFinishMax = 2048;
 constexpr uint32_t kFinishTable = 4096;  // LDS hash table of roots, >= 2 * kFinishMax, power of two
 constexpr uint32_t kFinishChunks = kFinishMax / kWave;
@@ -2405,7 +2423,7 @@ __device__ inline uint32_t finish_slot(uint32_t* keys, uint32_t key) {
 template <class G>
 __global__ void __launch_bounds__(kRedBlock)
 k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ act0,
-            const unsigned char* __restrict__ slab, Geo g, uint32_t r0, uint32_t last_round,
+            const uint32_t* __restrict__ mroot0, const unsigned char* __restrict__ slab, Geo g, uint32_t r0, uint32_t last_round,
             uint64_t* __restrict__ samp, uint32_t* __restrict__ rstats, const unsigned char* __restrict__ det_cpy,
             const unsigned char* __restrict__ hint, uint32_t* __restrict__ rep, uint32_t deep_skip) {
   __shared__ uint32_t s_key[kFinishTable], s_cnt[kFinishTable];
@@ -2415,7 +2433,6 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
   __shared__ uint64_t s_slot[kRedWaves * 2 * 2 * kWave];  // per wave: head and tail of its chunk
   __shared__ uint32_t s_slotroot[kRedWaves * 2];
   __shared__ uint64_t s_tot[2 * kWave];
-  __shared__ uint32_t s_wsum[kRedWaves];
   __shared__ uint32_t s_take, s_gfirst, s_walk, s_gcur, s_e, s_elect;
   __shared__ unsigned long long s_best;
   const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
@@ -2427,6 +2444,7 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     const uint32_t walk = st[kStSeg + 2 * ((r0 - 1) & 1)];
     s_take = (live && walk <= kFinishMax) ? 1u : 0u;
     s_gfirst = gfirst;
+    s_gcur = kNoRoot;
     s_best = 0;
     s_walk = walk;
   }
@@ -2445,9 +2463,14 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     return;
   }
   uint32_t walk = s_walk;
-  uint32_t v[kFinishPer];
+  // the walked vertices and their roots of the round before
+  uint32_t v[kFinishPer], old[kFinishPer];
 #pragma unroll
-  for (uint32_t k = 0; k < kFinishPer; ++k) v[k] = tid + k * kRedBlock < walk ? act0[tid + k * kRedBlock] : 0u;
+  for (uint32_t k = 0; k < kFinishPer; ++k) {
+    const bool in = tid + k * kRedBlock < walk;
+    v[k] = in ? act0[tid + k * kRedBlock] : 0u;
+    old[k] = in ? mroot0[tid + k * kRedBlock] : 0u;
+  }
   for (uint32_t c = tid; c < kFinishChunks * 2 * kWave; c += kRedBlock) s_acc[c] = 0;
   for (uint32_t c = tid; c < kFinishChunks; c += kRedBlock) s_accroot[c] = kNoRoot;
 
@@ -2457,61 +2480,68 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
       s_cnt[k] = 0;
     }
     if (tid < 2 * kWave) s_tot[tid] = 0;
-    if (tid == 0) {
+    // The giant's root (it only grows) by the last thread, beside the roots of the walked vertices, which
+    // start at the vertices' old roots: one round trip where the old root is one still.
+    if (tid == kRedBlock - 1) {
       if (s_gfirst == kNoRoot && s_best) s_gfirst = (uint32_t)s_best;
-      s_gcur = s_gfirst == kNoRoot ? kNoRoot : dsu_find_coherent(d.parent, s_gfirst);  // the giant only grows
+      if (s_gcur == kNoRoot) s_gcur = s_gfirst;
+      if (s_gcur != kNoRoot) s_gcur = dsu_find_coherent(d.parent, s_gcur);
       s_elect = kNoRoot;
+      s_e = 0;
     }
+    uint32_t rr[kFinishPer], up[kFinishPer], slot[kFinishPer], pos[kFinishPer];
+    bool more = false;
+#pragma unroll
+    for (uint32_t k = 0; k < kFinishPer; ++k) {
+      rr[k] = old[k];
+      up[k] = tid + k * kRedBlock < walk ? ld_acq(d.parent + old[k]) : old[k];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kFinishPer; ++k) more |= up[k] != rr[k];
+    while (more) {
+      more = false;
+#pragma unroll
+      for (uint32_t k = 0; k < kFinishPer; ++k)
+        if (up[k] != rr[k]) {
+          rr[k] = up[k];
+          up[k] = ld_acq(d.parent + rr[k]);
+        }
+#pragma unroll
+      for (uint32_t k = 0; k < kFinishPer; ++k) more |= up[k] != rr[k];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kFinishPer; ++k)
+      if (tid + k * kRedBlock >= walk) rr[k] = kNoRoot;
     __syncthreads();
     uint32_t gcur = s_gcur;
-    // roots of the walked vertices, full path compression, members per root (k_bv_find_count)
-    uint32_t rr[kFinishPer], slot[kFinishPer], pos[kFinishPer];
-#pragma unroll
-    for (uint32_t k = 0; k < kFinishPer; ++k) rr[k] = tid + k * kRedBlock < walk ? dsu_find_coherent(d.parent, v[k]) : kNoRoot;
-    __syncthreads();
+    // path compression, members per root (k_bv_find_count)
 #pragma unroll
     for (uint32_t k = 0; k < kFinishPer; ++k) {
       if (rr[k] == kNoRoot) continue;
-      st_rlx(d.parent + v[k], rr[k]);
+      if (rr[k] != old[k]) st_rlx(d.parent + v[k], rr[k]);
       if (rr[k] != gcur) {  // members of the giant are not regrouped
         slot[k] = finish_slot(s_key, rr[k]);
         pos[k] = atomicAdd(s_cnt + slot[k], 1u);
       }
     }
     __syncthreads();
+    // The first member counted takes its supernode's segment, from a cursor (segments need no order); its
+    // slot's count becomes the segment's start.
     if (gcur == kNoRoot) {  // the giant's election and candidates, as in k_bv_alloc
-      for (uint32_t k = tid; k < kFinishTable; k += kRedBlock) {
-        const uint32_t c = s_cnt[k];
-        if (2ull * c > d.n) s_elect = s_gfirst = s_key[k];  // at most one
-        else if (c >= 2 && c >= d.n / kCandidateDiv) atomicMax(&s_best, ((unsigned long long)c << 32) | s_key[k]);
+#pragma unroll
+      for (uint32_t k = 0; k < kFinishPer; ++k) {
+        if (rr[k] == kNoRoot || pos[k] != 0) continue;
+        const uint32_t c = s_cnt[slot[k]];
+        if (2ull * c > d.n) s_elect = s_gfirst = rr[k];  // at most one
+        else if (c >= 2 && c >= d.n / kCandidateDiv) atomicMax(&s_best, ((unsigned long long)c << 32) | rr[k]);
       }
       __syncthreads();
       gcur = s_elect;
     }
-    // segment starts: exclusive scan of the counts over the table (4 slots per thread)
-    {
-      constexpr uint32_t per = kFinishTable / kRedBlock;
-      uint32_t c[per], sum = 0;
 #pragma unroll
-      for (uint32_t k = 0; k < per; ++k) {
-        c[k] = s_key[tid * per + k] == gcur ? 0u : s_cnt[tid * per + k];
-        sum += c[k];
-      }
-      const uint32_t incl = (uint32_t)wave_incl_scan_u64(sum);
-      if (lane == kWave - 1) s_wsum[wid] = incl;
-      __syncthreads();
-      uint32_t pre = 0, tot = 0;
-      for (uint32_t w = 0; w < kRedWaves; ++w) {
-        if (w < wid) pre += s_wsum[w];
-        tot += s_wsum[w];
-      }
-      uint32_t o = pre + incl - sum;
-#pragma unroll
-      for (uint32_t k = 0; k < per; ++k) {
-        s_cnt[tid * per + k] = o;  // now the segment start
-        o += c[k];
-      }
-      if (tid == 0) s_e = tot;
+    for (uint32_t k = 0; k < kFinishPer; ++k) {
+      if (rr[k] == kNoRoot || rr[k] == gcur || pos[k] != 0) continue;
+      s_cnt[slot[k]] = atomicAdd(&s_e, s_cnt[slot[k]]);
     }
     __syncthreads();
     const uint32_t e = s_e;
@@ -2537,11 +2567,13 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     const uint32_t nchunks = (e + cw - 1) / cw;
     Slot hs{s_slot + (size_t)(2 * wid) * 2 * kWave, s_slotroot + 2 * wid};
     Slot ts{s_slot + (size_t)(2 * wid + 1) * 2 * kWave, s_slotroot + 2 * wid + 1};
+    bool modified = false;
+    uint64_t pend;
     for (uint32_t c = wid; c < nchunks; c += kRedWaves) {
       const uint32_t p0 = c * cw;
       const uint32_t len = e - p0 < cw ? e - p0 : cw;
       reduce_members<G>(p0, len, cw / 4, e, s_mem, s_mroot, slab, g, r, hs, ts, samp, d.flags, det_cpy, deep_skip != 0,
-                        gcur != kNoRoot ? s_tot : nullptr, nullptr, 0, 0, nullptr);
+                        gcur != kNoRoot ? s_tot : nullptr, nullptr, 0, 0, nullptr, &pend, r < last_round);
       const uint32_t hr = *hs.root, tr = *ts.root;
       if (hr != kNoRoot) {  // started in an earlier chunk
         uint64_t* acc = s_acc + (size_t)(s_seg[p0] / cw) * 2 * kWave;
@@ -2554,7 +2586,10 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
         lds_xor(acc + kWave + lane, ts.vals[kWave + lane]);
         if (lane == 0) s_accroot[c] = tr;
       }
+      if (apply_sample(d, pend, hint)) modified = true;
     }
+    pend = kSampZero;
+    uint32_t pended = 0;  // the wave's samples of supernodes past a chunk, one to a lane
     __syncthreads();
     for (uint32_t c = wid; c < nchunks; c += kRedWaves) {
       const uint32_t R = s_accroot[c];
@@ -2562,25 +2597,19 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
       uint64_t* acc = s_acc + (size_t)c * 2 * kWave;
       uint64_t idx;
       const int code = wave_sample<G>(acc[lane], (G)acc[kWave + lane], g.D, g.chk_bf, &idx);
-      if (lane == 0) samp[R] = sample_record(code, idx, g.n, d.flags);
+      const uint64_t rec = sample_record(code, idx, g.n, d.flags);
+      if (lane == pended++) pend = rec;
       acc[lane] = 0;  // zero for the next round
       acc[kWave + lane] = 0;
       if (lane == 0) s_accroot[c] = kNoRoot;
     }
-    if (wid == kRedWaves - 1 && gcur != kNoRoot) {  // the giant, from the complement
+    if (wid == kRedWaves - 1 && gcur != kNoRoot && e != 0) {  // the giant, from the complement
       uint64_t idx;
       const int code = wave_sample<G>(s_tot[lane], (G)s_tot[kWave + lane], g.D, g.chk_bf, &idx);
-      if (lane == 0) samp[gcur] = e == 0 ? kSampZero : sample_record(code, idx, g.n, d.flags);
+      const uint64_t rec = sample_record(code, idx, g.n, d.flags);
+      if (lane == pended) pend = rec;
     }
-    // The samples were written with plain stores; the merges read them with device-coherent loads,
-    // which a workgroup barrier alone does not order after those stores.
-    __threadfence();
-    __syncthreads();
-    // merges: every supernode root of the walk, and the giant
-    bool modified = false;
-    for (uint32_t k = tid; k < kFinishTable; k += kRedBlock)
-      if (s_key[k] != kEmptyKey && apply_sample(d, ld_acq(samp + s_key[k]), hint)) modified = true;
-    if (tid == 0 && gcur != kNoRoot && apply_sample(d, ld_acq(samp + gcur), hint)) modified = true;
+    if (apply_sample(d, pend, hint)) modified = true;
     const bool any = __syncthreads_or(modified);
     if (tid == 0 && any) st_rlx(d.mod + r, 1u);
     if (!any || r >= last_round) {
@@ -2591,7 +2620,11 @@ k_bv_finish(DsuDev d, uint32_t* __restrict__ st, const uint32_t* __restrict__ ac
     // the next round walks this round's members
     walk = e;
 #pragma unroll
-    for (uint32_t k = 0; k < kFinishPer; ++k) v[k] = tid + k * kRedBlock < walk ? s_mem[tid + k * kRedBlock] : 0u;
+    for (uint32_t k = 0; k < kFinishPer; ++k) {
+      const bool in = tid + k * kRedBlock < walk;
+      v[k] = in ? s_mem[tid + k * kRedBlock] : 0u;
+      old[k] = in ? s_mroot[tid + k * kRedBlock] : 0u;
+    }
     __syncthreads();
   }
 }
@@ -3048,11 +3081,12 @@ bool launch_finish(int gbytes, uint32_t r0, uint32_t last_round, const unsigned 
                    const DsuDev& d, const RoundBufs& rb, hipStream_t s, uint32_t* rep, bool deep_skip) {
   if (r0 < 2 || r0 > last_round) return false;  // round r0 walks round r0 - 1's member list
   const uint32_t* act0 = rb.members[(r0 - 1) & 1];
+  const uint32_t* mroot0 = rb.mroot[(r0 - 1) & 1];
   if (gbytes == 4)
-    hipLaunchKernelGGL(k_bv_finish<uint32_t>, dim3(1), dim3(kRedBlock), 0, s, d, rb.totals, act0, slab, g, r0,
+    hipLaunchKernelGGL(k_bv_finish<uint32_t>, dim3(1), dim3(kRedBlock), 0, s, d, rb.totals, act0, mroot0, slab, g, r0,
                        last_round, rb.samp, rb.rstats, rb.det_cpy, rb.hint, rep, deep_skip ? 1u : 0u);
   else
-    hipLaunchKernelGGL(k_bv_finish<uint64_t>, dim3(1), dim3(kRedBlock), 0, s, d, rb.totals, act0, slab, g, r0,
+    hipLaunchKernelGGL(k_bv_finish<uint64_t>, dim3(1), dim3(kRedBlock), 0, s, d, rb.totals, act0, mroot0, slab, g, r0,
                        last_round, rb.samp, rb.rstats, rb.det_cpy, rb.hint, rep, deep_skip ? 1u : 0u);
   return true;
 }
