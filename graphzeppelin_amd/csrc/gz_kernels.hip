@@ -1890,7 +1890,7 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
 // its partial XOR in the range's head or tail slot under its root; a slot left unused gets root
 // kNoRoot and a zero value.
 //
-// A workgroup of 16 waves covers 1024 entries: the waves leave their slots in LDS, then the wave in
+// A workgroup of 16 waves covers 1024 entries (512 or 256 in smaller rounds): the waves leave their slots in LDS, then the wave in
 // which a crossing supernode starts adds up that supernode's slots, so at most two supernodes of a
 // workgroup are unfinished: the one continuing from the previous workgroup and the one continuing
 // into the next.
@@ -2245,16 +2245,16 @@ __device__ inline void xacc_add(uint64_t* slot, uint64_t a, uint64_t gm) {
   __shared__ uint64_t s_tot[2 * kWave];                           \
   __shared__ uint32_t s_bnd[3];
 
-// The reduce of a whole round: one workgroup per 1024 entries of the member list (e1 entries,
-// written by k_bv_scatter), gridDim.x >= ceil(e1 / 1024).
+// The reduce of a whole round: one workgroup per 1024, 512 or 256 entries of the member list (e1 entries,
+// written by k_bv_scatter; ReduceShape), gridDim.x >= reduce_blocks(n).
 template <class G>
 __global__ void __launch_bounds__(kRedBlock)
 k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ members,
             const uint32_t* __restrict__ mroot, const unsigned char* __restrict__ slab, Geo g, uint32_t round,
             XAcc xa, uint64_t* __restrict__ samp, DsuDev d,
             const uint32_t* __restrict__ prev_mod, uint32_t* __restrict__ cur_mod, uint32_t* __restrict__ rstats,
-            const unsigned char* __restrict__ det_cpy, const unsigned char* __restrict__ hint, uint32_t small_walk,
-            uint32_t deep_skip) {
+            const unsigned char* __restrict__ det_cpy, const unsigned char* __restrict__ hint, uint32_t upto16,
+            uint32_t upto32, uint32_t deep_skip) {
   const uint32_t live = ld_acq(prev_mod);  // checked after the first reads
   GZ_REDUCE_LDS
   const uint32_t giant = st[kStGiantRound];
@@ -2269,10 +2269,7 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
     if (blockIdx.x == 0 && threadIdx.x == 0) samp[giant] = kSampZero;
     return;
   }
-  // Entries per wave: 64, or 32 for a round of at most small_walk entries (16 at most
-  // small_walk / 8), whose few workgroups would otherwise each wait out a long chain of dependent
-  // gathers (the grid holds enough workgroups for each choice).
-  const uint32_t W = e1 <= small_walk / 8 ? kWave / 4 : e1 <= small_walk ? kWave / 2 : kWave;
+  const uint32_t W = e1 <= upto16 ? kWave / 4 : e1 <= upto32 ? kWave / 2 : kWave;  // see ReduceShape
   const uint32_t span = kRedWaves * W;
   const uint32_t blk = blockIdx.x;
   if (blk * span >= e1) return;  // uniform over the workgroup
@@ -3032,11 +3029,26 @@ void launch_sample_round0(int gbytes, const unsigned char* slab, const Geo& g, c
   hipLaunchKernelGGL(k_apply_samples, dim3(grid_for(g.n, 256, 4096)), dim3(256), 0, s, samp, d, rb.hint);
 }
 
-// Host bound on each level's entry count (the kernels compute the exact counts on the device):
-// the larger of the chain without a supernode summed from its complement (level 2 = 2 * B1) and
-// with one (level 2 = 3 * B1); e1 <= n in both.
-uint32_t reduce_blocks(uint32_t n) { return 2 * std::max(1u, (n + kRedBlock - 1) / kRedBlock); }
-constexpr uint32_t kSmallWalkDiv = 2;  // rounds regrouping at most n / kSmallWalkDiv entries use 32 per wave
+// Entries per wave of the reduce: 64, but 16 in rounds of at most upto16 entries and 32 up to upto32.  Up
+// to 256 workgroups of 16 waves, fewer entries per wave cost nothing but bring in more CUs: 64 entries
+// per wave would leave a round of 32k entries on 32 of 256 CUs, each waiting for 16 loads per lane and
+// sampling for 16 waves.  Past that they cost atomics on the sums of supernodes that cross workgroups,
+// which a round much smaller than n, grouped into few supernodes or mostly into the giant, has less of.
+// Against bounds of n / 16 and n / 2 alone: reduces of 2^17 vertices with 8-byte checksums 29.3 -> 24.9 us
+// on average, of 2^18 31.3 -> 29.7, of 1000 vertices 23.4 -> 15.4.
+struct ReduceShape {
+  uint32_t upto16, upto32;
+  explicit ReduceShape(uint32_t n)
+      : upto16(std::max(n / 16, 256u * kRedWaves * 16)), upto32(std::max(n / 2, 256u * kRedWaves * 32)) {}
+};
+// Workgroups of a reduce, for any round of at most n entries.
+uint32_t reduce_blocks(uint32_t n) {
+  const ReduceShape s(n);
+  auto blocks = [](uint32_t entries, uint32_t per_wave) {
+    return (uint32_t)(((uint64_t)entries + kRedWaves * per_wave - 1) / (kRedWaves * per_wave));
+  };
+  return std::max({1u, blocks(std::min(n, s.upto16), 16), blocks(std::min(n, s.upto32), 32), blocks(n, 64)});
+}
 
 void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const Geo& g,
                   const DsuDev& d, const RoundBufs& rb, bool giant_ok, bool drop_ok, hipStream_t s, bool deep_skip) {
@@ -3065,16 +3077,17 @@ void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const G
   }
   // one accumulator slot per workgroup and one for the giant
   const uint32_t rgrid = reduce_blocks(n);
+  const ReduceShape shape(n);
   if (rgrid + 1 > rb.xslots) throw std::logic_error("reduce grid exceeds its cross-workgroup accumulator slots");
   const XAcc xa{rb.xacc, rb.xcnt, rb.xslots, rb.off, rb.cursor};
   if (gbytes == 4)
     hipLaunchKernelGGL(k_bv_reduce<uint32_t>, dim3(rgrid), dim3(kRedBlock), 0, s, st, members, rb.mroot[par],
-                       slab, g, round, xa, rb.samp, d, prev, cur, rb.rstats, rb.det_cpy, rb.hint, n / kSmallWalkDiv,
-                       deep_skip ? 1u : 0u);
+                       slab, g, round, xa, rb.samp, d, prev, cur, rb.rstats, rb.det_cpy, rb.hint, shape.upto16,
+                       shape.upto32, deep_skip ? 1u : 0u);
   else
     hipLaunchKernelGGL(k_bv_reduce<uint64_t>, dim3(rgrid), dim3(kRedBlock), 0, s, st, members, rb.mroot[par],
-                       slab, g, round, xa, rb.samp, d, prev, cur, rb.rstats, rb.det_cpy, rb.hint, n / kSmallWalkDiv,
-                       deep_skip ? 1u : 0u);
+                       slab, g, round, xa, rb.samp, d, prev, cur, rb.rstats, rb.det_cpy, rb.hint, shape.upto16,
+                       shape.upto32, deep_skip ? 1u : 0u);
 }
 
 bool launch_finish(int gbytes, uint32_t r0, uint32_t last_round, const unsigned char* slab, const Geo& g,
