@@ -1913,7 +1913,9 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
 // with device-scope XOR atomics into the accumulator slot of f, its first workgroup (only one
 // supernode per workgroup can continue past its end, so f identifies it).  Every workgroup of f..l
 // adds its part once and then counts itself in slot f's counter; the one that brings the count to
-// l - f + 1 samples the sum and clears the slot and the counter for the next round.  The segment
+// l - f + 1 samples the sum and clears the slot and the counter for the next round.  A release before
+// the count and an acquire after the last one are all the order this needs: with a full fence in both
+// places a reduce of 2^18 vertices took 29.7 us on average instead of 26.0, of 32k 13.7 instead of 11.8.  The segment
 // bounds come from k_bv_alloc / k_bv_scatter (off = start, cursor = end).  No workgroup waits for
 // another, and the XOR is order-free, so the sum is exactly the member-wise merge.
 //
@@ -2333,11 +2335,11 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
   auto cross = [&](uint32_t slot, uint32_t parts, uint32_t R, uint64_t a, uint64_t gm) {
     uint64_t* sv = xa.vals + (size_t)slot * 2 * kWave;
     xacc_add(sv, a, gm);
-    __threadfence();  // the part is visible before the arrival is counted
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // the part is visible before the arrival is counted
     uint32_t before = 0;
     if (lane == 0) before = atomicAdd(xa.cnt + slot, 1u);
     if (rd_lane_u32(before, 0) != parts - 1) return;
-    __threadfence();  // every part counted before ours is visible
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // every part counted before ours is visible
     sample_to(R, ld_acq(sv + lane), ld_acq(sv + kWave + lane));
     st_rlx(sv + lane, (uint64_t)0);
     st_rlx(sv + kWave + lane, (uint64_t)0);
