@@ -1738,92 +1738,43 @@ k_bv_scatter(const uint2* __restrict__ nd, uint32_t n, const uint32_t* __restric
 // nothing when the round is not live; indices computed from device data are bounded by n before
 // every store.
 
-__global__ void __launch_bounds__(kAggBlock)
-k_seg_find(uint32_t* __restrict__ parent, uint32_t n, uint32_t* __restrict__ cnt, uint2* __restrict__ nd,
-           uint32_t* __restrict__ st, uint32_t round, const RoundSeg* __restrict__ segs_old,
-           const uint32_t* __restrict__ prev_mod) {
-  const uint32_t live = ld_acq(prev_mod);
-  uint32_t gfirst = st[kStGiantFirst];
-  const uint64_t best = *reinterpret_cast<const uint64_t*>(st + kStBest);
-  const uint32_t nseg = st[kStSeg + 2 * ((round - 1) & 1) + 1];
-  const uint32_t i = blockIdx.x * kAggBlock + threadIdx.x;
-  const bool in = i < nseg;
-  RoundSeg sg{0, 0, 0, 0};
-  if (in) sg = segs_old[i];
-  // block 0 writes the round state even with no segments to walk
-  if (!live || (blockIdx.x > 0 && blockIdx.x * kAggBlock >= nseg)) return;
-  __shared__ uint32_t t_key[kAggTable], t_cnt[kAggTable];
-  for (uint32_t k = threadIdx.x; k < kAggTable; k += kAggBlock) {
-    t_key[k] = kEmptyKey;
-    t_cnt[k] = 0;
-  }
-  if (gfirst == kNoRoot && best) gfirst = (uint32_t)best;  // a candidate recorded by the previous round
-  const bool act = gfirst != kNoRoot;
-  const uint32_t gcur = act ? dsu_find_stable(parent, gfirst) : kNoRoot;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    st[kStSeg + 2 * (round & 1)] = 0;
-    st[kStSeg + 2 * (round & 1) + 1] = 0;
-    st[kStGiantRound] = gcur;
-    st[kStGiantFirst] = gfirst;
-    st[kStActMode] = act ? 1u : 0u;
-  }
-  __shared__ uint32_t t_base[kAggTable];
-  const bool ok = in && sg.root < n;
-  uint32_t r = 0;
-  if (ok) r = dsu_find_stable(parent, sg.root);
-  __syncthreads();
-  const bool counted = ok && r != gcur;
-  uint32_t my_slot = 0, my_pos = 0;
-  if (ok) parent[sg.root] = r;  // path compression of the old root (members are compressed in C)
-  if (counted) {
-    my_slot = lds_table_slot(t_key, r);
-    my_pos = atomicAdd(t_cnt + my_slot, sg.len);
-  }
-  __syncthreads();
-  for (uint32_t k = threadIdx.x; k < kAggTable; k += kAggBlock)
-    if (t_key[k] != kEmptyKey) t_base[k] = atomicAdd(cnt + t_key[k], t_cnt[k]);
-  __syncthreads();
-  // the run's offset in its new root's segment, minus its old start: a member at old position i
-  // goes to off[new root] + i + nd.y
-  if (ok) nd[sg.root] = make_uint2(r, counted ? t_base[my_slot] + my_pos - sg.start : 0u);
-}
-
-// B: a segment for every new root (an old root that is still a root) outside the giant; cnt is
-// cleared here, its last reader.  Giant election and candidate as in k_bv_alloc.
-__global__ void __launch_bounds__(kAggBlock)
-k_seg_alloc(uint32_t* __restrict__ cnt, uint32_t n, const uint2* __restrict__ nd, uint32_t* __restrict__ off,
-            uint32_t* __restrict__ cursor, RoundSeg* __restrict__ segs_new, uint32_t* __restrict__ st, uint32_t round,
-            const RoundSeg* __restrict__ segs_old, uint32_t giant_ok, const uint32_t* __restrict__ prev_mod,
-            const uint64_t* __restrict__ samp, uint32_t drop_ok) {
-  const uint32_t live = ld_acq(prev_mod);
+// What a round's segments are written to.
+struct SegOut {
+  uint32_t *off, *cursor;
+  RoundSeg* segs;
+};
+// A segment of c members for root v, whose segment of the last round had old_len (threads without one
+// pass c == 0), and the giant's election and candidate as in k_bv_alloc; every thread of the workgroup
+// takes part.  SINGLE: this workgroup has all of the round's segments, and one thread writes the round's
+// state, the giant elected here or the one known (gfirst, by its root gcur).
+template <bool SINGLE>
+__device__ inline void seg_allocate(uint32_t c, uint32_t v, uint32_t old_len, uint64_t sv, bool act, uint32_t n,
+                                    const SegOut& out, uint32_t* __restrict__ st, uint32_t round, uint32_t giant_ok,
+                                    uint32_t drop_ok, uint32_t gfirst, uint32_t gcur) {
   __shared__ uint64_t wsum[kAggBlock / kWave];
-  __shared__ uint32_t s_base, s_sbase, s_drop;
-  const bool act = st[kStActMode] != 0;
-  const uint32_t nseg = st[kStSeg + 2 * ((round - 1) & 1) + 1];
+  __shared__ uint32_t s_base, s_sbase, s_drop, s_elect;
   const uint32_t lane = lane_id(), wid = threadIdx.x / kWave;
-  const uint32_t i = blockIdx.x * kAggBlock + threadIdx.x;
-  const bool in = i < nseg;
-  const uint32_t v = in ? segs_old[i].root : 0, old_len = in ? segs_old[i].len : 0;
-  const bool ok = in && v < n;
-  const bool is_root = ok && nd[v].x == v;
-  uint32_t c = is_root ? cnt[v] : 0;  // zero for the giant's root: its members are not counted
-  const uint64_t sv = ok && drop_ok ? samp[v] : kSampFail;
-  if (!live || blockIdx.x * kAggBlock >= nseg) return;  // whole blocks past the segments
-  if (drop_ok) {  // uniform
-    if (threadIdx.x == 0) s_drop = 0;
+  if (SINGLE || drop_ok) {  // uniform
+    if (threadIdx.x == 0) {
+      s_drop = 0;
+      s_elect = kNoRoot;
+    }
     __syncthreads();
   }
-  if (c) cnt[v] = 0;
   if (!act && giant_ok && 2ull * c > n) {
-    st[kStGiantFirst] = v;
-    st[kStGiantRound] = v;
+    if (SINGLE) {
+      s_elect = v;
+    } else {
+      st[kStGiantFirst] = v;
+      st[kStGiantRound] = v;
+    }
     c = 0;
   } else if (!act && giant_ok && c >= 2 && c >= n / kCandidateDiv) {
     atomicMax(reinterpret_cast<unsigned long long*>(st + kStBest), ((unsigned long long)c << 32) | v);
   } else if (c != 0 && c == old_len && sv == kSampZero) {
     atomicAdd(&s_drop, c);
     c = 0;
-    off[v] = kDropped;
+    out.off[v] = kDropped;
   }
   const uint64_t x = c ? ((uint64_t)1 << kSegShift) | c : 0;
   const uint64_t incl = wave_incl_scan_u64(x);
@@ -1837,22 +1788,107 @@ k_seg_alloc(uint32_t* __restrict__ cnt, uint32_t n, const uint2* __restrict__ nd
   constexpr uint64_t kCntMask = ((uint64_t)1 << kSegShift) - 1;
   if (threadIdx.x == 0) {
     if (drop_ok && s_drop) atomicAdd(st + kStDropped, s_drop);
-    // entries and supernodes of the block in one 64-bit atomic (neither sum can reach 2^32)
+    // entries and supernodes of the block in one 64-bit word (neither sum can reach 2^32)
+    auto* both = reinterpret_cast<unsigned long long*>(st + kStSeg + 2 * (round & 1));
     const uint64_t add = ((tot >> kSegShift) << 32) | (tot & kCntMask);
-    const uint64_t old =
-        add ? atomicAdd(reinterpret_cast<unsigned long long*>(st + kStSeg + 2 * (round & 1)), (unsigned long long)add) : 0;
-    s_base = (uint32_t)old;
-    s_sbase = (uint32_t)(old >> 32);
+    uint64_t base = 0;
+    if (SINGLE) {
+      *both = add;
+      st[kStGiantRound] = s_elect != kNoRoot ? s_elect : gcur;
+      st[kStGiantFirst] = s_elect != kNoRoot ? s_elect : gfirst;
+      st[kStActMode] = act ? 1u : 0u;
+    } else if (add) base = atomicAdd(both, (unsigned long long)add);
+    s_base = (uint32_t)base;
+    s_sbase = (uint32_t)(base >> 32);
   }
   __syncthreads();
   if (c) {
     const uint64_t ex = pre + incl - x;
     const uint32_t o = s_base + (uint32_t)(ex & kCntMask);
     const uint32_t k = s_sbase + (uint32_t)(ex >> kSegShift);
-    off[v] = o;
-    cursor[v] = o + c;  // the segment end, as the vertex scatter leaves it
-    if (k < n) segs_new[k] = RoundSeg{v, o, c, 0};
+    out.off[v] = o;
+    out.cursor[v] = o + c;  // the segment end, as the vertex scatter leaves it
+    if (k < n) out.segs[k] = RoundSeg{v, o, c, 0};
   }
+}
+
+__global__ void __launch_bounds__(kAggBlock)
+k_seg_find(uint32_t* __restrict__ parent, uint32_t n, uint32_t* __restrict__ cnt, uint2* __restrict__ nd,
+           SegOut out, uint32_t* __restrict__ st, uint32_t round, const RoundSeg* __restrict__ segs_old,
+           uint32_t giant_ok, const uint32_t* __restrict__ prev_mod, const uint64_t* __restrict__ samp,
+           uint32_t drop_ok) {
+  const uint32_t live = ld_acq(prev_mod);
+  uint32_t gfirst = st[kStGiantFirst];
+  const uint64_t best = *reinterpret_cast<const uint64_t*>(st + kStBest);
+  const uint32_t nseg = st[kStSeg + 2 * ((round - 1) & 1) + 1];
+  const uint32_t i = blockIdx.x * kAggBlock + threadIdx.x;
+  const bool in = i < nseg;
+  RoundSeg sg{0, 0, 0, 0};
+  if (in) sg = segs_old[i];
+  const bool single = nseg <= kAggBlock;  // this workgroup meets every member of every new supernode
+  // block 0 writes the round state even with no segments to walk
+  if (!live || (blockIdx.x > 0 && blockIdx.x * kAggBlock >= nseg)) return;
+  __shared__ uint32_t t_key[kAggTable], t_cnt[kAggTable];
+  for (uint32_t k = threadIdx.x; k < kAggTable; k += kAggBlock) {
+    t_key[k] = kEmptyKey;
+    t_cnt[k] = 0;
+  }
+  if (gfirst == kNoRoot && best) gfirst = (uint32_t)best;  // a candidate recorded by the previous round
+  const bool act = gfirst != kNoRoot;
+  const uint32_t gcur = act ? dsu_find_stable(parent, gfirst) : kNoRoot;
+  if (!single && blockIdx.x == 0 && threadIdx.x == 0) {
+    st[kStSeg + 2 * (round & 1)] = 0;
+    st[kStSeg + 2 * (round & 1) + 1] = 0;
+    st[kStGiantRound] = gcur;
+    st[kStGiantFirst] = gfirst;
+    st[kStActMode] = act ? 1u : 0u;
+  }
+  __shared__ uint32_t t_base[kAggTable];
+  const bool ok = in && sg.root < n;
+  const uint64_t sv = single && ok && drop_ok ? samp[sg.root] : kSampFail;
+  uint32_t r = 0;
+  if (ok) r = dsu_find_stable(parent, sg.root);
+  __syncthreads();
+  const bool counted = ok && r != gcur;
+  uint32_t my_slot = 0, my_pos = 0;
+  if (ok) parent[sg.root] = r;  // path compression of the old root (members are compressed in C)
+  if (counted) {
+    my_slot = lds_table_slot(t_key, r);
+    my_pos = atomicAdd(t_cnt + my_slot, sg.len);
+  }
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < kAggTable; k += kAggBlock)
+    if (t_key[k] != kEmptyKey) t_base[k] = single ? 0u : atomicAdd(cnt + t_key[k], t_cnt[k]);
+  __syncthreads();
+  // the run's offset in its new root's segment, minus its old start: a member at old position i
+  // goes to off[new root] + i + nd.y
+  if (ok) nd[sg.root] = make_uint2(r, counted ? t_base[my_slot] + my_pos - sg.start : 0u);
+  // few supernodes: their segments are given out here, without the counters, and k_seg_alloc has nothing
+  // to do: a query over 32k vertices in 64 components 500 -> 490 us, a point query on 2^18 519 -> 510
+  if (single)
+    seg_allocate<true>(counted && r == sg.root ? t_cnt[my_slot] : 0u, sg.root, sg.len, sv, act, n, out, st, round,
+                       giant_ok, drop_ok, gfirst, gcur);
+}
+
+// B: a segment for every new root (an old root that is still a root) outside the giant; cnt is
+// cleared here, its last reader.
+__global__ void __launch_bounds__(kAggBlock)
+k_seg_alloc(uint32_t* __restrict__ cnt, uint32_t n, const uint2* __restrict__ nd, SegOut out, uint32_t* __restrict__ st,
+            uint32_t round, const RoundSeg* __restrict__ segs_old, uint32_t giant_ok,
+            const uint32_t* __restrict__ prev_mod, const uint64_t* __restrict__ samp, uint32_t drop_ok) {
+  const uint32_t live = ld_acq(prev_mod);
+  const bool act = st[kStActMode] != 0;
+  const uint32_t nseg = st[kStSeg + 2 * ((round - 1) & 1) + 1];
+  if (!live || nseg <= kAggBlock || blockIdx.x * kAggBlock >= nseg) return;  // whole blocks past the segments
+  const uint32_t i = blockIdx.x * kAggBlock + threadIdx.x;
+  const bool in = i < nseg;
+  const uint32_t v = in ? segs_old[i].root : 0, old_len = in ? segs_old[i].len : 0;
+  const bool ok = in && v < n;
+  const bool is_root = ok && nd[v].x == v;
+  const uint32_t c = is_root ? cnt[v] : 0;  // zero for the giant's root: its members are not counted
+  const uint64_t sv = ok && drop_ok ? samp[v] : kSampFail;
+  if (c) cnt[v] = 0;
+  seg_allocate<false>(c, v, old_len, sv, act, n, out, st, round, giant_ok, drop_ok, kNoRoot, kNoRoot);
 }
 
 // C: every member of the old list to its place, its new root beside it, its parent compressed to
@@ -3070,10 +3106,11 @@ void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const G
     hipLaunchKernelGGL(k_bv_scatter, dim3(grid), dim3(kAggBlock), 0, s, rb.nd, n, rb.off, members, rb.mroot[par],
                        st, round, act_list, prev);
   } else {  // whole runs of the previous round's member list
-    hipLaunchKernelGGL(k_seg_find, dim3(grid), dim3(kAggBlock), 0, s, d.parent, n, rb.cnt, rb.nd, st, round,
-                       rb.segs[opar], prev);
-    hipLaunchKernelGGL(k_seg_alloc, dim3(grid), dim3(kAggBlock), 0, s, rb.cnt, n, rb.nd, rb.off, rb.cursor,
-                       rb.segs[par], st, round, rb.segs[opar], giant_ok ? 1u : 0u, prev, rb.samp, drop_ok ? 1u : 0u);
+    const SegOut out{rb.off, rb.cursor, rb.segs[par]};
+    hipLaunchKernelGGL(k_seg_find, dim3(grid), dim3(kAggBlock), 0, s, d.parent, n, rb.cnt, rb.nd, out, st, round,
+                       rb.segs[opar], giant_ok ? 1u : 0u, prev, rb.samp, drop_ok ? 1u : 0u);
+    hipLaunchKernelGGL(k_seg_alloc, dim3(grid), dim3(kAggBlock), 0, s, rb.cnt, n, rb.nd, out, st, round,
+                       rb.segs[opar], giant_ok ? 1u : 0u, prev, rb.samp, drop_ok ? 1u : 0u);
     hipLaunchKernelGGL(k_seg_copy, dim3(grid_for(n, 256)), dim3(256), 0, s, n, rb.nd, rb.off, d.parent, rb.members[opar],
                        rb.mroot[opar], members, rb.mroot[par], st, round, prev);
   }
