@@ -1943,15 +1943,18 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
 // 16 lanes a member filled 16 of a load's 64 lanes and a wave took its members in 8 dependent
 // batches: the launched rounds of a 24M-update, 2^18-vertex serving trace went from 39.1 to 25.0 us on
 // average, those of 32k vertices from 34.3 to 15.0 us, of 2^20 R-MAT vertices from 147 to 79 us, and
-// the single-workgroup finish of about 1500 members from 95 to 47 us.
+// the single-workgroup finish of about 1500 members from 95 to 47 us (30 with its own changes).
 //
 // Cross-workgroup supernodes.  A supernode whose entries span workgroups f..l (f < l) is combined
 // with device-scope XOR atomics into the accumulator slot of f, its first workgroup (only one
 // supernode per workgroup can continue past its end, so f identifies it).  Every workgroup of f..l
 // adds its part once and then counts itself in slot f's counter; the one that brings the count to
-// l - f + 1 samples the sum and clears the slot and the counter for the next round.  A release before
-// the count and an acquire after the last one are all the order this needs: with a full fence in both
-// places a reduce of 2^18 vertices took 29.7 us on average instead of 26.0, of 32k 13.7 instead of 11.8.  The segment
+// l - f + 1 samples the sum and clears the slot and the counter for the next round.  The parts are
+// added with atomics that return, so they have been performed when the count is made, and the last one
+// takes the sum with exchanges that leave zeros: no fence, which would write caches back and invalidate
+// them for every part.  A reduce of 2^18 vertices took 29.7 us on average with a full fence before the
+// count and after the last one, 26.0 with a release and an acquire, 23.2 now; of 32k vertices 13.7, 11.8
+// and 10.8.  The segment
 // bounds come from k_bv_alloc / k_bv_scatter (off = start, cursor = end).  No workgroup waits for
 // another, and the XOR is order-free, so the sum is exactly the member-wise merge.
 //
@@ -2268,11 +2271,18 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
   if (holds_last && lane == 2) s_bnd[2] = bnd;
 }
 
-// Per lane: XOR (a, gm) into an accumulator slot with device-scope atomics (zero words skipped).
+// Per lane: XOR (a, gm) into an accumulator slot with device-scope atomics (zero words skipped), and wait
+// for their results, after which they have been performed.
 __device__ inline void xacc_add(uint64_t* slot, uint64_t a, uint64_t gm) {
   const uint32_t lane = lane_id();
-  if (a) __hip_atomic_fetch_xor(slot + lane, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (gm) __hip_atomic_fetch_xor(slot + kWave + lane, gm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint64_t was_a = 0, was_g = 0;
+  if (a) was_a = __hip_atomic_fetch_xor(slot + lane, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (gm) was_g = __hip_atomic_fetch_xor(slot + kWave + lane, gm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::"v"(was_a), "v"(was_g) : "memory");
+}
+// An accumulator word, left zero.
+__device__ inline uint64_t xacc_take(uint64_t* word) {
+  return __hip_atomic_exchange(word, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // LDS of one reduce workgroup: 32 slots of 128 u64 and their roots, the giant total and the segment
@@ -2371,14 +2381,11 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
   auto cross = [&](uint32_t slot, uint32_t parts, uint32_t R, uint64_t a, uint64_t gm) {
     uint64_t* sv = xa.vals + (size_t)slot * 2 * kWave;
     xacc_add(sv, a, gm);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // the part is visible before the arrival is counted
     uint32_t before = 0;
     if (lane == 0) before = atomicAdd(xa.cnt + slot, 1u);
     if (rd_lane_u32(before, 0) != parts - 1) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // every part counted before ours is visible
-    sample_to(R, ld_acq(sv + lane), ld_acq(sv + kWave + lane));
-    st_rlx(sv + lane, (uint64_t)0);
-    st_rlx(sv + kWave + lane, (uint64_t)0);
+    const uint64_t sum_a = xacc_take(sv + lane), sum_g = xacc_take(sv + kWave + lane);
+    sample_to(R, sum_a, sum_g);
     if (lane == 0) st_rlx(xa.cnt + slot, 0u);
   };
   if (wid < nw) {  // the supernode that starts in this wave and goes on
