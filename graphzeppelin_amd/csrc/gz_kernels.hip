@@ -2898,6 +2898,9 @@ void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_d
   const size_t lds = update_tiles_lds_bytes(g, gbytes);
   const uint32_t ldepth = lds_depth(g.C, gbytes);
   const bool wide = g.C * ldepth + 1 > kPerLane * kWave;
+  const uint32_t rb = 8 + gbytes, end = std::min(g.D, ldepth);  // the last column's deepest place in the delta
+  if (g.ovf + (end > g.low ? (g.C - 1) * g.opitch + (end - 1 - g.low) * rb : 0u) > 4u * 0xFFFFu)
+    throw std::logic_error("a row's records lie past the update kernel's 16-bit places");
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kWave), lds, s, tiles, ntiles_dev, ntiles_host, dsts, slab, g, col_bf,
                        ldepth, 65536 / ldepth + 1);

@@ -54,6 +54,12 @@ void launch_update_tiles(int gbytes, const Tile* tiles, const uint32_t* ntiles_d
 void launch_sketch_update(int gbytes, const uint64_t* idx, size_t count, unsigned char* slab, const Geo& g,
                           const uint64_t* col_bf, hipStream_t s);
 size_t update_tiles_lds_bytes(const Geo& g, int gbytes);
+// Most columns of a sketch: 424 with 4-byte checksums, 343 with 8-byte ones (64 KB hold a chunk, the
+// bitflips, and nine records and their 32-bit places a column).  The kernels would take some more, but the
+// update kernel keeps a record's place in its row as a 16-bit count of words, and rows of so many columns
+// reach past 262144 bytes within this card's memory: 456 columns of 4-byte checksums from 370729 vertices
+// on.  Up to the limit it takes 2^22 vertices and more than a terabyte.
+constexpr uint32_t max_columns(int gbytes) { return gbytes == 4 ? 424 : 343; }
 
 // ---- grouping of a device-resident stream of (src,dst) pairs into per-vertex tiles ----
 struct GroupBufs {

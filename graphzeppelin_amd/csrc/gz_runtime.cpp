@@ -70,7 +70,7 @@ GzSketch::GzSketch(uint64_t vector_len, uint64_t seed, size_t samples, size_t co
   check_gamma(gb);
   require_device();
   geo = make_geo(1, vector_len, seed, samples, cols, gb);
-  if (update_tiles_lds_bytes(geo, gb) > 64 * 1024) throw GzError(GZ_ERR_INVALID_ARG, "sketch too large for one workgroup's LDS");
+  if (geo.C > max_columns(gb)) throw GzError(GZ_ERR_INVALID_ARG, "sketch too large for one workgroup's LDS");
   GZ_HIP(hipGetDevice(&dev));
   GZ_HIP(hipStreamCreate(&st));
   slab.alloc(geo.row);
@@ -330,7 +330,7 @@ void GzAlg::init(BlockCache* cache, size_t keep) {
   check_gamma(gb);
   require_device();
   geo = make_geo(n, calc_vector_length(n), seed, calc_cc_samples(n, cfg.sketches_factor), 1, gb);
-  if (update_tiles_lds_bytes(geo, gb) > 64 * 1024) throw GzError(GZ_ERR_INVALID_ARG, "sketch too large for LDS");
+  if (geo.C > max_columns(gb)) throw GzError(GZ_ERR_INVALID_ARG, "sketch too large for LDS");
   tile = cfg.tile ? cfg.tile : kDefaultTile;
   const size_t lds = update_tiles_lds_bytes(geo, gb);
   // one-wave workgroups: up to 32 per CU (8 waves on each of 4 SIMDs), fewer if LDS runs out
