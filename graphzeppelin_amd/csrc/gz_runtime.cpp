@@ -281,7 +281,8 @@ void GzAlg::place_buffers(Arena& dev, Arena& host) {
   flags.place(dev, kNumFlags);
   mod.place(dev, geo.samples + 2);
   labels.place(dev, n + 1);
-  scratch.place(dev, 2 * (size_t)geo.nb);
+  sum_words.place(dev, 2 * (size_t)geo.nb);
+  digest_word.place(dev, 1);
   // Borůvka round buffers
   r_cnt.place(dev, n); r_off.place(dev, n); r_cursor.place(dev, n); r_samp.place(dev, n);
   r_members[0].place(dev, n); r_members[1].place(dev, n); r_mroot[0].place(dev, n); r_mroot[1].place(dev, n);
@@ -843,7 +844,7 @@ void GzAlg::ensure_answer() {
 // may not, so after those the sum is checked once (one pass over the sketches).
 bool GzAlg::sketches_sum_to_zero() {
   if (zero_sum == 0) {
-    uint64_t *sa = scratch.p, *sg = scratch.p + geo.nb;
+    uint64_t *sa = sum_words.p, *sg = sum_words.p + geo.nb;
     launch_sum_all(gb, slab.p, geo, sa, sg, st);
     std::vector<uint64_t> ha(geo.nb), hg(geo.nb);
     GZ_HIP(hipMemcpyAsync(ha.data(), sa, geo.nb * 8, hipMemcpyDeviceToHost, st));
@@ -1149,10 +1150,11 @@ void GzAlg::dump(uint32_t v0, uint32_t count, void* outp) {
 }
 
 uint64_t GzAlg::digest() {
+  std::lock_guard<std::mutex> lk(digest_mtx);  // calls may overlap, with queries too
   flush_all();
-  launch_digest(gb, slab.p, geo, scratch.p, st);
+  launch_digest(gb, slab.p, geo, digest_word.p, st);
   uint64_t h = 0;
-  GZ_HIP(hipMemcpyAsync(&h, scratch.p, 8, hipMemcpyDeviceToHost, st));
+  GZ_HIP(hipMemcpyAsync(&h, digest_word.p, 8, hipMemcpyDeviceToHost, st));
   GZ_HIP(hipStreamSynchronize(st));
   return h;
 }

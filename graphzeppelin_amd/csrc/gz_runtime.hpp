@@ -327,7 +327,9 @@ class GzAlg {
   bool prof = false;
   std::vector<Timed> timed;
   std::vector<hipEvent_t> ev_pool;
-  DevBuf<uint64_t> scratch;     // results read back by the host: the digest, or the sketches' sum
+  // Results read back by the host: the sketches' sum (used under query_mtx) and the digest (digest_mtx).
+  DevBuf<uint64_t> sum_words, digest_word;
+  std::mutex digest_mtx;
   DevBuf<uint64_t> prof_bytes;  // device accumulator for grouped-flush bytes
   gz_alg_profile profile{};
   hipEvent_t prof_begin(int kind, double host_bytes, bool dev_bytes, uint64_t items);
