@@ -315,12 +315,15 @@ __device__ inline bool sf_contains(const DsuDev& d, uint64_t key) {
 // n <= 2^32 - 1 after the range check, so it never equals the two sentinels (high half all ones)
 // that stand for ZERO and FAIL.
 constexpr uint64_t kSampZero = ~0ull;
-constexpr uint64_t kSampFail = ~0ull - 1;
+constexpr uint64_t kSampEmpty = ~0ull - 1;  // ZERO, and the column's buckets that were read are empty as well
+constexpr uint64_t kSampFail = ~0ull - 2;
 
 // An index whose endpoints are out of range (a checksum collision) counts as FAIL and raises the
 // bad-sample flag (plain store: every writer stores the same value).
+constexpr int kEmptyCode = 3;  // beside SampleCode
 __device__ inline uint64_t sample_record(int code, uint64_t idx, uint32_t n, uint32_t* flags) {
   if (code == kZero) return kSampZero;
+  if (code == kEmptyCode) return kSampEmpty;
   if (code != kGood) return kSampFail;
   if ((uint32_t)(idx >> 32) >= n || (uint32_t)idx >= n) {
     flags[kFlagBad] = 1;
@@ -332,14 +335,14 @@ __device__ inline uint64_t sample_record(int code, uint64_t idx, uint32_t n, uin
 // ---- sample (src/sketch.cpp:94-116) over one wave --------------------------------------------
 // Lane l < D holds bucket (column, depth l), lane D the deterministic bucket.  Every lane checks its
 // own record with one hash, so the deterministic bucket's check runs alongside the column's.
-// Returns the code; *idx gets the sampled index on GOOD.
+// Returns the code, kEmptyCode for a ZERO without a nonzero bucket; *idx gets the sampled index on GOOD.
 template <class G>
 __device__ inline int wave_sample(uint64_t a, G gm, uint32_t D, uint64_t chk_bf, uint64_t* idx) {
   const uint32_t lane = lane_id();
   const uint64_t mask = __ballot(lane <= D && (G)xxh3_mix(xxh3_prep(a), chk_bf) == gm);
   const uint64_t det_a = rd_lane_u64(a, (int)D);
   const G det_g = (G)rd_lane_u64((uint64_t)gm, (int)D);
-  if (det_a == 0 && det_g == 0) { *idx = 0; return kZero; }
+  if (det_a == 0 && det_g == 0) { *idx = 0; return __ballot((a | (uint64_t)gm) != 0) ? kZero : kEmptyCode; }
   if ((mask >> D) & 1) { *idx = det_a; return kGood; }
   const uint64_t col = mask & ((1ull << D) - 1);
   if (col) {
@@ -1431,7 +1434,7 @@ k_sample_round0(const unsigned char* __restrict__ slab, Geo g, uint64_t* __restr
     bool undecided = false;
     if (i == 0 && v < g.n) {
       hint[v] = (unsigned char)(gnz ? 32 - __builtin_clz(gnz) : 0);
-      if (det_a == 0 && det_g == 0) samp[v] = kSampZero;
+      if (det_a == 0 && det_g == 0) samp[v] = gnz ? kSampZero : kSampEmpty;
       else if ((gmask >> GD) & 1) put(v, sample_record(kGood, det_a, g.n, flags));
       else if (colm) put(v, sample_record(kGood, col_a, g.n, flags));
       else if (g.D <= GD) samp[v] = kSampFail;
@@ -1526,7 +1529,7 @@ __device__ inline uint32_t walk_vertex(const uint32_t* act_list, uint32_t round,
 }
 
 __device__ inline bool apply_sample(const DsuDev& d, uint64_t s, const unsigned char* hint) {
-  if (s == kSampZero) return false;
+  if (s == kSampZero || s == kSampEmpty) return false;
   if (s == kSampFail) return true;
   const uint32_t a = (uint32_t)(s >> 32), b = (uint32_t)s;
   const uint32_t child = dsu_link(d.parent, a, b, d.prio_seed, hint);
@@ -1631,10 +1634,14 @@ k_bv_find_count(uint32_t* __restrict__ parent, uint32_t n, uint2* __restrict__ n
 // Segments for the roots met in this round's walk (every non-giant root is a member of its own
 // supernode, so it is walked).  cnt is cleared here, its last reader.  Without a giant yet, a root
 // holding more than half of the vertices is elected: at most one can.
-// drop_ok: every update reached both of its ends' sketches, so a supernode without cut edges, which
-// samples ZERO, stays one: no other supernode has an edge into it, and its sums are zero.  A root that
-// was one vertex (rounds >= 2: one supernode) in the last round and sampled ZERO gets no segment
+// drop_ok: every update reached both of its ends' sketches, so a supernode without cut edges stays one:
+// no other supernode has an edge into it, and its sums are zero.  A root that was one vertex (rounds >= 2:
+// one supernode) in the last round and whose sums were all empty (kSampEmpty) gets no segment
 // (off = kDropped), so finished components are not walked again.  The giant's election comes first.
+// The deterministic bucket alone does not decide: edges whose indices cancel (any four of the form (v, x),
+// (v, x'), (v, y), (v, y') with x ^ x' == y ^ y') leave it zero when their checksums do, once in 2^32 such
+// sets, and the supernodes that later link with it would be walked without its members, or not at all
+// where its root stays one.  In a column such a set is empty only when all of it falls on one depth.
 // A query on 2^20 R-MAT vertices, a third of them isolated: the rounds' launches 1560 -> 700 us.
 // A root's segment goes into the round's segment list too (block scan of the counts and of the
 // roots, packed in one 64-bit scan: counts in the low 40 bits, roots above).
@@ -1666,7 +1673,7 @@ k_bv_alloc(uint32_t* __restrict__ cnt, uint32_t n, uint32_t* __restrict__ off, u
   } else if (!act && giant_ok && c >= 2 && c >= n / kCandidateDiv) {  // at most kCandidateDiv roots
     atomicMax(reinterpret_cast<unsigned long long*>(st + kStBest), ((unsigned long long)c << 32) | v);
   }
-  const bool drop = c == 1 && sv == kSampZero;
+  const bool drop = c == 1 && sv == kSampEmpty;
   if (drop) {
     c = 0;
     off[v] = kDropped;
@@ -1771,7 +1778,7 @@ __device__ inline void seg_allocate(uint32_t c, uint32_t v, uint32_t old_len, ui
     c = 0;
   } else if (!act && giant_ok && c >= 2 && c >= n / kCandidateDiv) {
     atomicMax(reinterpret_cast<unsigned long long*>(st + kStBest), ((unsigned long long)c << 32) | v);
-  } else if (c != 0 && c == old_len && sv == kSampZero) {
+  } else if (c != 0 && c == old_len && sv == kSampEmpty) {
     atomicAdd(&s_drop, c);
     c = 0;
     out.off[v] = kDropped;
@@ -2094,13 +2101,14 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
   const uint32_t before_me = i == kRowDet ? 0u : (1u << kRowDet) | ((1u << i) - 1);
   // Sample the runs of the rows with `done` set (the same in all lanes of a row); first: the run's first lane.
   auto emit = [&](bool done, uint64_t a, G gm, uint32_t first) {
-    const bool zero = i == kRowDet && (a | (uint64_t)gm) == 0;
+    const bool held = (a | (uint64_t)gm) != 0, zero = i == kRowDet && !held;
+    const bool empty = ((__ballot(held) >> base) & 0xffffu) == 0;
     const bool ok = done && live && (zero || (G)xxh3_mix(xxh3_prep(a), g.chk_bf) == gm);
     const uint32_t good = (uint32_t)(__ballot(ok) >> base) & 0xffffu;
     const bool left = done && i == kRowDet && good == 0;
     if (left || (ok && (good & before_me) == 0)) {
       const uint32_t x = (uint32_t)(a >> 32), y = (uint32_t)a;
-      recs[first] = left ? kRecLeft : zero ? kSampZero : (x > y ? x : y) < g.n ? a : kRecBad;
+      recs[first] = left ? kRecLeft : zero ? (empty ? kSampEmpty : kSampZero) : (x > y ? x : y) < g.n ? a : kRecBad;
     }
   };
 
@@ -2372,7 +2380,7 @@ k_bv_reduce(const uint32_t* __restrict__ st, const uint32_t* __restrict__ member
     const int code = wave_sample<G>(a, (G)gm, g.D, g.chk_bf, &idx);
     const uint64_t rec = sample_record(code, idx, g.n, d.flags);
     if (lane == 0) samp[R] = rec;
-    const uint64_t idle = __ballot(pend == kSampZero);
+    const uint64_t idle = __ballot(pend > kSampFail);
     if (!idle) modified |= lane == 0 && apply_sample(d, rec, hint);
     else if (lane == (uint32_t)__builtin_ctzll(idle)) pend = rec;
   };
