@@ -30,14 +30,10 @@ void require_device() {
     throw GzError(GZ_ERR_DEVICE, "no HIP device is available: the HIP library needs a GPU");
 }
 
-static Geo make_geo(uint32_t nsk, uint64_t vector_len, uint64_t seed, size_t samples, size_t cols, int gb) {
-  if (vector_len < 1) throw GzError(GZ_ERR_INVALID_ARG, "vector length must be >= 1");
-  if (samples < 1 || cols < 1) throw GzError(GZ_ERR_INVALID_ARG, "num_samples and cols_per_sample must be >= 1");
+static Geo plan_geo(uint32_t nsk, uint64_t vector_len, uint64_t seed, size_t samples, size_t cols, int gb) {
   Geo g{};
   g.n = nsk;
-  const size_t D = calc_bkt_per_col(vector_len);
-  if (D < 1 || D > 62) throw GzError(GZ_ERR_INVALID_ARG, "bkt_per_col out of the supported range [1, 62]");
-  g.D = (uint32_t)D;
+  g.D = (uint32_t)calc_bkt_per_col(vector_len);
   g.samples = (uint32_t)samples;
   g.cps = (uint32_t)cols;
   g.C = (uint32_t)(samples * cols);
@@ -51,6 +47,13 @@ static Geo make_geo(uint32_t nsk, uint64_t vector_len, uint64_t seed, size_t sam
   g.seed = seed;
   g.chk_bf = xxh3_bitflip(seed);
   return g;
+}
+static Geo make_geo(uint32_t nsk, uint64_t vector_len, uint64_t seed, size_t samples, size_t cols, int gb) {
+  if (vector_len < 1) throw GzError(GZ_ERR_INVALID_ARG, "vector length must be >= 1");
+  if (samples < 1 || cols < 1) throw GzError(GZ_ERR_INVALID_ARG, "num_samples and cols_per_sample must be >= 1");
+  const size_t D = calc_bkt_per_col(vector_len);
+  if (D < 1 || D > 62) throw GzError(GZ_ERR_INVALID_ARG, "bkt_per_col out of the supported range [1, 62]");
+  return plan_geo(nsk, vector_len, seed, samples, cols, gb);
 }
 
 static std::vector<uint64_t> column_bitflips(const Geo& g) {
@@ -157,25 +160,12 @@ static size_t default_cap_pairs(uint32_t n, size_t desired) {
   return std::min<size_t>(size_t(1) << 25, std::max<size_t>(size_t(1) << 20, want));
 }
 
+// What the constructor allocates, by its own layout, and what the runtime takes for its stream (1.3 MiB by
+// the device's account).  The buffers that come with first use (host staging, a query group of more than
+// kAnswerPoints pairs, profiling) are not counted.
 uint64_t GzAlg::footprint(uint32_t n, const gz_alg_config& c) {
-  const uint64_t len = calc_vector_length(n);
-  const size_t D = calc_bkt_per_col(len), C = calc_cc_samples(n, c.sketches_factor);
-  const uint64_t nb = C * D + 1;
-  const int gbytes = c.gamma_bytes ? c.gamma_bytes : 4;
-  const uint64_t slab = (uint64_t)n * row_layout((uint32_t)C, (uint32_t)D, 8 + gbytes).row;
-  const size_t desired = (size_t)(nb * (8 + gbytes) / 4 * c.batch_factor);
-  const uint64_t cap = c.flush_threshold ? c.flush_threshold : default_cap_pairs(n, desired);
-  const uint32_t t = c.tile ? c.tile : 1024;
-  const uint64_t part = n <= (1u << 24) ? cap * 16 /*records*/ + 8 * 1048577ull + (1 << 16) : 0;
-  const uint64_t ingest = cap * 8 /*pending*/ + cap * 8 /*dst_arr*/ + cap /*merged*/ + part +
-                          (2 * cap / t + n + 1) * sizeof(Tile) + (uint64_t)n * 20;
-  // per vertex: cnt, off, cursor, 2 member lists, 2 member-root lists, parent, labels (4 B each),
-  // sample record, forest edge, new root and shift (8 each), 2 segment lists (16 each), spanning-forest
-  // hash set (16), deterministic-bucket copy, degree class (1); the reduce's cross-workgroup
-  // accumulators (1 KiB + 4 B per 1024 vertices, and one more slot)
-  const uint64_t rounds =
-      (uint64_t)n * (9 * 4 + 8 + 8 + 8 + 2 * 16 + 16 + 8 + gbytes + 1) + ((uint64_t)n / 512 + 3) * 1028 + 8192;
-  return slab + ingest + rounds;
+  constexpr uint64_t kStream = uint64_t(2) << 20;
+  return n < 2 ? 0 : GzAlg(n, c).block_bytes().first + kStream;
 }
 
 // ---- instance memory ----
@@ -252,6 +242,8 @@ void BlockCache::trim(size_t keep) {
   for (const Block& b : out) free_block(b);
 }
 
+GzAlg::GzAlg(uint32_t n_, const gz_alg_config& c) : n(n_), seed(0), cfg(c) { plan(); }
+
 GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c, BlockCache* cache, size_t keep)
     : n(n_), seed(seed_), cfg(c) {
   try {
@@ -321,35 +313,44 @@ void GzAlg::place_buffers(Arena& dev, Arena& host) {
   aq_out.place(host, kNumFlags + kAnswerPoints / 4);
 }
 
-void GzAlg::init(BlockCache* cache, size_t keep) {
-  if (n < 2) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices must be >= 2");
-  if (n > (1u << 31)) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices above 2^31 is not supported");
+// Everything that sizes depend on; no device needed.
+void GzAlg::plan() {
   if (cfg.sketches_factor <= 0) cfg.sketches_factor = 1;  // cc_alg_configuration.cpp:15-23
   if (cfg.batch_factor <= 0) cfg.batch_factor = 1;        // cc_alg_configuration.cpp:25-33
   if (cfg.gamma_bytes == 0) cfg.gamma_bytes = 4;
   gb = cfg.gamma_bytes;
-  check_gamma(gb);
-  require_device();
-  geo = make_geo(n, calc_vector_length(n), seed, calc_cc_samples(n, cfg.sketches_factor), 1, gb);
-  if (geo.C > max_columns(gb)) throw GzError(GZ_ERR_INVALID_ARG, "sketch too large for LDS");
+  geo = plan_geo(n, calc_vector_length(n), seed, calc_cc_samples(n, cfg.sketches_factor), 1, gb);
   tile = cfg.tile ? cfg.tile : kDefaultTile;
+  cap_pairs = cfg.flush_threshold ? (size_t)cfg.flush_threshold : default_cap_pairs(n, desired_updates_per_batch());
+  if (cap_pairs > (size_t(1) << 30)) cap_pairs = size_t(1) << 30;
+}
+
+// Bytes of the instance's device block and of its pinned host block.
+std::pair<size_t, size_t> GzAlg::block_bytes() {
+  Arena dev, host;
+  place_buffers(dev, host);
+  auto round_up = [](size_t x, size_t to) { return (x + to - 1) / to * to; };
+  return {round_up(dev.used, size_t(2) << 20), round_up(host.used, size_t(32) << 10)};
+}
+
+void GzAlg::init(BlockCache* cache, size_t keep) {
+  if (n < 2) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices must be >= 2");
+  if (n > (1u << 31)) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices above 2^31 is not supported");
+  if (cfg.gamma_bytes) check_gamma(cfg.gamma_bytes);
+  require_device();
+  plan();
+  if (geo.C > max_columns(gb)) throw GzError(GZ_ERR_INVALID_ARG, "sketch too large for LDS");
   const size_t lds = update_tiles_lds_bytes(geo, gb);
   // one-wave workgroups: up to 32 per CU (8 waves on each of 4 SIMDs), fewer if LDS runs out
   const size_t per_cu = std::max<size_t>(1, std::min<size_t>(32, (160 * 1024) / lds));
   grid_cap = (uint32_t)(device_cu_count() * per_cu);
   GZ_HIP(hipStreamCreate(&st));
 
-  cap_pairs = cfg.flush_threshold ? (size_t)cfg.flush_threshold : default_cap_pairs(n, desired_updates_per_batch());
-  if (cap_pairs > (size_t(1) << 30)) cap_pairs = size_t(1) << 30;
-
-  Arena dev, host;
-  place_buffers(dev, host);
-  auto round_up = [](size_t x, size_t to) { return (x + to - 1) / to * to; };
-  const size_t dev_bytes = round_up(dev.used, size_t(2) << 20), host_bytes = round_up(host.used, size_t(32) << 10);
+  const auto [dev_bytes, host_bytes] = block_bytes();
   mem.b = cache ? cache->take(dev_bytes, host_bytes, keep) : allocate_block(dev_bytes, host_bytes);
   mem.cache = cache;
-  dev = Arena{nullptr, static_cast<uint8_t*>(mem.b.dev), 0};
-  host = Arena{static_cast<uint8_t*>(mem.b.host), static_cast<uint8_t*>(mem.b.host_dev), 0};
+  Arena dev{nullptr, static_cast<uint8_t*>(mem.b.dev), 0};
+  Arena host{static_cast<uint8_t*>(mem.b.host), static_cast<uint8_t*>(mem.b.host_dev), 0};
   place_buffers(dev, host);
 
   // Nothing is assumed about the memory's contents.

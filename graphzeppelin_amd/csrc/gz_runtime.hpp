@@ -10,6 +10,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/gz_hip.h"
@@ -434,6 +435,9 @@ class GzAlg {
   uint64_t unranked_seen = 0;
   // src != pairs: the batch is copied from src into pairs (device memory) by the same launch
   void eager_batch(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged);
+  GzAlg(uint32_t n, const gz_alg_config& cfg);  // sizes only, without a device
+  void plan();
+  std::pair<size_t, size_t> block_bytes();
   void init(BlockCache* cache, size_t keep);
   void place_buffers(Arena& dev, Arena& host);
   void enqueue_query_prefix(bool giant_ok, bool drop_ok, uint32_t last);
