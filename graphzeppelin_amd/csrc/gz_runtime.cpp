@@ -194,18 +194,14 @@ Block BlockCache::take(size_t dev_bytes, size_t host_bytes, size_t keep) {
   GZ_HIP(hipGetDevice(&device));
   {
     std::lock_guard<std::mutex> lk(mtx_);
-    // the smallest block that is large enough and at most 1/32 larger than asked for
-    auto best = blocks_.end();
+    // blocks of this very size only: what an instance holds is what was reserved for it
     for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
-      if (it->device == device && it->dev_bytes >= dev_bytes && it->dev_bytes <= dev_bytes + dev_bytes / 32 &&
-          it->host_bytes >= host_bytes && (best == blocks_.end() || it->dev_bytes < best->dev_bytes))
-        best = it;
-    if (best != blocks_.end()) {
-      const Block b = *best;
-      blocks_.erase(best);
-      held_ -= b.dev_bytes;
-      return b;
-    }
+      if (it->device == device && it->dev_bytes == dev_bytes && it->host_bytes >= host_bytes) {
+        const Block b = *it;
+        blocks_.erase(it);
+        held_ -= b.dev_bytes;
+        return b;
+      }
   }
   trim(keep);
   try {

@@ -167,7 +167,7 @@ class BlockCache {
   BlockCache(const BlockCache&) = delete;
   BlockCache& operator=(const BlockCache&) = delete;
   ~BlockCache() { trim(0); }
-  // A block of at least these sizes, with at most `keep` bytes held besides it.
+  // A block of dev_bytes and at least host_bytes, with at most `keep` bytes held besides it.
   Block take(size_t dev_bytes, size_t host_bytes, size_t keep);
   void put(const Block& b);
   void trim(size_t keep);

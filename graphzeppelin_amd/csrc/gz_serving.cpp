@@ -213,15 +213,21 @@ class Server {
   void release(int id) {
     std::unique_ptr<GzAlg> a;
     std::unique_ptr<gz_alg> view;
+    uint64_t fp = 0;
     {
       std::lock_guard<std::mutex> lk(mtx);
       auto it = tenants.find(id);
       if (it == tenants.end()) throw GzError(GZ_ERR_INVALID_ARG, "unknown tenant");
       a = std::move(it->second.alg);
       view = std::move(it->second.view);
-      reserved -= it->second.footprint;
+      fp = it->second.footprint;
       tenants.erase(it);
     }
+    // The memory is in `kept`, or given back, before an admission may count on it: `reserved` and what is
+    // kept never exceed the budget together.
+    a.reset();
+    std::lock_guard<std::mutex> lk(mtx);
+    reserved -= fp;
   }
   GzAlg* get(int id) {
     std::lock_guard<std::mutex> lk(mtx);
