@@ -187,6 +187,8 @@ _SIGS = {
     "gz_server_tenant_alg": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.POINTER(_vp)]),
     "gz_server_reserved_bytes": (ctypes.c_uint64, [_vp]),
     "gz_server_budget_bytes": (ctypes.c_uint64, [_vp]),
+    "gz_server_kept_bytes": (ctypes.c_uint64, [_vp]),
+    "gz_server_trim": (ctypes.c_int, [_vp]),
     "gz_server_run_trace": (ctypes.c_int, [_vp, _vp, _sz, _vp, _vp, _vp, _sz, ctypes.POINTER(_AlgConfig), ctypes.c_int,
                                            _vp, _vp, _vp, _vp, ctypes.POINTER(ServeStats)]),
 }
@@ -668,6 +670,15 @@ class Server:
     @property
     def reserved_bytes(self) -> int:
         return int(lib().gz_server_reserved_bytes(self._h))
+
+    @property
+    def kept_bytes(self) -> int:
+        """Device memory of released tenants that the server keeps for later ones."""
+        return int(lib().gz_server_kept_bytes(self._h))
+
+    def trim(self):
+        """Gives back what the server keeps of released tenants, for other users of the device."""
+        _check(lib().gz_server_trim(self._h))
 
     def admit(self, n: int, seed: int, config: CCAlgConfiguration | None = None) -> int:
         t = ctypes.c_int(-1)

@@ -169,10 +169,49 @@ uint64_t GzAlg::footprint(uint32_t n, const gz_alg_config& c) {
 }
 
 // ---- instance memory ----
+namespace {
+// The process's caches.  Never destroyed: a server may outlive static objects.
+struct CacheList {
+  std::mutex mtx;
+  std::vector<BlockCache*> caches;
+};
+CacheList& cache_list() {
+  static CacheList* list = new CacheList;
+  return *list;
+}
+}  // namespace
+BlockCache::BlockCache(size_t bound) : bound_(bound) {
+  std::lock_guard<std::mutex> lk(cache_list().mtx);
+  cache_list().caches.push_back(this);
+}
+BlockCache::~BlockCache() {
+  {
+    std::lock_guard<std::mutex> lk(cache_list().mtx);
+    auto& all = cache_list().caches;
+    all.erase(std::find(all.begin(), all.end(), this));
+  }
+  trim(0);
+}
+size_t BlockCache::held() {
+  std::lock_guard<std::mutex> lk(mtx_);
+  return held_;
+}
+void give_back_kept() {
+  std::lock_guard<std::mutex> lk(cache_list().mtx);
+  for (BlockCache* c : cache_list().caches) c->trim(0);
+}
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  give_back_kept();
+  e = hipMalloc(p, bytes);
+  (void)hipGetLastError();  // the next call of anyone on this thread shall not report this one's error
+  return e;
+}
 Block allocate_block(size_t dev_bytes, size_t host_bytes) {
   Block b;
   GZ_HIP(hipGetDevice(&b.device));
-  GZ_HIP(hipMalloc(&b.dev, dev_bytes));
+  GZ_HIP(device_malloc(&b.dev, dev_bytes));
   b.dev_bytes = dev_bytes;
   try {
     GZ_HIP(hipHostMalloc(&b.host, host_bytes, hipHostMallocMapped | hipHostMallocCoherent));
@@ -204,13 +243,6 @@ Block BlockCache::take(size_t dev_bytes, size_t host_bytes, size_t keep) {
       }
   }
   trim(keep);
-  try {
-    return allocate_block(dev_bytes, host_bytes);
-  } catch (const GzError& e) {
-    if (e.code != GZ_ERR_OOM) throw;
-  }
-  (void)hipGetLastError();
-  trim(0);
   return allocate_block(dev_bytes, host_bytes);
 }
 void BlockCache::put(const Block& b) {

@@ -31,6 +31,10 @@ struct GzError : std::runtime_error {
                           std::string(#x) + " failed: " + hipGetErrorString(e_));                   \
   } while (0)
 
+// hipMalloc; what is kept of released instances (BlockCache) goes back to the device first where it does
+// not succeed otherwise.
+hipError_t device_malloc(void** p, size_t bytes);
+
 // One allocation cut into buffers on 256-byte boundaries.  The same sequence of place() calls runs
 // twice: without memory, which only adds up the size, then on the memory.
 struct Arena {
@@ -61,7 +65,7 @@ struct DevBuf {
   void alloc(size_t count) {
     release();
     if (count == 0) return;
-    GZ_HIP(hipMalloc((void**)&p, count * sizeof(T)));
+    GZ_HIP(device_malloc((void**)&p, count * sizeof(T)));
     n = count;
   }
   void ensure(size_t count) {
@@ -159,18 +163,20 @@ struct Block {
 };
 // Blocks of released instances, kept for later ones: the driver hands out tens of GB/s at most, so a
 // server that admits and releases streams spends most of its time in allocation otherwise.  Holds at
-// most `bound` bytes; what does not fit, and everything at the end, goes back to the device.  Safe
-// with several threads; a block is put back once its instance's streams are idle.
+// most `bound` bytes; what does not fit, and everything at the end, when asked to (trim) or when any
+// allocation of the library needs it (device_malloc), goes back to the device.  Safe with several threads;
+// a block is put back once its instance's streams are idle.
 class BlockCache {
  public:
-  explicit BlockCache(size_t bound) : bound_(bound) {}
+  explicit BlockCache(size_t bound);
   BlockCache(const BlockCache&) = delete;
   BlockCache& operator=(const BlockCache&) = delete;
-  ~BlockCache() { trim(0); }
+  ~BlockCache();
   // A block of dev_bytes and at least host_bytes, with at most `keep` bytes held besides it.
   Block take(size_t dev_bytes, size_t host_bytes, size_t keep);
   void put(const Block& b);
   void trim(size_t keep);
+  size_t held();
 
  private:
   std::mutex mtx_;
@@ -178,6 +184,8 @@ class BlockCache {
   size_t held_ = 0;
   const size_t bound_;
 };
+// Everything that any cache of the process holds goes back to the device.
+void give_back_kept();
 Block allocate_block(size_t dev_bytes, size_t host_bytes);
 void free_block(const Block& b);
 

@@ -481,6 +481,7 @@ int gz_server_create(uint64_t budget, int workers, gz_server** out) {
     *out = nullptr;
     gz::require_device();
     if (budget == 0) {
+      gz::give_back_kept();  // what other servers keep of released tenants is free memory
       size_t fr = 0, tot = 0;
       GZ_HIP(hipMemGetInfo(&fr, &tot));
       budget = fr;
@@ -523,6 +524,13 @@ uint64_t gz_server_reserved_bytes(const gz_server* s) {
   if (!s) return 0;
   std::lock_guard<std::mutex> lk(s->s->mtx);
   return s->s->reserved;
+}
+uint64_t gz_server_kept_bytes(const gz_server* s) { return s ? s->s->kept.held() : 0; }
+int gz_server_trim(gz_server* s) {
+  return gz::guarded_call([&] {
+    if (!s) throw gz::GzError(GZ_ERR_INVALID_ARG, "null server");
+    s->s->kept.trim(0);
+  });
 }
 uint64_t gz_server_budget_bytes(const gz_server* s) { return s ? s->s->budget : 0; }
 

@@ -69,7 +69,15 @@ int gz_server_destroy(gz_server* s);
 /* Admit a stream of num_vertices vertices.  Returns GZ_ERR_ADMISSION (and *tenant = -1) when its
  * footprint (gz_alg_footprint_bytes) does not fit in the unreserved budget. */
 int gz_server_admit(gz_server* s, uint32_t num_vertices, uint64_t seed, const gz_alg_config* cfg, int* tenant);
+/* The tenant ends.  Its device memory may stay with the server for later tenants of the same size: at most
+ * a quarter of the budget or 16 GiB, whichever is less, and never more than tenants have left of the budget.
+ * It goes back to the device when gz_server_trim asks for it, when an allocation of this library would fail
+ * otherwise, when a server with budget 0 is created, and with gz_server_destroy; other users of the device
+ * (another library's allocator) have to be preceded by gz_server_trim. */
 int gz_server_release(gz_server* s, int tenant);
+/* Gives back what the server keeps of released tenants; how much that is. */
+int gz_server_trim(gz_server* s);
+uint64_t gz_server_kept_bytes(const gz_server* s);
 /* A borrowed handle to an admitted tenant's instance (owned by the server; never pass it to
  * gz_alg_destroy).  It stays valid until the tenant is released or the server destroyed; every call
  * for one tenant returns the same handle. */
@@ -79,7 +87,8 @@ uint64_t gz_server_budget_bytes(const gz_server* s);
 
 /* Run a mixed trace.  Tenants named in the trace that are not admitted yet are admitted on first
  * use in the order they appear, waiting (queued) until enough admitted tenants finish and release
- * their memory; a tenant is released after its last request when release_when_done != 0.
+ * their share of the budget; a tenant is released (as by gz_server_release) after its last request when
+ * release_when_done != 0.
  * tenant_pairs[t] is tenant t's stream in device memory; tenant_n / tenant_seed give each tenant's
  * parameters for admission (tenant ids index these arrays).  Requests of one tenant are applied in
  * trace order, none before its arrival time; latency = completion - arrival.  Different tenants'
