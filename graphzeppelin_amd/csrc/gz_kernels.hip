@@ -648,12 +648,16 @@ k_update_tiles(const Tile* __restrict__ tiles, const uint32_t* __restrict__ ntil
 // words and one per deep pair.  A lane keeps its index and takes the columns one after the other from
 // a column of its own on, which spreads a step's 64 lanes over the columns.  VALU-bound like the long
 // tiles of k_update_tiles: 4.19M indices of 25 columns 446 -> 113 us.
+// SPLIT (batches that leave lanes of one workgroup idle): 2^sub lanes share an index and take every
+// 2^sub-th column, where one lane's walk through all columns was most of the kernel: a call with one index
+// of 30, 160 and 300 columns 21, 49 and 68 us -> 16, 17 and 17 (tiles of a wave each: 20, 25 and 32), 48
+// indices of 300 columns 22 (82 by tiles).
 constexpr uint32_t kOneBlock = 1024, kOneGrid = 512;
 constexpr uint32_t kOneDepth = 17, kOneMaxCols = 160;  // deltas of kOneDepth records up to this many columns
-template <class G>
+template <class G, bool SPLIT>
 __global__ void __launch_bounds__(kOneBlock, 8)
 k_sketch_update(const uint64_t* __restrict__ idxs, size_t count, unsigned char* __restrict__ slab, Geo g,
-                const uint64_t* __restrict__ col_bf, uint32_t depth) {
+                const uint64_t* __restrict__ col_bf, uint32_t depth, uint32_t sub) {
   extern __shared__ __align__(16) unsigned char smem[];
   const uint32_t C = g.C, D = g.D, lds_n = C * depth + 1, lds_d = D < depth ? D : depth;
   uint64_t* s_bf = reinterpret_cast<uint64_t*>(smem);  // spread bitflips
@@ -669,30 +673,41 @@ k_sketch_update(const uint64_t* __restrict__ idxs, size_t count, unsigned char* 
   const uint32_t near_cap = 1u << depth;
   uint64_t det_a = 0;
   G det_g = 0;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x) {
-    const uint64_t idx = idxs[i];
+  auto add = [&](uint64_t sp, uint32_t c, uint64_t idx, G chk) {
+    const uint64_t x = sp ^ s_bf[c];
+    const uint32_t low = hash_low28(x);
+    const uint32_t near = (uint32_t)__builtin_ctz(low | near_cap);
+    if (near < lds_d) {
+      const uint32_t e = mad24(c, depth, near);
+      lds_xor(s_a + e, idx);
+      lds_xor(s_g + e, chk);
+    } else {
+      const uint32_t d = bucket_depth(low, x, depth_cap);
+      if (d < D) {
+        xor_rec_atomic<G>(slab + rec_col_off<G>(g, c, d), idx, chk);
+        if (kDeepFlags<G> && rec_is_deep(g, d)) st_rlx(reinterpret_cast<uint32_t*>(slab + deep_flag_off(c)), 1u);
+      }
+    }
+  };
+  const size_t lanes = SPLIT ? count << sub : count;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < lanes; i += (size_t)gridDim.x * blockDim.x) {
+    const uint64_t idx = idxs[SPLIT ? i >> sub : i];
     const uint64_t sp = xxh3_spread(xxh3_prep(idx));
     uint64_t ck = xxh3_products(sp ^ chk_sbf);
     ck ^= ck >> 28;
     const G chk = (G)ck;
-    det_a ^= idx;
-    det_g ^= chk;
+    const uint32_t part = SPLIT ? (uint32_t)i & ((1u << sub) - 1) : 0u;
+    if (part == 0) {
+      det_a ^= idx;
+      det_g ^= chk;
+    }
+    if (SPLIT) {
+      for (uint32_t c = part; c < C; c += 1u << sub) add(sp, c, idx, chk);
+      continue;
+    }
     uint32_t c = lane_id() % C;
     for (uint32_t k = 0; k < C; ++k) {
-      const uint64_t x = sp ^ s_bf[c];
-      const uint32_t low = hash_low28(x);
-      const uint32_t near = (uint32_t)__builtin_ctz(low | near_cap);
-      if (near < lds_d) {
-        const uint32_t e = mad24(c, depth, near);
-        lds_xor(s_a + e, idx);
-        lds_xor(s_g + e, chk);
-      } else {
-        const uint32_t d = bucket_depth(low, x, depth_cap);
-        if (d < D) {
-          xor_rec_atomic<G>(slab + rec_col_off<G>(g, c, d), idx, chk);
-          if (kDeepFlags<G> && rec_is_deep(g, d)) st_rlx(reinterpret_cast<uint32_t*>(slab + deep_flag_off(c)), 1u);
-        }
-      }
+      add(sp, c, idx, chk);
       ++c;
       c = c < c - C ? c : c - C;  // C - C, or c - C below zero
     }
@@ -2921,13 +2936,21 @@ void launch_sketch_update(int gbytes, const uint64_t* idx, size_t count, unsigne
                           const uint64_t* col_bf, hipStream_t s) {
   if (!count) return;
   const uint32_t depth = g.C <= kOneMaxCols ? kOneDepth : kLdsDepthMin;
-  const uint32_t block = (uint32_t)std::min<size_t>(kOneBlock, (count + kWave - 1) / kWave * kWave);
-  const uint32_t grid = (uint32_t)std::min<size_t>(kOneGrid, (count + block - 1) / block);
-  const size_t lds = g.C * size_t(8) + ((size_t)g.C * depth + 1) * (8 + gbytes);
-  if (gbytes == 4)
-    hipLaunchKernelGGL(k_sketch_update<uint32_t>, dim3(grid), dim3(block), lds, s, idx, count, slab, g, col_bf, depth);
-  else
-    hipLaunchKernelGGL(k_sketch_update<uint64_t>, dim3(grid), dim3(block), lds, s, idx, count, slab, g, col_bf, depth);
+  const uint32_t lds_n = g.C * depth + 1;
+  // Lanes of an index: as many as one workgroup has for the batch, at most a wave's or one per column.  Its
+  // threads then also cover the delta's entries, which a wave alone would clear and write back in up to 80
+  // steps.
+  uint32_t sub = 0;
+  while (sub < 6 && (1u << sub) < g.C && (count << (sub + 1)) <= kOneBlock) ++sub;
+  const size_t work = sub ? std::max<size_t>(count << sub, lds_n) : count;
+  const uint32_t block = (uint32_t)std::min<size_t>(kOneBlock, (work + kWave - 1) / kWave * kWave);
+  const uint32_t grid = sub ? 1u : (uint32_t)std::min<size_t>(kOneGrid, (count + block - 1) / block);
+  const size_t lds = g.C * size_t(8) + (size_t)lds_n * (8 + gbytes);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, s, idx, count, slab, g, col_bf, depth, sub);
+  };
+  if (gbytes == 4) sub ? go(k_sketch_update<uint32_t, true>) : go(k_sketch_update<uint32_t, false>);
+  else sub ? go(k_sketch_update<uint64_t, true>) : go(k_sketch_update<uint64_t, false>);
 }
 
 size_t group_partials_len(uint32_t n) { return (n + kScanSpan - 1) / kScanSpan + 1; }
