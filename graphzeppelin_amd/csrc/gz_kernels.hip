@@ -1829,7 +1829,7 @@ __device__ inline void seg_allocate(uint32_t c, uint32_t v, uint32_t old_len, ui
     const uint32_t o = s_base + (uint32_t)(ex & kCntMask);
     const uint32_t k = s_sbase + (uint32_t)(ex >> kSegShift);
     out.off[v] = o;
-    out.cursor[v] = o + c;  // the segment end, as the vertex scatter leaves it
+    out.cursor[v] = o + c;  // the segment end
     if (k < n) out.segs[k] = RoundSeg{v, o, c, 0};
   }
 }
@@ -1974,11 +1974,13 @@ k_seg_copy(uint32_t n, const uint2* __restrict__ nd, const uint32_t* __restrict_
 // l - f + 1 samples the sum and clears the slot and the counter for the next round.  The parts are
 // added with atomics that return, so they have been performed when the count is made, and the last one
 // takes the sum with exchanges that leave zeros: no fence, which would write caches back and invalidate
-// them for every part.  A reduce of 2^18 vertices took 29.7 us on average with a full fence before the
+// them for every part.  That order is a property of this card (a device-scope atomic that has returned was
+// performed where every workgroup's next one sees it), not of the language's memory model: until the last
+// workgroup has cleared a slot, every access to it and to its counter has to stay a returning
+// read-modify-write of device scope.  A reduce of 2^18 vertices took 29.7 us on average with a full fence before the
 // count and after the last one, 26.0 with a release and an acquire, 23.2 now; of 32k vertices 13.7, 11.8
-// and 10.8.  The segment
-// bounds come from k_bv_alloc / k_bv_scatter (off = start, cursor = end).  No workgroup waits for
-// another, and the XOR is order-free, so the sum is exactly the member-wise merge.
+// and 10.8.  The segment bounds are those that k_bv_alloc or seg_allocate gave out (off = start, cursor =
+// end).  No workgroup waits for another, and the XOR is order-free, so the sum is exactly the member-wise merge.
 //
 // Giant supernode.  Every edge update XORs the same buckets into both endpoints' sketches, so the
 // XOR of all vertex sketches is zero and a supernode's sum equals the XOR of every vertex outside
@@ -2002,7 +2004,7 @@ struct XAcc {
   uint32_t* cnt;
   uint32_t nslots;
   const uint32_t* seg_off;  // segment start per root
-  const uint32_t* seg_end;  // segment end per root (the scatter cursor after k_bv_scatter)
+  const uint32_t* seg_end;  // segment end per root
 };
 
 // Value of lane K of every row of 16 lanes, given to all lanes of that row.  Every lane must be active.
@@ -2296,6 +2298,7 @@ __device__ inline void reduce_members(uint32_t p0, uint32_t len, uint32_t q, uin
 
 // Per lane: XOR (a, gm) into an accumulator slot with device-scope atomics (zero words skipped), and wait
 // for their results, after which they have been performed.
+// (See "Cross-workgroup supernodes" above: the wait is what orders the part before the count.)
 __device__ inline void xacc_add(uint64_t* slot, uint64_t a, uint64_t gm) {
   const uint32_t lane = lane_id();
   uint64_t was_a = 0, was_g = 0;

@@ -118,7 +118,7 @@ constexpr uint32_t kRoundStats = 192;
 struct RoundBufs {
   uint32_t* cnt;         // n      members per root (zero between rounds)
   uint32_t* off;         // n      segment start per root
-  uint32_t* cursor;      // n      scatter cursor per root (the segment end after the scatter)
+  uint32_t* cursor;      // n      segment end per root
   uint32_t* members[2];  // n each vertices grouped by root, by round parity (also the next active list)
   uint32_t* mroot[2];    // n each the root of members[parity][p] at position p
   RoundSeg* segs[2];     // n each the round's supernodes outside the giant, by round parity
@@ -141,7 +141,7 @@ void launch_round_state_init(const RoundBufs& rb, uint32_t n, hipStream_t s);
 // Writes rb.samp: a sample record per vertex.
 void launch_sample_round0(int gbytes, const unsigned char* slab, const Geo& g, const DsuDev& d, const RoundBufs& rb,
                           hipStream_t s);
-// Workgroups of a round's reduce over n vertices (enough for 512 member entries each).
+// Workgroups of a round's reduce over n vertices, whatever the entries per wave that the round takes.
 uint32_t reduce_blocks(uint32_t n);
 // Rounds r0, r0 + 1, ... up to last_round in one workgroup, when round r0 - 1 changed something and
 // round r0 walks at most finish_max() vertices; otherwise a no-op.  Only for sketches known to XOR to
@@ -155,7 +155,7 @@ uint32_t finish_max();
 // Queue round `round` (>= 1); every kernel of it is a no-op when d.mod[round - 1] == 0.
 // giant_ok: the vertex sketches are known to XOR to zero, so a supernode holding more than half of
 // the vertices may be summed from its complement.  drop_ok: the sketches were built from updates that
-// reached both ends, so supernodes that sample ZERO are finished and leave the lists.  deep_skip: the reduce reads a member's records
+// reached both ends, so supernodes whose sums are all empty are finished and leave the lists.  deep_skip: the reduce reads a member's records
 // past the first overflow line of the round's column only when its deep flag is set (rows of
 // 12-byte records); false reads them all (same result).
 void launch_round(int gbytes, uint32_t round, const unsigned char* slab, const Geo& g,

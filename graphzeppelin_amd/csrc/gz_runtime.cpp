@@ -1045,9 +1045,10 @@ bool GzAlg::boruvka(const std::function<void()>* speculate, bool gated, bool* sk
 
 void GzAlg::eager_batch(const uint32_t* src, uint32_t* pairs, size_t count, uint8_t* merged) {
   if (!count) return;
+  // builds the forest set when pending
   launch_eager(src, pairs, count, merged, dsu, st, sf_pending, rb.hint, unranked_seen >= 4ull * n,
                dsu_map.p);
-  unranked_seen += count;  // builds the forest set when pending
+  unranked_seen += count;
   sf_pending = false;
 }
 
