@@ -163,9 +163,11 @@ static size_t default_cap_pairs(uint32_t n, size_t desired) {
 // What the constructor allocates, by its own layout, and what the runtime takes for its stream (1.3 MiB by
 // the device's account).  The buffers that come with first use (host staging, a query group of more than
 // kAnswerPoints pairs, profiling) are not counted.
-uint64_t GzAlg::footprint(uint32_t n, const gz_alg_config& c) {
+GzAlg::Sizes GzAlg::sizes(uint32_t n, const gz_alg_config& c) {
   constexpr uint64_t kStream = uint64_t(2) << 20;
-  return n < 2 ? 0 : GzAlg(n, c).block_bytes().first + kStream;
+  if (n < 2) return {};
+  const auto [dev, host] = GzAlg(n, c).block_bytes();
+  return {dev + kStream, dev, host};
 }
 
 // ---- instance memory ----
@@ -190,7 +192,7 @@ BlockCache::~BlockCache() {
     auto& all = cache_list().caches;
     all.erase(std::find(all.begin(), all.end(), this));
   }
-  trim(0);
+  trim();
 }
 size_t BlockCache::held() {
   std::lock_guard<std::mutex> lk(mtx_);
@@ -198,7 +200,7 @@ size_t BlockCache::held() {
 }
 void give_back_kept() {
   std::lock_guard<std::mutex> lk(cache_list().mtx);
-  for (BlockCache* c : cache_list().caches) c->trim(0);
+  for (BlockCache* c : cache_list().caches) c->trim();
 }
 hipError_t device_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
@@ -228,22 +230,19 @@ void free_block(const Block& b) {
   if (b.host) (void)hipHostFree(b.host);
 }
 
-Block BlockCache::take(size_t dev_bytes, size_t host_bytes, size_t keep) {
+Block BlockCache::take(size_t dev_bytes, size_t host_bytes) {
   int device = 0;
   GZ_HIP(hipGetDevice(&device));
-  {
-    std::lock_guard<std::mutex> lk(mtx_);
-    // blocks of this very size only: what an instance holds is what was reserved for it
-    for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
-      if (it->device == device && it->dev_bytes == dev_bytes && it->host_bytes >= host_bytes) {
-        const Block b = *it;
-        blocks_.erase(it);
-        held_ -= b.dev_bytes;
-        return b;
-      }
-  }
-  trim(keep);
-  return allocate_block(dev_bytes, host_bytes);
+  std::lock_guard<std::mutex> lk(mtx_);
+  // blocks of this very size only: what an instance holds is what was reserved for it
+  for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
+    if (it->device == device && it->dev_bytes == dev_bytes && it->host_bytes >= host_bytes) {
+      const Block b = *it;
+      blocks_.erase(it);
+      held_ -= b.dev_bytes;
+      return b;
+    }
+  return Block{};
 }
 void BlockCache::put(const Block& b) {
   if (!b.dev) return;
@@ -257,25 +256,25 @@ void BlockCache::put(const Block& b) {
   }
   free_block(b);
 }
-void BlockCache::trim(size_t keep) {
+std::vector<Block> BlockCache::cut(size_t keep) {
   std::vector<Block> out;
-  {
-    std::lock_guard<std::mutex> lk(mtx_);
-    while (held_ > keep) {
-      held_ -= blocks_.front().dev_bytes;
-      out.push_back(blocks_.front());
-      blocks_.erase(blocks_.begin());
-    }
+  std::lock_guard<std::mutex> lk(mtx_);
+  while (held_ > keep) {
+    held_ -= blocks_.front().dev_bytes;
+    out.push_back(blocks_.front());
+    blocks_.erase(blocks_.begin());
   }
-  for (const Block& b : out) free_block(b);
+  return out;
 }
 
 GzAlg::GzAlg(uint32_t n_, const gz_alg_config& c) : n(n_), seed(0), cfg(c) { plan(); }
 
-GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c, BlockCache* cache, size_t keep)
+GzAlg::GzAlg(uint32_t n_, uint64_t seed_, const gz_alg_config& c, BlockCache* cache, const Block& have)
     : n(n_), seed(seed_), cfg(c) {
+  mem.b = have;
+  mem.cache = cache;
   try {
-    init(cache, keep);
+    init();
   } catch (...) {  // the members are about to give memory back that queued work may still use
     if (st) {
       (void)hipStreamSynchronize(st);
@@ -361,7 +360,7 @@ std::pair<size_t, size_t> GzAlg::block_bytes() {
   return {round_up(dev.used, size_t(2) << 20), round_up(host.used, size_t(32) << 10)};
 }
 
-void GzAlg::init(BlockCache* cache, size_t keep) {
+void GzAlg::init() {
   if (n < 2) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices must be >= 2");
   if (n > (1u << 31)) throw GzError(GZ_ERR_INVALID_ARG, "num_vertices above 2^31 is not supported");
   if (cfg.gamma_bytes) check_gamma(cfg.gamma_bytes);
@@ -375,8 +374,7 @@ void GzAlg::init(BlockCache* cache, size_t keep) {
   GZ_HIP(hipStreamCreate(&st));
 
   const auto [dev_bytes, host_bytes] = block_bytes();
-  mem.b = cache ? cache->take(dev_bytes, host_bytes, keep) : allocate_block(dev_bytes, host_bytes);
-  mem.cache = cache;
+  if (!mem.b.dev) mem.b = allocate_block(dev_bytes, host_bytes);
   Arena dev{nullptr, static_cast<uint8_t*>(mem.b.dev), 0};
   Arena host{static_cast<uint8_t*>(mem.b.host), static_cast<uint8_t*>(mem.b.host_dev), 0};
   place_buffers(dev, host);

@@ -161,6 +161,9 @@ struct Block {
   size_t host_bytes = 0;
   int device = 0;  // the device dev is on
 };
+Block allocate_block(size_t dev_bytes, size_t host_bytes);
+void free_block(const Block& b);
+
 // Blocks of released instances, kept for later ones: the driver hands out tens of GB/s at most, so a
 // server that admits and releases streams spends most of its time in allocation otherwise.  Holds at
 // most `bound` bytes; what does not fit, and everything at the end, when asked to (trim) or when any
@@ -172,10 +175,14 @@ class BlockCache {
   BlockCache(const BlockCache&) = delete;
   BlockCache& operator=(const BlockCache&) = delete;
   ~BlockCache();
-  // A block of dev_bytes and at least host_bytes, with at most `keep` bytes held besides it.
-  Block take(size_t dev_bytes, size_t host_bytes, size_t keep);
+  // A block of dev_bytes and at least host_bytes, or an empty one.
+  Block take(size_t dev_bytes, size_t host_bytes);
   void put(const Block& b);
-  void trim(size_t keep);
+  // Takes blocks out until at most `keep` bytes are held; the caller frees them.
+  std::vector<Block> cut(size_t keep);
+  void trim() {
+    for (const Block& b : cut(0)) free_block(b);
+  }
   size_t held();
 
  private:
@@ -186,8 +193,6 @@ class BlockCache {
 };
 // Everything that any cache of the process holds goes back to the device.
 void give_back_kept();
-Block allocate_block(size_t dev_bytes, size_t host_bytes);
-void free_block(const Block& b);
 
 // An instance's block, given back when the instance ends.
 struct Memory {
@@ -234,9 +239,9 @@ class GzSketch {
 // CCSketchAlg (include/cc_sketch_alg.h) with every vertex sketch resident in HBM.
 class GzAlg {
  public:
-  // cache (or nullptr): where the instance's memory comes from and goes back to, with at most `keep`
-  // bytes left in it meanwhile; it outlives the instance.
-  GzAlg(uint32_t n, uint64_t seed, const gz_alg_config& cfg, BlockCache* cache = nullptr, size_t keep = 0);
+  // cache (or nullptr): where the instance's memory goes back to; it outlives the instance.  have: a block
+  // of block_bytes() that the instance takes over, or an empty one.
+  GzAlg(uint32_t n, uint64_t seed, const gz_alg_config& cfg, BlockCache* cache = nullptr, const Block& have = Block{});
   ~GzAlg();
 
   Memory mem;  // declared before the buffers placed in it
@@ -364,7 +369,13 @@ class GzAlg {
     size_t num = sketch_bytes() / sizeof(uint32_t);
     return (size_t)(num * cfg.batch_factor);
   }
-  static uint64_t footprint(uint32_t n, const gz_alg_config& cfg);
+  // Device bytes that an instance is accounted with, and the sizes of its device and pinned host blocks.
+  struct Sizes {
+    uint64_t footprint = 0;
+    size_t dev_bytes = 0, host_bytes = 0;
+  };
+  static Sizes sizes(uint32_t n, const gz_alg_config& cfg);
+  static uint64_t footprint(uint32_t n, const gz_alg_config& cfg) { return sizes(n, cfg).footprint; }
   double batch_alg_bytes(const std::vector<uint32_t>& counts) const;
 
   void pre_insert(uint32_t src, uint32_t dst);
@@ -446,7 +457,7 @@ class GzAlg {
   GzAlg(uint32_t n, const gz_alg_config& cfg);  // sizes only, without a device
   void plan();
   std::pair<size_t, size_t> block_bytes();
-  void init(BlockCache* cache, size_t keep);
+  void init();
   void place_buffers(Arena& dev, Arena& host);
   void enqueue_query_prefix(bool giant_ok, bool drop_ok, uint32_t last);
   hipGraphExec_t get_query_graph(bool giant_ok, bool drop_ok, uint32_t last);

@@ -186,19 +186,25 @@ class Server {
   Server(uint64_t b, int w) : budget(b), kept(std::min<uint64_t>(b / 4, kKeepMax)), workers(std::max(1, w)) {}
 
   int admit(uint32_t n, uint64_t seed, const gz_alg_config& cfg) {
-    const uint64_t fp = GzAlg::footprint(n, cfg);
-    uint64_t unreserved;
+    const GzAlg::Sizes sz = GzAlg::sizes(n, cfg);
+    const uint64_t fp = sz.footprint;
+    Block have;
+    std::vector<Block> out;
     {
       std::lock_guard<std::mutex> lk(mtx);
       if (reserved + fp > budget)
         throw GzError(GZ_ERR_ADMISSION, "tenant footprint " + std::to_string(fp) + " B exceeds the unreserved budget " +
                                             std::to_string(budget - reserved) + " B");
+      // The reservation and what is taken or cut from `kept` for it are one step: of two admissions at
+      // once, neither counts on memory that the other has just taken.
+      have = kept.take(sz.dev_bytes, sz.host_bytes);
       reserved += fp;
-      unreserved = budget - reserved;
+      if (!have.dev) out = kept.cut(budget - reserved);
     }
+    for (const Block& b : out) free_block(b);
     std::unique_ptr<GzAlg> a;
     try {
-      a.reset(new GzAlg(n, seed, cfg, &kept, unreserved));
+      a.reset(new GzAlg(n, seed, cfg, &kept, have));
     } catch (...) {
       std::lock_guard<std::mutex> lk(mtx);
       reserved -= fp;
@@ -529,7 +535,7 @@ uint64_t gz_server_kept_bytes(const gz_server* s) { return s ? s->s->kept.held()
 int gz_server_trim(gz_server* s) {
   return gz::guarded_call([&] {
     if (!s) throw gz::GzError(GZ_ERR_INVALID_ARG, "null server");
-    s->s->kept.trim(0);
+    s->s->kept.trim();
   });
 }
 uint64_t gz_server_budget_bytes(const gz_server* s) { return s ? s->s->budget : 0; }

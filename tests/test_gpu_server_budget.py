@@ -61,3 +61,77 @@ def test_release_beside_admission():
     for t in tenants:
         server.release(t)
     server.close()
+
+
+def test_admissions_and_releases_at_once():
+    sizes = [1000, 4096]
+    budget = 6 * gz.footprint_bytes(sizes[1])
+    server = gz.Server(budget, 1)
+    for phase in range(15):
+        print(f"server churn phase {phase}", flush=True)
+        errors = []
+
+        def churn(seed):
+            rng = np.random.default_rng(seed)
+            mine = []
+            try:
+                for _ in range(40):
+                    if mine and rng.random() < 0.5:
+                        server.release(mine.pop(int(rng.integers(len(mine)))))
+                        continue
+                    try:
+                        mine.append(server.admit(sizes[int(rng.random() < 0.5)], 1))
+                    except gz.AdmissionError:
+                        if mine:
+                            server.release(mine.pop())
+                for t in mine:
+                    left.append(t)
+            except BaseException as e:  # noqa: BLE001 (handed to the test)
+                errors.append(e)
+
+        left = []
+        threads = [threading.Thread(target=churn, args=(4 * phase + t,)) for t in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors
+        assert server.reserved_bytes + server.kept_bytes <= budget
+        for t in left:
+            server.release(t)
+        assert server.reserved_bytes == 0 and server.kept_bytes <= budget // 4
+    server.close()
+
+
+def test_one_takes_what_is_kept_while_another_allocates():
+    # 30 small tenants and ten kept blocks of their size fill the budget but for 20 MB; a larger tenant, which
+    # needs some of the kept memory given back, and a small one, which takes a kept block, arrive at once
+    small, large = 1000, 2000
+    fp = gz.footprint_bytes(small)
+    budget = 40 * fp
+    assert gz.footprint_bytes(large) > fp
+    server = gz.Server(budget, 1)
+    for _ in range(30):
+        server.admit(small, 1)
+    for k in range(40):
+        print(f"server arrivals pass {k}", flush=True)
+        server.trim()
+        for t in [server.admit(small, 1) for _ in range(10)]:
+            server.release(t)
+        assert server.kept_bytes > 9 * (fp - (4 << 20))
+        arrived, gate = [], threading.Barrier(2)
+
+        def admit(n):
+            gate.wait()
+            arrived.append(server.admit(n, 1))
+
+        threads = [threading.Thread(target=admit, args=(n,)) for n in (large, small)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert len(arrived) == 2
+        assert server.reserved_bytes + server.kept_bytes <= budget
+        for t in arrived:
+            server.release(t)
+    server.close()
