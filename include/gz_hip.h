@@ -186,9 +186,9 @@ int gz_alg_set_query_graphs(gz_alg* a, int enable);
  * the giant's root (0xFFFFFFFF when none).  Returns the number of rounds written (<= cap). */
 size_t gz_alg_last_query_round_sizes(gz_alg* a, uint32_t* entries, uint32_t* giant_root, size_t cap);
 /* No counterpart in the reference (a device execution knob).  enable != 0 (the default): once a
- * giant supernode exists and at most 2048 vertices remain outside it, one single-workgroup launch
- * runs every remaining Borůvka round; 0: every round runs as its own launches.  Results are
- * identical. */
+ * round regroups at most 2048 vertices (of sketches known to sum to zero), one single-workgroup
+ * launch runs every remaining Borůvka round; 0: every round runs as its own launches.  Results
+ * are identical. */
 int gz_alg_set_round_finish(gz_alg* a, int enable);
 /* No counterpart in the reference (a device execution knob).  enable != 0 (the default): a
  * Borůvka reduce reads a member's records of the round's column that lie past the first line of
